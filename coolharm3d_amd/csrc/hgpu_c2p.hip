@@ -10,11 +10,10 @@
 // per-zone decision sequence is the one-pass solve's exactly.
 //
 // Network: inference is one thread per zone with the weights as wave-uniform
-// (scalar) operands.  The gradient is one wavefront per 64 samples: the
-// forward pass is per sample, the weight gradients are sums over the
-// wavefront's samples formed from activations staged in LDS (rows padded to 65
-// words, conflict-free), and the per-workgroup partials are summed in fixed
-// order, so gradients are deterministic.
+// (scalar) operands.  The gradient is one workgroup per 64 samples, its
+// products on the matrix cores from activations staged in LDS, and the
+// per-workgroup partials are summed in fixed order, so gradients are
+// deterministic.
 #include "hgpu_c2p_api.h"
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -327,138 +326,244 @@ __global__ __launch_bounds__(CB) void k_mlp_forward(long long n, const float* __
 }
 
 // Gradient partial of one workgroup of MLP_GT samples.  Samples are
-// s = blockIdx.x*MLP_GT + lane (< batch): index s itself, or with random set
+// s = blockIdx.x*MLP_GT + row (< batch): index s itself, or with random set
 // the draw of training step `step`.
-constexpr int LP = MLP_H + 1;   // padded LDS row
-__global__ __launch_bounds__(MLP_GT) void k_mlp_grad(long long n, const float* __restrict__ w, const float* feat,
+// A batch is few workgroups (64 at 4096 samples), so the kernel is bound by
+// the latency of one workgroup, not by a rate: the five products (forward
+// 64x8x64 and 64x64x64, backward 64x64x64, the weight gradients 64x64x64 and
+// 8x64x64) run on the matrix cores in FP32 (v_mfma_f32_16x16x4_f32, the lane
+// layout of mlp_forward_wave()), eight wavefronts each owning two 16x16
+// tiles, with a sample's units and a unit's samples both read from LDS rows.
+// One thread per sample on the vector units took 98 us for 4096 samples;
+// this form takes 13 us.  The rows are padded to 68 words: an A operand's 16 rows x 4
+// columns then fall on distinct banks.
+constexpr int LP = MLP_H + 4;          // padded LDS row
+constexpr int GRAD_T = 512;            // threads of a gradient workgroup
+__device__ __forceinline__ mfma_f4 mfma4(float a, float b, mfma_f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__global__ __launch_bounds__(GRAD_T) void k_mlp_grad(long long n, const float* __restrict__ w, const float* feat,
                                                     const float* target, long long batch, int random,
                                                     unsigned long long seed, int step, float* part) {
-  __shared__ float sX[MLP_GT][MLP_IN];
+  static_assert(MLP_GT == 64 && MLP_H == 64 && MLP_IN == 8 && MLP_OUT == 2 && GRAD_T == 8 * MLP_GT, "tiling");
+  __shared__ float sX[MLP_GT][MLP_IN + 1];
+  __shared__ float sW1[MLP_IN][LP];
+  __shared__ float sW2[MLP_H][LP];
+  __shared__ float sW3[MLP_H][MLP_OUT];
+  __shared__ float sB1[MLP_H], sB2[MLP_H];
   __shared__ float sH1[MLP_GT][LP];
   __shared__ float sH2[MLP_GT][LP];    // h2, later dz1
   __shared__ float sDZ2[MLP_GT][LP];
   __shared__ float sDY[MLP_GT][MLP_OUT];
   __shared__ float sLoss[MLP_GT];
-  const int lane = threadIdx.x;
-  const long long s = (long long)blockIdx.x * MLP_GT + lane;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int row = tid >> 3, sub = tid & 7;          // 8 threads per sample (or per unit)
+  const int g = lane >> 4, c = lane & 15;           // MFMA lane coordinates
+  const int mt = wv >> 1, nt0 = 2 * (wv & 1);       // this wavefront's tiles: (mt, nt0) and (mt, nt0 + 1)
+  // sample `row`: its features (one per thread) and targets (threads 0, 1)
+  const long long s = (long long)blockIdx.x * MLP_GT + row;
   const bool valid = s < batch;
-  long long k = 0;
-  if (valid) k = random ? mlp_batch_index(seed, step, s, batch, n) : s;
-  // forward, one sample per lane
-  float x[MLP_IN], z1[MLP_H];
-  for (int i = 0; i < MLP_IN; i++)
-    x[i] = valid ? (feat[i*n + k] - w[MLP_OFF_MU + i]) * w[MLP_OFF_ISD + i] : 0.f;
-  for (int i = 0; i < MLP_IN; i++) sX[lane][i] = x[i];
-  for (int j = 0; j < MLP_H; j++) {
-    float z = w[MLP_OFF_B1 + j];
-    for (int i = 0; i < MLP_IN; i++) z = fmaf(x[i], w[MLP_OFF_W1 + i*MLP_H + j], z);
-    z1[j] = z;
-    sH1[lane][j] = gelu(z);
+  float tn = 0.f;
+  {
+    const long long k = !valid ? 0 : (random ? mlp_batch_index(seed, step, s, batch, n) : s);
+    sX[row][sub] = valid ? (feat[sub*n + k] - w[MLP_OFF_MU + sub]) * w[MLP_OFF_ISD + sub] : 0.f;
+    if (sub < MLP_OUT && valid) tn = (target[sub*n + k] - w[MLP_OFF_YMU + sub]) / w[MLP_OFF_YSD + sub];
   }
-  float o[MLP_OUT] = {w[MLP_OFF_B3 + 0], w[MLP_OFF_B3 + 1]};
-  float z2l[MLP_H];
-  for (int j = 0; j < MLP_H; j++) {
-    float z = w[MLP_OFF_B2 + j];
-    for (int i = 0; i < MLP_H; i++) z = fmaf(sH1[lane][i], w[MLP_OFF_W2 + i*MLP_H + j], z);
-    z2l[j] = z;
-    const float h2 = gelu(z);
-    sH2[lane][j] = h2;
-    for (int q = 0; q < MLP_OUT; q++) o[q] = fmaf(h2, w[MLP_OFF_W3 + j*MLP_OUT + q], o[q]);
+#pragma unroll
+  for (int e = tid; e < MLP_H * MLP_H; e += GRAD_T) sW2[e >> 6][e & 63] = w[MLP_OFF_W2 + e];
+  sW1[tid >> 6][tid & 63] = w[MLP_OFF_W1 + tid];
+  if (tid < MLP_H * MLP_OUT) sW3[tid >> 1][tid & 1] = w[MLP_OFF_W3 + tid];
+  if (tid < MLP_H) { sB1[tid] = w[MLP_OFF_B1 + tid]; sB2[tid] = w[MLP_OFF_B2 + tid]; }
+  __syncthreads();
+  // layer 1; element r of a tile: sample 16 mt + 4 g + r, unit 16 nt + c
+  float gr1[2][4], gr2[2][4];   // GELU derivatives of this wavefront's tiles
+  mfma_f4 acc[2];
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    const float b = sB1[16*(nt0 + t) + c];
+    acc[t] = (mfma_f4){b, b, b, b};
   }
-  float dy[MLP_OUT], loss = 0.f;
-  for (int q = 0; q < MLP_OUT; q++) {
-    const float tn = valid ? (target[q*n + k] - w[MLP_OFF_YMU + q]) / w[MLP_OFF_YSD + q] : 0.f;
-    dy[q] = valid ? o[q] - tn : 0.f;
-    loss += 0.5f*dy[q]*dy[q];
-    sDY[lane][q] = dy[q];
+#pragma unroll
+  for (int st = 0; st < MLP_IN / 4; st++) {
+    const float a = sX[16*mt + c][4*st + g];
+#pragma unroll
+    for (int t = 0; t < 2; t++) acc[t] = mfma4(a, sW1[4*st + g][16*(nt0 + t) + c], acc[t]);
   }
-  sLoss[lane] = loss;
-  for (int j = 0; j < MLP_H; j++) {
-    float dh = 0.f;
-    for (int q = 0; q < MLP_OUT; q++) dh = fmaf(w[MLP_OFF_W3 + j*MLP_OUT + q], dy[q], dh);
-    sDZ2[lane][j] = dh*gelu_grad(z2l[j]);
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const float z = acc[t][r];
+      sH1[16*mt + 4*g + r][16*(nt0 + t) + c] = gelu(z);
+      gr1[t][r] = gelu_grad(z);
+    }
+  __syncthreads();
+  // layer 2
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    const float b = sB2[16*(nt0 + t) + c];
+    acc[t] = (mfma_f4){b, b, b, b};
+  }
+#pragma unroll
+  for (int st = 0; st < MLP_H / 4; st++) {
+    const float a = sH1[16*mt + c][4*st + g];
+#pragma unroll
+    for (int t = 0; t < 2; t++) acc[t] = mfma4(a, sW2[4*st + g][16*(nt0 + t) + c], acc[t]);
+  }
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const float z = acc[t][r];
+      sH2[16*mt + 4*g + r][16*(nt0 + t) + c] = gelu(z);
+      gr2[t][r] = gelu_grad(z);
+    }
+  __syncthreads();
+  // output layer: 8 threads per sample, 8 units each
+  {
+    float o0 = 0.f, o1 = 0.f;
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const int u = sub + 8*m;
+      const float h = sH2[row][u];
+      o0 = fmaf(h, sW3[u][0], o0);
+      o1 = fmaf(h, sW3[u][1], o1);
+    }
+#pragma unroll
+    for (int x = 1; x < 8; x <<= 1) { o0 += __shfl_xor(o0, x, 64); o1 += __shfl_xor(o1, x, 64); }
+    const float o = (sub == 0) ? o0 : o1;
+    const float dy = (valid && sub < MLP_OUT) ? (o + w[MLP_OFF_B3 + (sub & 1)]) - tn : 0.f;
+    const float l = 0.5f*dy*dy, l2 = l + __shfl_xor(l, 1, 64);
+    if (sub < MLP_OUT) sDY[row][sub] = dy;
+    if (sub == 0) sLoss[row] = l2;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; t++) {
+    const int u = 16*(nt0 + t) + c;
+    const float w30 = sW3[u][0], w31 = sW3[u][1];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int sr = 16*mt + 4*g + r;
+      sDZ2[sr][u] = fmaf(w31, sDY[sr][1], w30*sDY[sr][0])*gr2[t][r];
+    }
   }
   __syncthreads();
   float* P = part + (long long)blockIdx.x * MLP_PART;   // gradient slot of blob offset o: P[o - MLP_TRAIN_OFF]
   constexpr int GW1 = MLP_OFF_W1 - MLP_TRAIN_OFF, GB1 = MLP_OFF_B1 - MLP_TRAIN_OFF, GW2 = MLP_OFF_W2 - MLP_TRAIN_OFF,
                 GB2 = MLP_OFF_B2 - MLP_TRAIN_OFF, GW3 = MLP_OFF_W3 - MLP_TRAIN_OFF, GB3 = MLP_OFF_B3 - MLP_TRAIN_OFF;
-  // sums over the samples: lane = hidden unit j (or i)
-  {
-    const int j = lane;
-    float g3[MLP_OUT] = {0.f, 0.f}, gb2 = 0.f;
-    for (int r = 0; r < MLP_GT; r++) {
-      const float h2 = sH2[r][j];
-      for (int q = 0; q < MLP_OUT; q++) g3[q] = fmaf(h2, sDY[r][q], g3[q]);
-      gb2 += sDZ2[r][j];
-    }
-    for (int q = 0; q < MLP_OUT; q++) P[GW3 + j*MLP_OUT + q] = g3[q];
-    P[GB2 + j] = gb2;
-    if (lane < MLP_OUT) {
-      float gb3 = 0.f;
-      for (int r = 0; r < MLP_GT; r++) gb3 += sDY[r][lane];
-      P[GB3 + lane] = gb3;
-    }
-    if (lane == 0) {
-      float l = 0.f;
-      for (int r = 0; r < MLP_GT; r++) l += sLoss[r];
-      part[(long long)blockIdx.x * MLP_PART + MLP_NTRAIN] = l;
+  // dh1 = dz2 W2^T and gW2 = h1^T dz2 (rows: units of layer 1)
+  mfma_f4 dh[2], gw[2];
+#pragma unroll
+  for (int t = 0; t < 2; t++) dh[t] = gw[t] = (mfma_f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int st = 0; st < MLP_H / 4; st++) {
+    const float a = sDZ2[16*mt + c][4*st + g], a2 = sH1[4*st + g][16*mt + c];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      dh[t] = mfma4(a, sW2[16*(nt0 + t) + c][4*st + g], dh[t]);
+      gw[t] = mfma4(a2, sDZ2[4*st + g][16*(nt0 + t) + c], gw[t]);
     }
   }
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) P[GW2 + (16*mt + 4*g + r)*MLP_H + 16*(nt0 + t) + c] = gw[t][r];
+  // gW3, gb2: 8 threads per unit, 8 samples each
   {
-    const int i = lane;
-    float acc[MLP_H];
-    for (int jj = 0; jj < MLP_H; jj++) acc[jj] = 0.f;
-    for (int r = 0; r < MLP_GT; r++) {
-      const float h1 = sH1[r][i];
-      for (int jj = 0; jj < MLP_H; jj++) acc[jj] = fmaf(h1, sDZ2[r][jj], acc[jj]);
+    float g30 = 0.f, g31 = 0.f, gb2 = 0.f;
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      const int r = sub + 8*m;
+      const float h2 = sH2[r][row];
+      g30 = fmaf(h2, sDY[r][0], g30);
+      g31 = fmaf(h2, sDY[r][1], g31);
+      gb2 += sDZ2[r][row];
     }
-    for (int jj = 0; jj < MLP_H; jj++) P[GW2 + i*MLP_H + jj] = acc[jj];
+#pragma unroll
+    for (int x = 1; x < 8; x <<= 1) {
+      g30 += __shfl_xor(g30, x, 64); g31 += __shfl_xor(g31, x, 64); gb2 += __shfl_xor(gb2, x, 64);
+    }
+    if (sub == 0) {
+      P[GW3 + row*MLP_OUT + 0] = g30;
+      P[GW3 + row*MLP_OUT + 1] = g31;
+      P[GB2 + row] = gb2;
+    }
+  }
+  if (wv == 0) {   // gb3 and the loss: sums over the 64 samples
+    float b30 = sDY[lane][0], b31 = sDY[lane][1], l = sLoss[lane];
+#pragma unroll
+    for (int x = 1; x < 64; x <<= 1) {
+      b30 += __shfl_xor(b30, x, 64); b31 += __shfl_xor(b31, x, 64); l += __shfl_xor(l, x, 64);
+    }
+    if (lane == 0) { P[GB3 + 0] = b30; P[GB3 + 1] = b31; P[MLP_NTRAIN] = l; }
   }
   __syncthreads();
-  // dz1 of this lane's sample into sH2 (h2 is no longer needed)
-  for (int i = 0; i < MLP_H; i++) {
-    float dh = 0.f;
-    for (int j = 0; j < MLP_H; j++) dh = fmaf(w[MLP_OFF_W2 + i*MLP_H + j], sDZ2[lane][j], dh);
-    sH2[lane][i] = dh*gelu_grad(z1[i]);
-  }
+  // dz1 into sH2 (h2 is no longer needed)
+#pragma unroll
+  for (int t = 0; t < 2; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) sH2[16*mt + 4*g + r][16*(nt0 + t) + c] = dh[t][r]*gr1[t][r];
   __syncthreads();
-  {
-    const int i = lane;
-    float g1[MLP_IN], gb1 = 0.f;
-    for (int q = 0; q < MLP_IN; q++) g1[q] = 0.f;
-    for (int r = 0; r < MLP_GT; r++) {
-      const float dz1 = sH2[r][i];
-      gb1 += dz1;
-      for (int q = 0; q < MLP_IN; q++) g1[q] = fmaf(sX[r][q], dz1, g1[q]);
-    }
-    for (int q = 0; q < MLP_IN; q++) P[GW1 + q*MLP_H + i] = g1[q];
-    P[GB1 + i] = gb1;
+  if (wv < 4) {    // gW1 = x^T dz1: 8 rows of a 16-row tile
+    mfma_f4 g1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int st = 0; st < MLP_GT / 4; st++)
+      g1 = mfma4((c < MLP_IN) ? sX[4*st + g][c & (MLP_IN - 1)] : 0.f, sH2[4*st + g][16*wv + c], g1);
+    if (g < 2)
+#pragma unroll
+      for (int r = 0; r < 4; r++) P[GW1 + (4*g + r)*MLP_H + 16*wv + c] = g1[r];
+  } else {         // gb1: 4 threads per unit, 16 samples each
+    const int u = (tid - 256) >> 2, q = tid & 3;
+    float gb1 = 0.f;
+#pragma unroll
+    for (int m = 0; m < 16; m++) gb1 += sH2[q + 4*m][u];
+    gb1 += __shfl_xor(gb1, 1, 64);
+    gb1 += __shfl_xor(gb1, 2, 64);
+    if (q == 0) P[GB1 + u] = gb1;
   }
 }
 
-// grad[p] = sum over workgroups of part[b][p] / batch (fixed order); the last
-// slot is the mean loss, also copied to *loss_out when given.
-__global__ __launch_bounds__(CB) void k_mlp_reduce(const float* part, long long nblk, long long batch,
-                                                  float* grad, float* loss_out) {
-  const int p = blockIdx.x * CB + threadIdx.x;
-  if (p >= MLP_PART) return;
+// grad[p] = sum over workgroups of part[b][p] / batch (fixed order: RS slices
+// of consecutive workgroups, then the slices); the last slot is the mean
+// loss, also copied to *loss_out when given.  ADAM: the step's weight update
+// follows at once in the thread that holds the gradient (m and v start from
+// zero at the first step), so a training step is two launches.  Bound by the
+// latency of its loads: 32 parameters x 8 slices per workgroup keep every
+// slice's loads in flight together (one thread per parameter took 16 us over
+// 64 partials, the separate update 5 us; both together 4 us now).
+constexpr int RP = 32, RS = CB / RP;
+template <bool ADAM>
+__global__ __launch_bounds__(CB) void k_mlp_reduce(const float* part, long long nblk, long long batch, float* grad,
+                                                  float* loss_out, float* w, float* m, float* v, float lr_t, float c1,
+                                                  float c2, int first) {
+  __shared__ float sS[RS][RP];
+  const int q = threadIdx.x % RP, sl = threadIdx.x / RP;
+  const int p = blockIdx.x * RP + q;
+  const long long per = (nblk + RS - 1) / RS, b0 = sl * per, b1 = (b0 + per < nblk) ? b0 + per : nblk;
   float acc = 0.f;
-  for (long long b = 0; b < nblk; b++) acc += part[b * MLP_PART + p];
-  acc /= (float)batch;
-  grad[p] = acc;
-  if (p == MLP_NTRAIN && loss_out) *loss_out = acc;
-}
-
-__global__ __launch_bounds__(CB) void k_mlp_adam(float* w, const float* grad, float* m, float* v, float lr_t,
-                                                float c1, float c2) {
-  const int p = blockIdx.x * CB + threadIdx.x;
-  if (p >= MLP_NTRAIN) return;
-  adam_update(&w[MLP_TRAIN_OFF + p], grad[p], &m[p], &v[p], lr_t, c1, c2);
-}
-
-__global__ __launch_bounds__(CB) void k_zero_f32(float* p, long long m) {
-  const long long t = (long long)blockIdx.x * CB + threadIdx.x;
-  if (t < m) p[t] = 0.f;
+  if (p < MLP_PART) {
+#pragma unroll 8
+    for (long long b = b0; b < b1; b++) acc += part[b * MLP_PART + p];
+  }
+  sS[sl][q] = acc;
+  __syncthreads();
+  if (sl != 0 || p >= MLP_PART) return;
+  float tot = sS[0][q];
+#pragma unroll
+  for (int r = 1; r < RS; r++) tot += sS[r][q];
+  tot /= (float)batch;
+  if (p == MLP_NTRAIN && loss_out) *loss_out = tot;
+  if constexpr (ADAM) {
+    if (p < MLP_NTRAIN) {
+      float mm = first ? 0.f : m[p], vv = first ? 0.f : v[p];
+      adam_update(&w[MLP_TRAIN_OFF + p], tot, &mm, &vv, lr_t, c1, c2);
+      m[p] = mm;
+      v[p] = vv;
+    }
+  } else {
+    grad[p] = tot;
+  }
 }
 
 // Moments of features and targets: one workgroup, fixed reduction order.
@@ -489,13 +594,12 @@ __global__ __launch_bounds__(CB) void k_mlp_moments(long long n, const float* fe
 unsigned nb(long long n) { return (unsigned)((n + CB - 1) / CB); }
 hipStream_t st(void* s) { return static_cast<hipStream_t>(s); }
 
-int grad_launch(hipStream_t stream, long long n, const float* w, const float* feat, const float* target,
-                long long batch, int random, unsigned long long seed, int step, const MlpWork& W, float* loss_out) {
+// Gradient partials of a batch into W.part; the caller launches k_mlp_reduce
+void grad_launch(hipStream_t stream, long long n, const float* w, const float* feat, const float* target,
+                 long long batch, int random, unsigned long long seed, int step, const MlpWork& W) {
   const long long nblk = (batch + MLP_GT - 1) / MLP_GT;
-  hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)nblk), dim3(MLP_GT), 0, stream, n, w, feat, target, batch, random,
+  hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)nblk), dim3(GRAD_T), 0, stream, n, w, feat, target, batch, random,
                      seed, step, W.part);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3(nb(MLP_PART)), dim3(CB), 0, stream, W.part, nblk, batch, W.grad, loss_out);
-  return hipc(hipGetLastError(), "k_mlp_grad");
 }
 
 // Launches of a compacted solve: the persistent first pass of budget_first
@@ -697,7 +801,10 @@ int hgpu_mlp_grad(void* stream, long long n, const float* w, const float* feat, 
   if (work_bytes < mlp_work_bytes(n)) return set_error(-3, "workspace smaller than hgpu_mlp_workspace_bytes()");
   hipStream_t s = st(stream);
   MlpWork W = mlp_work_layout(work, n);
-  if (int rc = grad_launch(s, n, w, feat, target, n, 0, 0ull, 0, W, loss)) return rc;
+  grad_launch(s, n, w, feat, target, n, 0, 0ull, 0, W);
+  hipLaunchKernelGGL(k_mlp_reduce<false>, dim3((MLP_PART + RP - 1) / RP), dim3(CB), 0, s, W.part,
+                     (n + MLP_GT - 1) / MLP_GT, n, W.grad, loss, nullptr, nullptr, nullptr, 0.f, 1.f, 1.f, 0);
+  if (int rc = hipc(hipGetLastError(), "k_mlp_grad")) return rc;
   return hipc(hipMemcpyAsync(grad, W.grad, sizeof(float) * MLP_NTRAIN, hipMemcpyDeviceToDevice, s),
               "hipMemcpyAsync");
 }
@@ -728,17 +835,18 @@ int hgpu_mlp_train(void* stream, long long n, const float* feat, const float* ta
   if (work_bytes < mlp_work_bytes(batch)) return set_error(-3, "workspace smaller than hgpu_mlp_workspace_bytes()");
   hipStream_t s = st(stream);
   MlpWork W = mlp_work_layout(work, batch);
-  hipLaunchKernelGGL(k_zero_f32, dim3(nb(2 * MLP_NTRAIN)), dim3(CB), 0, s, W.m, (long long)(2 * MLP_NTRAIN));
   float c1 = 1.f, c2 = 1.f;
   for (int t = 1; t <= steps; t++) {
-    if (int rc = grad_launch(s, n, w, feat, target, batch, 1, seed, t, W, loss_hist ? loss_hist + (t - 1) : nullptr))
-      return rc;
+    grad_launch(s, n, w, feat, target, batch, 1, seed, t, W);
     c1 *= ADAM_B1;
     c2 *= ADAM_B2;
-    hipLaunchKernelGGL(k_mlp_adam, dim3(nb(MLP_NTRAIN)), dim3(CB), 0, s, w, W.grad, W.m, W.v,
-                       cosine_lr(lr, t - 1, steps), 1.f - c1, 1.f - c2);
+    hipLaunchKernelGGL(k_mlp_reduce<true>, dim3((MLP_PART + RP - 1) / RP), dim3(CB), 0, s, W.part,
+                       (long long)(batch + MLP_GT - 1) / MLP_GT, (long long)batch, nullptr,
+                       loss_hist ? loss_hist + (t - 1) : nullptr, w, W.m, W.v, cosine_lr(lr, t - 1, steps), 1.f - c1,
+                       1.f - c2, t == 1 ? 1 : 0);
+    if (int rc = hipc(hipGetLastError(), "k_mlp_grad")) return rc;
   }
-  return hipc(hipGetLastError(), "k_mlp_adam");
+  return 0;
 }
 
 }  // extern "C"
