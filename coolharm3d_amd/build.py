@@ -1,7 +1,8 @@
 """Builds the native libraries in-tree.
 
 * ``coolharm3d_amd/libhgpu.so`` -- the product: HIP kernels for gfx950 behind the
-  C ABI of ``include/hgpu.h`` (hipcc): the GRMHD advance (hgpu_kernels.hip) and
+  C ABI of ``include/hgpu.h`` (hipcc): the GRMHD advance (hgpu_kernels.hip, its face
+  fluxes hgpu_flux.hip) and
   the batched con-to-prim with its learned guess (hgpu_c2p.hip), and the
   binary-black-hole metric (hgpu_pn.hip).
 * ``coolharm3d_amd/libhgpu_hostcheck.so`` -- the same kernel bodies compiled for
@@ -29,6 +30,8 @@ HIP_FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-shared", "-std=c++17", "
 HOST_FLAGS = ["-O2", "-fPIC", "-shared", "-std=c++17", "-ffp-contract=off", "-D__HIP_PLATFORM_AMD__",
               "-I" + os.path.join(ROCM, "include")]
 
+GPU_SOURCES = ["hgpu_kernels.hip", "hgpu_flux.hip", "hgpu_c2p.hip", "hgpu_pn.hip"]
+
 GPU_LIB = os.path.join(PKG, "libhgpu.so")
 HOSTCHECK_LIB = os.path.join(PKG, "libhgpu_hostcheck.so")
 
@@ -46,8 +49,7 @@ def _run(cmd):
 def build_gpu():
     hipcc = shutil.which("hipcc") or os.path.join(ROCM, "bin", "hipcc")
     tmp = GPU_LIB + ".tmp"
-    _run([hipcc] + HIP_FLAGS + ["-o", tmp, os.path.join(CSRC, "hgpu_kernels.hip"),
-                                os.path.join(CSRC, "hgpu_c2p.hip"), os.path.join(CSRC, "hgpu_pn.hip")])
+    _run([hipcc] + HIP_FLAGS + ["-o", tmp] + [os.path.join(CSRC, f) for f in GPU_SOURCES])
     os.replace(tmp, GPU_LIB)
 
 

@@ -176,11 +176,11 @@ HD void ppm_faces(const Params& P, const Ptrs& X, const double* __restrict__ src
 }
 
 // Signal speeds of a face from its two states (src/step_ch.c:706-714)
-HD void face_speeds(const State& ql, const State& qr, const Geom* g, int dim, double gam,
-                    double* cmax, double* cmin, double* ctop) {
+template <int dim, class GP>
+HD void face_speeds(const State& ql, const State& qr, GP g, double gam, double* cmax, double* cmin, double* ctop) {
   double cmaxl, cminl, cmaxr, cminr;
-  vchar_fast(&ql, g, dim, gam, &cmaxl, &cminl);
-  vchar_fast(&qr, g, dim, gam, &cmaxr, &cminr);
+  vchar_fast<dim>(&ql, g, gam, &cmaxl, &cminl);
+  vchar_fast<dim>(&qr, g, gam, &cmaxr, &cminr);
   *cmax = fabs(dmax(dmax(0., cmaxl), cmaxr));
   *cmin = fabs(dmax(dmax(0., -cminl), -cminr));
   *ctop = dmax(*cmin, *cmax);
@@ -190,9 +190,9 @@ HD void face_speeds(const State& ql, const State& qr, const Geom* g, int dim, do
 // interior speed (the rest of numerical_flux(), src/step_ch.c:681-764).  The
 // fluxes go to X.F, or to out[8] when the caller stores them itself.
 // g: the face's geometry record (flux_riemann() reads the stored one).
-template <int d>
+template <int d, class GP>
 HD void flux_riemann_g(const Params& P, const Ptrs& X, const double* pl, const double* pr,
-                       int i, int j, int k, FailRec& fr, double* out, const Geom* g) {
+                       int i, int j, int k, FailRec& fr, double* out, GP g) {
   const long long NT = P.nt;
   constexpr int dim = d + 1;
   State ql, qr;
@@ -204,7 +204,7 @@ HD void flux_riemann_g(const Params& P, const Ptrs& X, const double* pl, const d
   primtoflux(pl, &ql, dim, g, Fl);
   primtoflux(pr, &qr, dim, g, Fr);
   double cmax, cmin, ctop;
-  face_speeds(ql, qr, g, dim, P.gam, &cmax, &cmin, &ctop);
+  face_speeds<dim>(ql, qr, g, P.gam, &cmax, &cmin, &ctop);
 
   // fastest speed over interior faces (timestep(), src/step_ch.c:716-724),
   // reduced over the launch by the caller
@@ -230,10 +230,11 @@ HD void flux_riemann_g(const Params& P, const Ptrs& X, const double* pl, const d
   }
 }
 
-template <int d>
+// K: structure of the geometry records (GK_*)
+template <int d, int K = GK_GEN>
 HD void flux_riemann(const Params& P, const Ptrs& X, const double* pl, const double* pr,
                      int i, int j, int k, FailRec& fr, double* out = nullptr) {
-  flux_riemann_g<d>(P, X, pl, pr, i, j, k, fr, out, geom_at(P, X, i, j, k, d));
+  flux_riemann_g<d>(P, X, pl, pr, i, j, k, fr, out, GeomView<K, const Geom*>{geom_at(P, X, i, j, k, d)});
 }
 
 // Entropy flux of face (i,j,k) in direction d for fixup_entropy_eq()
@@ -257,7 +258,7 @@ HD double entropy_face_d(const Params& P, const Ptrs& X, const double* src, int 
   get_state(pl, g, P.gam, &ql);   // failures were counted by the face solve
   get_state(pr, g, P.gam, &qr);
   double cmax, cmin, ctop;
-  face_speeds(ql, qr, g, dim, P.gam, &cmax, &cmin, &ctop);
+  face_speeds<dim>(ql, qr, g, P.gam, &cmax, &cmin, &ctop);
   double uL0 = g->g * ql.ucon[0], uL1 = g->g * ql.ucon[dim];
   double uR0 = g->g * qr.ucon[0], uR1 = g->g * qr.ucon[dim];
   double s = (P.gam - 1.) * pl[UU] * pow(pl[RHO], 1. - P.gam);
@@ -268,12 +269,12 @@ HD double entropy_face_d(const Params& P, const Ptrs& X, const double* src, int 
   return 0.5*(Gl + Gr - ctop*(Sr - Sl));
 }
 
-template <int d>
+template <int d, int K = GK_GEN>
 HD void flux_face(const Params& P, const Ptrs& X, const double* __restrict__ src,
                   int i, int j, int k, FailRec& fr) {
   double pl[NP], pr[NP];
   flux_recon<d>(P, X, src, i, j, k, pl, pr);
-  flux_riemann<d>(P, X, pl, pr, i, j, k, fr);
+  flux_riemann<d, K>(P, X, pl, pr, i, j, k, fr);
 }
 
 // --------------------------------------------------------------------------
@@ -375,7 +376,8 @@ struct SrcDyn {
   double f_cool, ucov[4];
   int gfail;
 };
-HD void source_dyn_state(const Params& P, const Ptrs& X, const double* ph, const Geom* g, int i, SrcDyn& s) {
+template <class GP>
+HD void source_dyn_state(const Params& P, const Ptrs& X, const double* ph, GP g, int i, SrcDyn& s) {
   State q;
   s.gfail = get_state(ph, g, P.gam, &q);
   double mhd[4][4];
@@ -445,13 +447,14 @@ HD int source(const Params& P, const Ptrs& X, const double* ph, GP g, int i, int
       SrcDyn s;
       source_dyn_state(P, X, ph, g, i, s);
       if constexpr (MET == 3) {
-        source_dyn_finish(P, s, dgl, 1, g->g, dU);
+        source_dyn_finish(P, s, dgl, 1, g_det(g), dU);
       } else {
-        source_dyn_finish(P, s, X.conn + conn_id(P, i, j, k), P.nconn, g->g, dU);
+        source_dyn_finish(P, s, X.conn + conn_id(P, i, j, k), P.nconn, g_det(g), dU);
       }
       return s.gfail;
     }
   }
+  if constexpr (geom_kind<GP>::value == GK_FLAT) return 0;   // no connection, no cooling
   int gfail = 0;
   State q;
   bool have_q = false;
@@ -509,10 +512,10 @@ HD int source(const Params& P, const Ptrs& X, const double* ph, GP g, int i, int
     dU[U2] -= f_cool * q.ucov[2];
     dU[U3] -= f_cool * q.ucov[3];
   }
-  dU[UU] *= g->g;
-  dU[U1] *= g->g;
-  dU[U2] *= g->g;
-  dU[U3] *= g->g;
+  dU[UU] *= g_det(g);
+  dU[U1] *= g_det(g);
+  dU[U2] *= g_det(g);
+  dU[U3] *= g_det(g);
   return gfail;
 }
 
@@ -829,7 +832,8 @@ HD bool update_zone_fast_g(const Params& P, const Ptrs& X, int stage, double dt,
   return true;
 }
 
-template <bool MIXED, int MET = -1, bool UNI = false>
+// K: structure of the static metric's records (GK_*)
+template <bool MIXED, int MET = -1, bool UNI = false, int K = GK_GEN>
 HD bool update_zone_fast(const Params& P, const Ptrs& X, int stage, double dt, int i, int j, int k,
                          FailRec& fr, double* U) {
   const int gid = geom_id(P, i, j, k, CENT);
@@ -837,21 +841,23 @@ HD bool update_zone_fast(const Params& P, const Ptrs& X, int stage, double dt, i
   if constexpr (UNI) {
     // the wavefront's zones share one record: read through the scalar cache
     typedef const __attribute__((address_space(4))) Geom* CGp;
+    typedef GeomView<K, CGp> CGv;
     const int gu = __builtin_amdgcn_readfirstlane(gid);
-    return update_zone_fast_g<MIXED, MET, UNI>(P, X, stage, dt, i, j, k, fr, U, (CGp)(X.geom_n + gu),
-                                               (CGp)(X.geom + gu), (CGp)(X.geom_new + gu));
+    return update_zone_fast_g<MIXED, MET, UNI>(P, X, stage, dt, i, j, k, fr, U, CGv{(CGp)(X.geom_n + gu)},
+                                               CGv{(CGp)(X.geom + gu)}, CGv{(CGp)(X.geom_new + gu)});
   }
 #endif
-  return update_zone_fast_g<MIXED, MET, UNI>(P, X, stage, dt, i, j, k, fr, U, X.geom_n + gid, X.geom + gid,
-                                             X.geom_new + gid);
+  typedef GeomView<K, const Geom*> Gv;
+  return update_zone_fast_g<MIXED, MET, UNI>(P, X, stage, dt, i, j, k, fr, U, Gv{X.geom_n + gid}, Gv{X.geom + gid},
+                                             Gv{X.geom_new + gid});
 }
 
-template <bool MIXED>
 // Returns U^{n+1}[RHO], the zone's term of M_tot (src/step_ch.c:389).
+template <bool MIXED, int K = GK_GEN>
 HD double update_zone(const Params& P, const Ptrs& X, int stage, double dt, int i, int j, int k,
                       FailRec& fr) {
   double U[NP];
-  if (!update_zone_fast<MIXED>(P, X, stage, dt, i, j, k, fr, U)) {
+  if (!update_zone_fast<MIXED, -1, false, K>(P, X, stage, dt, i, j, k, fr, U)) {
     Ptrs Xn = X;
     Xn.geom = X.geom_new;   // the full tree works at the result's time level
     recover_zone<MIXED>(P, Xn, stage, dt, i, j, k, U, fr);

@@ -1,0 +1,323 @@
+// hgpu_flux.hip -- face-flux kernels of the GRMHD advance (reconstruction and
+// Riemann solve), FP64 and mixed precision, static and binary metric.
+#include "hgpu_launch.h"
+
+namespace hgpu {
+
+// W: minimum waves per SIMD the register allocation must allow (1 = the
+// compiler's choice; larger values cap the VGPRs, trading spills for occupancy).
+// K: structure of the geometry records (GK_*).
+template <int D, int W, int K>
+__global__ __launch_bounds__(BLOCK, W) void k_flux(Params P, Ptrs X, const double* __restrict__ src, Box b, Tiling T) {
+  int i, j, k;
+  const bool active = tile_index(b, T, i, j, k);
+  FailRec fr; fr.clear();
+  long long c = 0;
+  if (active) {
+    flux_face<D, K>(P, X, src, i, j, k, fr);
+    c = cidx(P, i, j, k);
+  }
+  commit_fail(P, X, fr, active, c, MASK_GAMMA, D + 1);
+}
+
+template <int D, int W, int K>
+__global__ __launch_bounds__(BLOCK, W) void k_flux_mixed(Params P, Ptrs X, const double* __restrict__ src, Box b,
+                                                         Tiling T) {
+  int i, j, k;
+  const bool active = tile_index(b, T, i, j, k);
+  FailRec fr; fr.clear();
+  long long c = 0;
+  if (active) {
+    flux_face_mixed<D, K>(P, X, src, i, j, k, fr);
+    c = cidx(P, i, j, k);
+  }
+  commit_fail(P, X, fr, active, c, MASK_GAMMA, D + 1);
+}
+
+__device__ __forceinline__ long long wave_min_ll(long long v) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const long long o = __shfl_xor(v, off, 64);
+    v = (o < v) ? o : v;
+  }
+  return v;
+}
+__device__ __forceinline__ long long wave_max_ll(long long v) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const long long o = __shfl_xor(v, off, 64);
+    v = (o > v) ? o : v;
+  }
+  return v;
+}
+
+// LDS capacity (doubles) of one primitive's x3 pencil of a wavefront: 64 face
+// groups of F faces need 64 F + 5 consecutive zones, plus the ghost zones
+// skipped where the wavefront's groups continue on the next (i,j) row.
+template <int F> constexpr int stage_cap() { return 64 * F + 5 + 3 * (F + 8); }
+
+// PPM+MC face states of the F consecutive x3 faces of every lane (ppm_faces()
+// with d = 2) from LDS-staged pencils.  The zones the wavefront's stencils
+// cover form one contiguous range of the array (k is its fastest index), so
+// each primitive's range is loaded once, coalesced, by all 64 lanes (about
+// F + 1 loads per lane instead of F + 5), stored to LDS, and each lane reads
+// its F + 5 window from there; the next primitive's loads are in flight
+// while this one's limiters run (double-buffered).  A wavefront whose range
+// exceeds the buffer (rows shorter than the wavefront) reads its windows from
+// global memory instead.  Same values, same arithmetic as ppm_faces(): the
+// face states are bit-identical.  Every lane of the wavefront must call it;
+// inactive lanes only help stage.
+template <int F>
+__device__ void ppm_faces_x3_staged(const Params& P, const Ptrs& X, const double* __restrict__ src, bool active,
+                                    int i, int j, int k, double (*pl)[NP], double (*pr)[NP], double* buf) {
+  constexpr int M = F + 5;
+  constexpr int CAP = stage_cap<F>();
+  constexpr int NL = (CAP + 63) / 64;
+  const long long NT = P.nt;
+  const int lane = threadIdx.x & 63;
+  int ii = i, jj = j;
+  if (P.degen[0]) ii = NG;
+  if (P.degen[1]) jj = NG;
+  const long long c0 = active ? cidx(P, ii, jj, k - 3) : 0;
+  int zm[M];
+#pragma unroll
+  for (int m = 0; m < M; m++) zm[m] = imin(m, P.n3t - 1 - (k - 3));
+  const long long lo = wave_min_ll(active ? c0 : LLONG_MAX);
+  const long long hi = wave_max_ll(active ? c0 + zm[M - 1] : LLONG_MIN);
+  const long long span = (hi >= lo) ? hi - lo + 1 : 0;
+  const bool staged = span > 0 && span <= CAP;   // wavefront-uniform
+  const int off = (int)(c0 - lo);
+  double r[NL];
+  if (staged) {
+#pragma unroll
+    for (int q = 0; q < NL; q++) {
+      const int e = q * 64 + lane;
+      r[q] = (e < span) ? src[lo + e] : 0.;
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < NP; v++) {
+    double* bv = buf + (v & 1) * CAP;
+    if (staged) {
+#pragma unroll
+      for (int q = 0; q < NL; q++) {
+        const int e = q * 64 + lane;
+        if (e < span) bv[e] = r[q];
+      }
+      if (v + 1 < NP) {
+#pragma unroll
+        for (int q = 0; q < NL; q++) {
+          const int e = q * 64 + lane;
+          r[q] = (e < span) ? src[(v + 1) * NT + lo + e] : 0.;
+        }
+      }
+    }
+    // the wavefront's own buffer: LDS operations of one wavefront complete in
+    // order, so a wavefront-scope fence (no workgroup barrier) orders the
+    // stores before the other lanes' reads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (active) {
+      const int s = rs_slot(v);
+      const double ra = X.rscale[s * P.n1t + ii], ri = X.irscale[s * P.n1t + ii];
+      double y[M];
+#pragma unroll
+      for (int m = 0; m < M; m++) {
+        const double raw = staged ? bv[off + zm[m]] : src[v * NT + c0 + zm[m]];
+        y[m] = (raw * ra) * ri;
+      }
+      double dq[M - 1], fi[M - 2], le[M - 2], re[M - 2];
+#pragma unroll
+      for (int m = 1; m < M - 1; m++) dq[m] = mc_slope_vect(y[m - 1], y[m], y[m + 1]);
+#pragma unroll
+      for (int m = 1; m < M - 2; m++) fi[m] = 0.5 * (y[m + 1] + y[m]) - PPM_FACTOR * (dq[m + 1] - dq[m]);
+#pragma unroll
+      for (int m = 2; m < M - 2; m++) ppm_limit(fi[m - 1], fi[m], y[m], &le[m], &re[m]);
+#pragma unroll
+      for (int f = 0; f < F; f++) {
+        pl[f][v] = re[2 + f];
+        pr[f][v] = le[3 + f];
+      }
+    }
+  }
+}
+
+// F consecutive faces along D per thread (PPM+MC, D not degenerate): the
+// thread's tile index along D counts groups of F faces from bg.lo[D]; faces
+// past hi_d (the flux box end) are skipped.  Each zone's parabola is computed
+// once per group.  The per-face fail() tally goes to the face's zone here,
+// the block totals through commit_fail().
+// Along x3 (the fastest index of the arrays) a lane's F faces are adjacent in
+// memory, so the fluxes go through LDS: slot s of lane l stores element
+// s*64 + l of the wavefront's F*64 faces, and each store instruction writes
+// consecutive faces.
+// OTF: the face records are evaluated from the orbit of level lvl (binary
+// metric) instead of read.
+// STG (x3, FP64): reconstruction from LDS-staged pencils (ppm_faces_x3_staged).
+// K: structure of the stored geometry records (the evaluated ones are GK_DIAG).
+template <int D, int F, int W, bool MIXED, int K, bool OTF = false, bool STG = false>
+__global__ __launch_bounds__(BLOCK, W) void k_flux_multi(Params P, Ptrs X, const double* __restrict__ src, Box bg,
+                                                         Tiling T, int hi_d, PnGrid G, int lvl) {
+  using Real = typename std::conditional<MIXED, float, double>::type;
+  static_assert(!STG || (D == 2 && !MIXED && !OTF), "staged pencils: FP64 x3 faces of a static metric");
+  constexpr bool TRANSPOSE = (D == 2);
+  __shared__ Real tbuf[TRANSPOSE ? BLOCK * F : 1];
+  __shared__ double sbuf[STG ? (BLOCK / 64) * 2 * stage_cap<F>() : 1];
+  int i, j, k;
+  const bool active = tile_index(bg, T, i, j, k);
+  FailRec fr; fr.clear();
+  Real fo[F][NP];
+  long long cb = 0;
+  int nv = 0;
+  Real pl[F][NP], pr[F][NP];
+  if (active) {
+    const int lo = bg.lo[D];
+    if (D == 0) i = lo + (i - lo) * F;
+    else if (D == 1) j = lo + (j - lo) * F;
+    else k = lo + (k - lo) * F;
+  }
+  if constexpr (STG) ppm_faces_x3_staged<F>(P, X, src, active, i, j, k, pl, pr, sbuf + (threadIdx.x >> 6) * 2 * stage_cap<F>());
+  if (active) {
+    constexpr int di = (D == 0), dj = (D == 1), dk = (D == 2);
+    const int nvalid = min(F, hi_d - ((D == 0) ? i : ((D == 1) ? j : k)) + 1);
+    if constexpr (STG) {
+    } else if constexpr (MIXED) {
+      ppm_faces_mixed<D, F>(P, X, src, i, j, k, pl, pr);
+    } else {
+      ppm_faces<D, F>(P, X, src, i, j, k, pl, pr);
+    }
+    PnOrbit orb;
+    if constexpr (OTF) orb = orbit_load(X.orbit + lvl);
+#pragma unroll
+    for (int f = 0; f < F; f++) {
+      if (f >= nvalid) break;
+      const int g0 = fr.nf[NFAIL_GAMMA_CALC];
+      const int fi = i + f*di, fj = j + f*dj, fk = k + f*dk;
+      if constexpr (OTF) {
+        if constexpr (MIXED) {
+          GeomF gfb;
+          pn_zone_geomf(P, G, orb, fi, fj, fk, D, &gfb);
+          flux_riemann_mixed_g<D>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr,
+                                  GeomView<GK_DIAG, const GeomF*>{&gfb});
+        } else {
+          Geom gb;
+          pn_zone_geom(P, G, orb, fi, fj, fk, D, &gb);
+          flux_riemann_g<D>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr,
+                            GeomView<GK_DIAG, const Geom*>{&gb});
+        }
+      } else {
+        if constexpr (MIXED) flux_riemann_mixed<D, K>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr);
+        else flux_riemann<D, K>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr);
+      }
+      const int dv = fr.nf[NFAIL_GAMMA_CALC] - g0;
+      if (P.track_nfail && dv) X.nfail[NFAIL_GAMMA_CALC*P.nt + cidx(P, fi, fj, fk)] += dv;
+    }
+    cb = cidx(P, i, j, k);
+    nv = nvalid;
+  }
+  if constexpr (TRANSPOSE) {
+    Real* Fa = MIXED ? (Real*)X.Ff : (Real*)X.F;
+    const int lane = threadIdx.x & 63;
+    Real* wbuf = tbuf + (threadIdx.x & ~63) * F;
+    long long cs[F];
+    bool ok[F];
+#pragma unroll
+    for (int s = 0; s < F; s++) {
+      const int e = s*64 + lane, sl = e / F, f = e % F;
+      cs[s] = __shfl(cb, sl, 64) + f;
+      ok[s] = f < __shfl(nv, sl, 64);
+    }
+#pragma unroll
+    for (int l = 0; l < NP; l++) {
+      if (l == B3) continue;   // the normal field's flux: never read
+      __syncthreads();
+#pragma unroll
+      for (int f = 0; f < F; f++) wbuf[lane*F + f] = fo[f][l];
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < F; s++)
+        if (ok[s]) Fa[(2*NFLUX + l)*(long long)P.nt + cs[s]] = wbuf[s*64 + lane];
+    }
+  }
+  commit_fail(P, X, fr, active, 0, MASK_GAMMA, D + 1, false);
+}
+
+// f(constant of the geometry records' structure)
+template <class F>
+static void with_kind(int kind, F&& f) {
+  if (kind == GK_FLAT) f(std::integral_constant<int, GK_FLAT>());
+  else if (kind == GK_KS) f(std::integral_constant<int, GK_KS>());
+  else f(std::integral_constant<int, GK_GEN>());
+}
+
+// Face fluxes along D with launch shape L: one face per thread, or fpt faces
+// per thread (PPM+MC with D not degenerate) over the box of face groups.
+template <int D, int F, bool MIXED>
+static void launch_flux_multi(const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, const Box& b,
+                              hipStream_t st, const PnGrid& G, int lvl) {
+  Box bg = b;
+  const int n = b.hi[D] - b.lo[D] + 1;
+  bg.hi[D] = b.lo[D] + (n + F - 1) / F - 1;
+  const Tiling T = make_tiling(bg, L);
+  const dim3 grid(T.nblocks), blk(T.bs);
+  if (P.otf) {
+    // three waves per SIMD fit the FP32 face solve without spilling
+    if constexpr (MIXED) hipLaunchKernelGGL((k_flux_multi<D, F, 3, true, GK_GEN, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
+    else hipLaunchKernelGGL((k_flux_multi<D, F, 1, false, GK_GEN, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
+    return;
+  }
+  if constexpr (D == 2 && !MIXED) {
+    if (L.stage) {   // reconstruction from LDS-staged pencils
+      if (L.occ) hipLaunchKernelGGL((k_flux_multi<D, F, 3, false, GK_GEN, false, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
+      else hipLaunchKernelGGL((k_flux_multi<D, F, 1, false, GK_GEN, false, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
+      return;
+    }
+  }
+  // register-capped variants: 4 waves/SIMD for the FP32 solve, 3 for FP64
+  const auto go = [&](auto K) {
+    constexpr int k = decltype(K)::value;
+    if (L.occ) hipLaunchKernelGGL((k_flux_multi<D, F, MIXED ? 4 : 3, MIXED, k>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
+    else hipLaunchKernelGGL((k_flux_multi<D, F, 1, MIXED, k>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
+  };
+  if (P.gkind == GK_KS) go(std::integral_constant<int, GK_KS>());
+  else go(std::integral_constant<int, GK_GEN>());
+}
+
+// G, lvl: the binary metric's grid and the stage's level, read when P.otf
+// (which implies PPM and no degenerate direction: the face-group kernels,
+// with at least 2 faces per thread).
+template <int D>
+static void launch_flux_d(const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, const Box& b,
+                          hipStream_t st, const PnGrid& G, int lvl) {
+  if ((L.fpt > 1 || P.otf) && P.recon == RECON_PPM_MC && !P.degen[D]) {
+    if (P.mixed) {
+      if (L.fpt == 4) launch_flux_multi<D, 4, true>(P, X, L, src, b, st, G, lvl);
+      else launch_flux_multi<D, 2, true>(P, X, L, src, b, st, G, lvl);
+    } else {
+      if (L.fpt == 4) launch_flux_multi<D, 4, false>(P, X, L, src, b, st, G, lvl);
+      else launch_flux_multi<D, 2, false>(P, X, L, src, b, st, G, lvl);
+    }
+    return;
+  }
+  const Tiling T = make_tiling(b, L);
+  const dim3 grid(T.nblocks), blk(T.bs);
+  with_kind(P.gkind, [&](auto K) {
+    constexpr int k = decltype(K)::value;
+    if (P.mixed) {
+      if (L.occ) hipLaunchKernelGGL((k_flux_mixed<D, 6, k>), grid, blk, 0, st, P, X, src, b, T);
+      else hipLaunchKernelGGL((k_flux_mixed<D, 1, k>), grid, blk, 0, st, P, X, src, b, T);
+    } else {
+      if (L.occ) hipLaunchKernelGGL((k_flux<D, 4, k>), grid, blk, 0, st, P, X, src, b, T);
+      else hipLaunchKernelGGL((k_flux<D, 1, k>), grid, blk, 0, st, P, X, src, b, T);
+    }
+  });
+}
+
+void launch_flux_dir(int d, const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, hipStream_t st,
+                     const PnGrid& G, int lvl) {
+  const Box b = flux_box(P, d);
+  if (d == 0) launch_flux_d<0>(P, X, L, src, b, st, G, lvl);
+  else if (d == 1) launch_flux_d<1>(P, X, L, src, b, st, G, lvl);
+  else launch_flux_d<2>(P, X, L, src, b, st, G, lvl);
+}
+
+}  // namespace hgpu

@@ -6,6 +6,7 @@
 // machine without a GPU; it is never loaded by the product path (the Python
 // wrapper loads libhgpu.so and fails if that is missing).
 #include "hgpu_core.h"
+#include <type_traits>
 
 namespace hgpu {
 
@@ -22,6 +23,14 @@ static void host_commit(const Params& P, const Ptrs& X, const FailRec& fr, long 
     if (fr.boundary & 1) X.status[ST_BOUNDARY_PHYS] = 1;
     if (fr.boundary & 2) X.status[ST_BOUNDARY_MPI] = 1;
   }
+}
+
+// f(constant of the geometry's structure), as the device picks its kernels
+template <class F>
+static void with_kind(int kind, F&& f) {
+  if (kind == GK_FLAT) f(std::integral_constant<int, GK_FLAT>());
+  else if (kind == GK_KS) f(std::integral_constant<int, GK_KS>());
+  else f(std::integral_constant<int, GK_GEN>());
 }
 
 struct HostBE {
@@ -73,15 +82,17 @@ struct HostBE {
       int i, j, k;
       b.at(t, i, j, k);
       FailRec fr; fr.clear();
-      if (c->P.mixed) {
-        if (d == 0) flux_face_mixed<0>(c->P, c->X, src, i, j, k, fr);
-        else if (d == 1) flux_face_mixed<1>(c->P, c->X, src, i, j, k, fr);
-        else flux_face_mixed<2>(c->P, c->X, src, i, j, k, fr);
-      } else {
-        if (d == 0) flux_face<0>(c->P, c->X, src, i, j, k, fr);
-        else if (d == 1) flux_face<1>(c->P, c->X, src, i, j, k, fr);
-        else flux_face<2>(c->P, c->X, src, i, j, k, fr);
-      }
+      with_kind(c->P.gkind, [&](auto K) {
+        if (c->P.mixed) {
+          if (d == 0) flux_face_mixed<0, K.value>(c->P, c->X, src, i, j, k, fr);
+          else if (d == 1) flux_face_mixed<1, K.value>(c->P, c->X, src, i, j, k, fr);
+          else flux_face_mixed<2, K.value>(c->P, c->X, src, i, j, k, fr);
+        } else {
+          if (d == 0) flux_face<0, K.value>(c->P, c->X, src, i, j, k, fr);
+          else if (d == 1) flux_face<1, K.value>(c->P, c->X, src, i, j, k, fr);
+          else flux_face<2, K.value>(c->P, c->X, src, i, j, k, fr);
+        }
+      });
       host_commit(c->P, c->X, fr, cidx(c->P, i, j, k), true);
       if (fr.vmax > 0.) {
         unsigned long long& w = c->X.status[ST_VMAX + d + 1];
@@ -109,8 +120,10 @@ struct HostBE {
       int i, j, k;
       b.at(t, i, j, k);
       FailRec fr; fr.clear();
-      if (c->P.mixed) mtot += update_zone<true>(c->P, c->X, stage, dt, i, j, k, fr);
-      else mtot += update_zone<false>(c->P, c->X, stage, dt, i, j, k, fr);
+      with_kind(c->P.gkind, [&](auto K) {
+        if (c->P.mixed) mtot += update_zone<true, K.value>(c->P, c->X, stage, dt, i, j, k, fr);
+        else mtot += update_zone<false, K.value>(c->P, c->X, stage, dt, i, j, k, fr);
+      });
       host_commit(c->P, c->X, fr, cidx(c->P, i, j, k), true);
     }
     c->X.scal[SC_MTOT] = mtot;

@@ -5,27 +5,9 @@
 // coalesced SoA loads; the 2D geometry record is a wavefront-wide broadcast);
 // the stencil kernels map workgroups to tiles XCD by XCD (Tiling below).
 // Failure counters are summed across the wavefront before one atomic per wave.
-#include "hgpu_core.h"
-#include <hip/hip_runtime.h>
-#include <algorithm>
-#include <type_traits>
+#include "hgpu_launch.h"
 
 namespace hgpu {
-
-constexpr int BLOCK = 256;
-
-// Launch shape of a stencil-kernel family (tile decomposition below).
-struct LaunchShape {
-  unsigned bs = 256;     // threads per workgroup: 64, 128 or 256
-  unsigned kc = 0;       // k-extent of a 2D tile, dividing bs; 0 = flat tiles
-  unsigned remap = 1;    // XCD-contiguous tile order
-  unsigned order = 0;    // 0: plane after plane; 1: x1 fastest (one (j,k) tile through consecutive planes)
-  unsigned occ = 0;      // 1: the register-capped kernel variant (flux, conserved update)
-  unsigned fused = 0;    // conserved update only: 1 = update and inversion in one kernel
-  unsigned fpt = 1;      // face fluxes only: faces per thread along the direction (1, 2, 4)
-  unsigned stage = 0;    // x3 face fluxes (FP64, PPM, fpt > 1): reconstruction from LDS-staged pencils
-};
-enum { FAM_FLUX1 = 0, FAM_FLUX2, FAM_FLUX3, FAM_EMF, FAM_CONS, FAM_INV, N_FAM };
 
 struct ProfEvent { std::string name; hipEvent_t a, b; };
 
@@ -51,459 +33,10 @@ static int hip_check(hipError_t e, const char* what) {
   return set_error(-4, std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// --------------------------------------------------------------------------
-__device__ __forceinline__ int wave_sum(int v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    const unsigned long long o = __shfl_xor(v, off, 64);
-    v = (o > v) ? o : v;
-  }
-  return v;
-}
-
-// Writes the fail() tallies of a workgroup: per-zone nfail, and block totals of
-// nfailtot, the failure words and the fastest face speed (vmax_slot >= 0),
-// reduced in LDS so each status word receives at most one atomic per
-// workgroup.  Every thread of the block must call it.
-__device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, const FailRec& fr,
-                                            bool active, long long c, unsigned mask, int vmax_slot = -1,
-                                            bool zone_map = true) {
-  __shared__ unsigned s_cnt[N_NFAIL];
-  __shared__ unsigned s_flags;
-  __shared__ unsigned long long s_vmax;
-  const long long NT = P.nt;
-  const int tid = threadIdx.x;
-  if (tid < N_NFAIL) s_cnt[tid] = 0;
-  if (tid == 0) { s_flags = 0; s_vmax = 0; }
-  __syncthreads();
-  if (active) {
-    for (int l = 0; l < N_NFAIL; l++) {
-      if (!(mask & (1u << l))) continue;
-      const int v = fr.nf[l];
-      if (v) {
-        if (P.track_nfail && zone_map) X.nfail[l*NT + c] += v;
-        atomicAdd(&s_cnt[l], (unsigned)v);
-      }
-    }
-    if (fr.pflag) {
-      unsigned f = 1u | ((fr.pflag == PFLAG_INTERP_PRIM) ? 2u : 4u) | ((fr.boundary & 1) ? 8u : 0u) |
-                   ((fr.boundary & 2) ? 16u : 0u);
-      atomicOr(&s_flags, f);
-    }
-  }
-  if (vmax_slot >= 0) {
-    const unsigned long long m = wave_max_u64(active ? dbl_bits(fr.vmax) : 0ull);
-    if ((tid & 63) == 0 && m) atomicMax(&s_vmax, m);
-  }
-  __syncthreads();
-  if (tid < N_NFAIL && s_cnt[tid]) atomicAdd(&X.status[ST_NFAILTOT + tid], (unsigned long long)s_cnt[tid]);
-  if (tid == 0) {
-    const unsigned f = s_flags;
-    if (f) {
-      atomicOr(&X.status[ST_FAILURE_EXISTS], 1ull);
-      if (f & 2u) atomicOr(&X.status[ST_FAILTYPE_PRIM], 1ull);
-      if (f & 4u) atomicOr(&X.status[ST_FAILTYPE_V], 1ull);
-      if (f & 8u) atomicOr(&X.status[ST_BOUNDARY_PHYS], 1ull);
-      if (f & 16u) atomicOr(&X.status[ST_BOUNDARY_MPI], 1ull);
-    }
-    if (vmax_slot >= 0 && s_vmax) atomicMax(&X.status[ST_VMAX + vmax_slot], s_vmax);
-  }
-}
-
-// Work decomposition of the stencil kernels.  The index box is cut into
-// x1-planes of (j,k) and each plane into tiles of one workgroup: either bs
-// consecutive (j,k) points (k fastest; kc = 0), or kc k-points x bs/kc j-rows
-// (kc > 0).  Hardware dispatches workgroup p to XCD p % 8, and each XCD has its
-// own L2; with remap set, the logical tile of workgroup p is chosen so that
-// every XCD gets one contiguous range of tiles (whole x1-slabs), processed in
-// order, so the +-3-zone stencils of neighbouring tiles hit the same L2.  With
-// order = 1 consecutive workgroups take one (j,k) tile through consecutive
-// x1-planes, so an x1 stencil finds the planes it shares with the previous
-// workgroup in L2.  The shape of each kernel family is picked by the autotuner
-// (or set by the caller).
-struct Tiling {
-  unsigned ni, nj, nk;  // box extents
-  unsigned bs, kc, jr;  // tile: kc x jr (kc > 0) or bs consecutive points (kc = 0)
-  unsigned nkt;         // tiles along k (2D tiles)
-  unsigned X;           // tiles per plane
-  unsigned nblocks;     // X * ni, rounded up to a multiple of 8 when remapped
-  unsigned remap;
-  unsigned order;
-};
-
-static inline Tiling make_tiling(const Box& b, const LaunchShape& L = LaunchShape()) {
-  Tiling T;
-  T.nk = (unsigned)(b.hi[2] - b.lo[2] + 1);
-  T.nj = (unsigned)(b.hi[1] - b.lo[1] + 1);
-  T.ni = (unsigned)(b.hi[0] - b.lo[0] + 1);
-  T.bs = L.bs;
-  T.remap = L.remap;
-  T.order = L.order;
-  if (L.kc > 0 && L.kc < T.nk && L.bs % L.kc == 0) {
-    T.kc = L.kc;
-    T.jr = L.bs / L.kc;
-    T.nkt = (T.nk + T.kc - 1) / T.kc;
-    T.X = T.nkt * ((T.nj + T.jr - 1) / T.jr);
-  } else {
-    T.kc = 0;
-    T.jr = 0;
-    T.nkt = 0;
-    T.X = (T.nj * T.nk + T.bs - 1) / T.bs;
-  }
-  T.nblocks = T.X * T.ni;
-  if (T.remap) T.nblocks = ((T.nblocks + 7u) / 8u) * 8u;
-  return T;
-}
-
-__device__ __forceinline__ bool tile_index(const Box& b, const Tiling& T, int& i, int& j, int& k) {
-  const unsigned p = blockIdx.x;
-  const unsigned L = T.remap ? (p & 7u) * (T.nblocks >> 3) + (p >> 3) : p;
-  unsigned ii, t;
-  if (T.order == 0) {
-    ii = L / T.X;
-    t = L - ii * T.X;
-  } else {
-    t = L / T.ni;
-    ii = L - t * T.ni;
-    if (t >= T.X) return false;
-  }
-  if (ii >= T.ni) return false;
-  unsigned jj, kk;
-  if (T.kc == 0) {
-    const unsigned q = t * T.bs + threadIdx.x;
-    jj = q / T.nk;
-    kk = q - jj * T.nk;
-    if (jj >= T.nj) return false;
-  } else {
-    const unsigned tj = t / T.nkt;
-    const unsigned tk = t - tj * T.nkt;
-    const unsigned r = threadIdx.x / T.kc;
-    kk = tk * T.kc + (threadIdx.x - r * T.kc);
-    jj = tj * T.jr + r;
-    if (kk >= T.nk || jj >= T.nj) return false;
-  }
-  i = b.lo[0] + (int)ii;
-  j = b.lo[1] + (int)jj;
-  k = b.lo[2] + (int)kk;
-  return true;
-}
-
-constexpr unsigned MASK_GAMMA = 1u << NFAIL_GAMMA_CALC;
-constexpr unsigned MASK_ALL = (1u << N_NFAIL) - 1u;
-
-// W: minimum waves per SIMD the register allocation must allow (1 = the
-// compiler's choice; larger values cap the VGPRs, trading spills for occupancy).
-template <int D, int W>
-__global__ __launch_bounds__(BLOCK, W) void k_flux(Params P, Ptrs X, const double* __restrict__ src, Box b, Tiling T) {
-  int i, j, k;
-  const bool active = tile_index(b, T, i, j, k);
-  FailRec fr; fr.clear();
-  long long c = 0;
-  if (active) {
-    flux_face<D>(P, X, src, i, j, k, fr);
-    c = cidx(P, i, j, k);
-  }
-  commit_fail(P, X, fr, active, c, MASK_GAMMA, D + 1);
-}
-
-template <int D, int W>
-__global__ __launch_bounds__(BLOCK, W) void k_flux_mixed(Params P, Ptrs X, const double* __restrict__ src, Box b,
-                                                         Tiling T) {
-  int i, j, k;
-  const bool active = tile_index(b, T, i, j, k);
-  FailRec fr; fr.clear();
-  long long c = 0;
-  if (active) {
-    flux_face_mixed<D>(P, X, src, i, j, k, fr);
-    c = cidx(P, i, j, k);
-  }
-  commit_fail(P, X, fr, active, c, MASK_GAMMA, D + 1);
-}
-
-// Positions and velocities of a level's orbit record (the 12 values the
-// metric records read; not the time derivatives, which only the metric
-// derivatives need): the same address in every lane, read through the
-// scalar cache (constant address space) so they sit in SGPRs.
-__device__ __forceinline__ PnOrbit orbit_load(const PnOrbit* p) {
-  const __attribute__((address_space(4))) double* q = (const __attribute__((address_space(4))) double*)p;
-  PnOrbit o;
-  double* d = &o.y[0][0];
-#pragma unroll
-  for (int m = 0; m < 12; m++) d[m] = q[m];
-  return o;
-}
-
 // The holes' positions and velocities at the step's three levels
 __global__ __launch_bounds__(64) void k_orbit(Ptrs X, PnBinary B, PnOrbit* out) {
   const int l = threadIdx.x;
   if (l < 3) pn_orbit_at(B, level_time(X, l), &out[l]);
-}
-
-__device__ __forceinline__ long long wave_min_ll(long long v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    const long long o = __shfl_xor(v, off, 64);
-    v = (o < v) ? o : v;
-  }
-  return v;
-}
-__device__ __forceinline__ long long wave_max_ll(long long v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    const long long o = __shfl_xor(v, off, 64);
-    v = (o > v) ? o : v;
-  }
-  return v;
-}
-
-// LDS capacity (doubles) of one primitive's x3 pencil of a wavefront: 64 face
-// groups of F faces need 64 F + 5 consecutive zones, plus the ghost zones
-// skipped where the wavefront's groups continue on the next (i,j) row.
-template <int F> constexpr int stage_cap() { return 64 * F + 5 + 3 * (F + 8); }
-
-// PPM+MC face states of the F consecutive x3 faces of every lane (ppm_faces()
-// with d = 2) from LDS-staged pencils.  The zones the wavefront's stencils
-// cover form one contiguous range of the array (k is its fastest index), so
-// each primitive's range is loaded once, coalesced, by all 64 lanes (about
-// F + 1 loads per lane instead of F + 5), stored to LDS, and each lane reads
-// its F + 5 window from there; the next primitive's loads are in flight
-// while this one's limiters run (double-buffered).  A wavefront whose range
-// exceeds the buffer (rows shorter than the wavefront) reads its windows from
-// global memory instead.  Same values, same arithmetic as ppm_faces(): the
-// face states are bit-identical.  Every lane of the wavefront must call it;
-// inactive lanes only help stage.
-template <int F>
-__device__ void ppm_faces_x3_staged(const Params& P, const Ptrs& X, const double* __restrict__ src, bool active,
-                                    int i, int j, int k, double (*pl)[NP], double (*pr)[NP], double* buf) {
-  constexpr int M = F + 5;
-  constexpr int CAP = stage_cap<F>();
-  constexpr int NL = (CAP + 63) / 64;
-  const long long NT = P.nt;
-  const int lane = threadIdx.x & 63;
-  int ii = i, jj = j;
-  if (P.degen[0]) ii = NG;
-  if (P.degen[1]) jj = NG;
-  const long long c0 = active ? cidx(P, ii, jj, k - 3) : 0;
-  int zm[M];
-#pragma unroll
-  for (int m = 0; m < M; m++) zm[m] = imin(m, P.n3t - 1 - (k - 3));
-  const long long lo = wave_min_ll(active ? c0 : LLONG_MAX);
-  const long long hi = wave_max_ll(active ? c0 + zm[M - 1] : LLONG_MIN);
-  const long long span = (hi >= lo) ? hi - lo + 1 : 0;
-  const bool staged = span > 0 && span <= CAP;   // wavefront-uniform
-  const int off = (int)(c0 - lo);
-  double r[NL];
-  if (staged) {
-#pragma unroll
-    for (int q = 0; q < NL; q++) {
-      const int e = q * 64 + lane;
-      r[q] = (e < span) ? src[lo + e] : 0.;
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < NP; v++) {
-    double* bv = buf + (v & 1) * CAP;
-    if (staged) {
-#pragma unroll
-      for (int q = 0; q < NL; q++) {
-        const int e = q * 64 + lane;
-        if (e < span) bv[e] = r[q];
-      }
-      if (v + 1 < NP) {
-#pragma unroll
-        for (int q = 0; q < NL; q++) {
-          const int e = q * 64 + lane;
-          r[q] = (e < span) ? src[(v + 1) * NT + lo + e] : 0.;
-        }
-      }
-    }
-    // the wavefront's own buffer: LDS operations of one wavefront complete in
-    // order, so a wavefront-scope fence (no workgroup barrier) orders the
-    // stores before the other lanes' reads
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (active) {
-      const int s = rs_slot(v);
-      const double ra = X.rscale[s * P.n1t + ii], ri = X.irscale[s * P.n1t + ii];
-      double y[M];
-#pragma unroll
-      for (int m = 0; m < M; m++) {
-        const double raw = staged ? bv[off + zm[m]] : src[v * NT + c0 + zm[m]];
-        y[m] = (raw * ra) * ri;
-      }
-      double dq[M - 1], fi[M - 2], le[M - 2], re[M - 2];
-#pragma unroll
-      for (int m = 1; m < M - 1; m++) dq[m] = mc_slope_vect(y[m - 1], y[m], y[m + 1]);
-#pragma unroll
-      for (int m = 1; m < M - 2; m++) fi[m] = 0.5 * (y[m + 1] + y[m]) - PPM_FACTOR * (dq[m + 1] - dq[m]);
-#pragma unroll
-      for (int m = 2; m < M - 2; m++) ppm_limit(fi[m - 1], fi[m], y[m], &le[m], &re[m]);
-#pragma unroll
-      for (int f = 0; f < F; f++) {
-        pl[f][v] = re[2 + f];
-        pr[f][v] = le[3 + f];
-      }
-    }
-  }
-}
-
-// F consecutive faces along D per thread (PPM+MC, D not degenerate): the
-// thread's tile index along D counts groups of F faces from bg.lo[D]; faces
-// past hi_d (the flux box end) are skipped.  Each zone's parabola is computed
-// once per group.  The per-face fail() tally goes to the face's zone here,
-// the block totals through commit_fail().
-// Along x3 (the fastest index of the arrays) a lane's F faces are adjacent in
-// memory, so the fluxes go through LDS: slot s of lane l stores element
-// s*64 + l of the wavefront's F*64 faces, and each store instruction writes
-// consecutive faces.
-// OTF: the face records are evaluated from the orbit of level lvl (binary
-// metric) instead of read.
-// STG (x3, FP64): reconstruction from LDS-staged pencils (ppm_faces_x3_staged).
-template <int D, int F, int W, bool MIXED, bool OTF = false, bool STG = false>
-__global__ __launch_bounds__(BLOCK, W) void k_flux_multi(Params P, Ptrs X, const double* __restrict__ src, Box bg,
-                                                         Tiling T, int hi_d, PnGrid G, int lvl) {
-  using Real = typename std::conditional<MIXED, float, double>::type;
-  static_assert(!STG || (D == 2 && !MIXED && !OTF), "staged pencils: FP64 x3 faces of a static metric");
-  constexpr bool TRANSPOSE = (D == 2);
-  __shared__ Real tbuf[TRANSPOSE ? BLOCK * F : 1];
-  __shared__ double sbuf[STG ? (BLOCK / 64) * 2 * stage_cap<F>() : 1];
-  int i, j, k;
-  const bool active = tile_index(bg, T, i, j, k);
-  FailRec fr; fr.clear();
-  Real fo[F][NP];
-  long long cb = 0;
-  int nv = 0;
-  Real pl[F][NP], pr[F][NP];
-  if (active) {
-    const int lo = bg.lo[D];
-    if (D == 0) i = lo + (i - lo) * F;
-    else if (D == 1) j = lo + (j - lo) * F;
-    else k = lo + (k - lo) * F;
-  }
-  if constexpr (STG) ppm_faces_x3_staged<F>(P, X, src, active, i, j, k, pl, pr, sbuf + (threadIdx.x >> 6) * 2 * stage_cap<F>());
-  if (active) {
-    constexpr int di = (D == 0), dj = (D == 1), dk = (D == 2);
-    const int nvalid = min(F, hi_d - ((D == 0) ? i : ((D == 1) ? j : k)) + 1);
-    if constexpr (STG) {
-    } else if constexpr (MIXED) {
-      ppm_faces_mixed<D, F>(P, X, src, i, j, k, pl, pr);
-    } else {
-      ppm_faces<D, F>(P, X, src, i, j, k, pl, pr);
-    }
-    PnOrbit orb;
-    if constexpr (OTF) orb = orbit_load(X.orbit + lvl);
-#pragma unroll
-    for (int f = 0; f < F; f++) {
-      if (f >= nvalid) break;
-      const int g0 = fr.nf[NFAIL_GAMMA_CALC];
-      const int fi = i + f*di, fj = j + f*dj, fk = k + f*dk;
-      if constexpr (OTF) {
-        if constexpr (MIXED) {
-          GeomF gfb;
-          pn_zone_geomf(P, G, orb, fi, fj, fk, D, &gfb);
-          flux_riemann_mixed_g<D>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr, &gfb);
-        } else {
-          Geom gb;
-          pn_zone_geom(P, G, orb, fi, fj, fk, D, &gb);
-          flux_riemann_g<D>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr, &gb);
-        }
-      } else {
-        if constexpr (MIXED) flux_riemann_mixed<D>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr);
-        else flux_riemann<D>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr);
-      }
-      const int dv = fr.nf[NFAIL_GAMMA_CALC] - g0;
-      if (P.track_nfail && dv) X.nfail[NFAIL_GAMMA_CALC*P.nt + cidx(P, fi, fj, fk)] += dv;
-    }
-    cb = cidx(P, i, j, k);
-    nv = nvalid;
-  }
-  if constexpr (TRANSPOSE) {
-    Real* Fa = MIXED ? (Real*)X.Ff : (Real*)X.F;
-    const int lane = threadIdx.x & 63;
-    Real* wbuf = tbuf + (threadIdx.x & ~63) * F;
-    long long cs[F];
-    bool ok[F];
-#pragma unroll
-    for (int s = 0; s < F; s++) {
-      const int e = s*64 + lane, sl = e / F, f = e % F;
-      cs[s] = __shfl(cb, sl, 64) + f;
-      ok[s] = f < __shfl(nv, sl, 64);
-    }
-#pragma unroll
-    for (int l = 0; l < NP; l++) {
-      if (l == B3) continue;   // the normal field's flux: never read
-      __syncthreads();
-#pragma unroll
-      for (int f = 0; f < F; f++) wbuf[lane*F + f] = fo[f][l];
-      __syncthreads();
-#pragma unroll
-      for (int s = 0; s < F; s++)
-        if (ok[s]) Fa[(2*NFLUX + l)*(long long)P.nt + cs[s]] = wbuf[s*64 + lane];
-    }
-  }
-  commit_fail(P, X, fr, active, 0, MASK_GAMMA, D + 1, false);
-}
-
-// Face fluxes along D with launch shape L: one face per thread, or fpt faces
-// per thread (PPM+MC with D not degenerate) over the box of face groups.
-template <int D, int F, bool MIXED>
-static void launch_flux_multi(const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, const Box& b,
-                              hipStream_t st, const PnGrid& G, int lvl) {
-  Box bg = b;
-  const int n = b.hi[D] - b.lo[D] + 1;
-  bg.hi[D] = b.lo[D] + (n + F - 1) / F - 1;
-  const Tiling T = make_tiling(bg, L);
-  const dim3 grid(T.nblocks), blk(T.bs);
-  if (P.otf) {
-    // three waves per SIMD fit the FP32 face solve without spilling
-    if constexpr (MIXED) hipLaunchKernelGGL((k_flux_multi<D, F, 3, true, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
-    else hipLaunchKernelGGL((k_flux_multi<D, F, 1, false, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
-    return;
-  }
-  if constexpr (D == 2 && !MIXED) {
-    if (L.stage) {   // reconstruction from LDS-staged pencils
-      if (L.occ) hipLaunchKernelGGL((k_flux_multi<D, F, 3, false, false, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
-      else hipLaunchKernelGGL((k_flux_multi<D, F, 1, false, false, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
-      return;
-    }
-  }
-  // register-capped variants: 4 waves/SIMD for the FP32 solve, 3 for FP64
-  if (L.occ) {
-    if constexpr (MIXED) hipLaunchKernelGGL((k_flux_multi<D, F, 4, true>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
-    else hipLaunchKernelGGL((k_flux_multi<D, F, 3, false>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
-  } else {
-    hipLaunchKernelGGL((k_flux_multi<D, F, 1, MIXED>), grid, blk, 0, st, P, X, src, bg, T, b.hi[D], G, lvl);
-  }
-}
-
-// G, lvl: the binary metric's grid and the stage's level, read when P.otf
-// (which implies PPM and no degenerate direction: the face-group kernels,
-// with at least 2 faces per thread).
-template <int D>
-static void launch_flux_dir(const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, const Box& b,
-                            hipStream_t st, const PnGrid& G, int lvl) {
-  if ((L.fpt > 1 || P.otf) && P.recon == RECON_PPM_MC && !P.degen[D]) {
-    if (P.mixed) {
-      if (L.fpt == 4) launch_flux_multi<D, 4, true>(P, X, L, src, b, st, G, lvl);
-      else launch_flux_multi<D, 2, true>(P, X, L, src, b, st, G, lvl);
-    } else {
-      if (L.fpt == 4) launch_flux_multi<D, 4, false>(P, X, L, src, b, st, G, lvl);
-      else launch_flux_multi<D, 2, false>(P, X, L, src, b, st, G, lvl);
-    }
-    return;
-  }
-  const Tiling T = make_tiling(b, L);
-  const dim3 grid(T.nblocks), blk(T.bs);
-  if (P.mixed) {
-    if (L.occ) hipLaunchKernelGGL((k_flux_mixed<D, 6>), grid, blk, 0, st, P, X, src, b, T);
-    else hipLaunchKernelGGL((k_flux_mixed<D, 1>), grid, blk, 0, st, P, X, src, b, T);
-  } else {
-    if (L.occ) hipLaunchKernelGGL((k_flux<D, 4>), grid, blk, 0, st, P, X, src, b, T);
-    else hipLaunchKernelGGL((k_flux<D, 1>), grid, blk, 0, st, P, X, src, b, T);
-  }
 }
 
 __global__ __launch_bounds__(BLOCK) void k_emf(Params P, Ptrs X, Box b, Tiling T) {
@@ -659,7 +192,8 @@ __global__ __launch_bounds__(BLOCK) void k_invert(Params P, Ptrs X, int stage, B
 // evaluated records); each kernel carries only its metric's source branch.
 // UNI: row-aligned tiles (each wavefront in one (i, j) column of a 2D static
 // metric): the connection records are read through the scalar cache.
-template <bool MIXED, int W, bool OTF = false, int MET = 0, bool UNI = false>
+// K: structure of the static metric's records (GK_*).
+template <bool MIXED, int W, bool OTF = false, int MET = 0, bool UNI = false, int K = GK_GEN>
 __global__ __launch_bounds__(BLOCK, W) void k_update(Params P, Ptrs X, int stage, Box b, Tiling T, PnGrid G,
                                                      int lvl) {
   int i, j, k;
@@ -682,17 +216,18 @@ __global__ __launch_bounds__(BLOCK, W) void k_update(Params P, Ptrs X, int stage
       {
         Geom gs;
         if (stage == 0) pn_zone_geom(P, G, orbit_load(X.orbit + lvl), i, j, k, CENT, &gs);
-        zone_conserved<MIXED, 2>(P, X, stage, (stage == 0) ? 0.5*dt : dt, i, j, k, &gs, &gs, fr, U);
+        const GeomView<GK_DIAG, const Geom*> gv{&gs};
+        zone_conserved<MIXED, 2>(P, X, stage, (stage == 0) ? 0.5*dt : dt, i, j, k, gv, gv, fr, U);
       }
       Geom gnew;
       pn_zone_geom(P, G, orbit_load(X.orbit + lvl + 1), i, j, k, CENT, &gnew);
       double pf[NP];
       zone_guess(P, X, stage, i, c, pf);
       double pgam = 1.;
-      done = recover_fast(P, X, i, j, k, pf, U, &gnew, floor_rho(P, X, i, c), floor_uu(P, X, i, c), &pgam, fr);
+      done = recover_fast(P, X, i, j, k, pf, U, GeomView<GK_DIAG, const Geom*>{&gnew}, floor_rho(P, X, i, c), floor_uu(P, X, i, c), &pgam, fr);
       if (done) store_zone(P, X, stage, c, pf, pgam, fr);
     } else {
-      done = update_zone_fast<MIXED, MET, UNI>(P, X, stage, dt, i, j, k, fr, U);
+      done = update_zone_fast<MIXED, MET, UNI, K>(P, X, stage, dt, i, j, k, fr, U);
     }
     urho = U[RHO];
     if (!done) {
@@ -983,7 +518,7 @@ __global__ __launch_bounds__(BLOCK, 2) void k_source_otf(Params P, Ptrs X, PnGri
       double phz[NP];
 #pragma unroll
       for (int v = 0; v < NP; v++) phz[v] = rt_val(P, X, v, i, src[v*P.nt + c]);
-      source_dyn_state(P, X, phz, &gs, i, sd);
+      source_dyn_state(P, X, phz, GeomView<GK_DIAG, const Geom*>{&gs}, i, sd);
       gdet = gs.g;
     }
     double Xc[4];
@@ -1272,25 +807,28 @@ struct GpuBE {
     }
     // row-aligned flat tiles: every wavefront's 64 zones share one (i, j)
     const bool uni = c->P.metric_dim == 2 && !c->P.flat && T.kc == 0 && T.nk % 64 == 0 && T.bs % 64 == 0;
-    if (c->P.mixed) {
-      if (uni) {
-        // capped at 4 waves per SIMD (some registers spilled): 5 % faster
-        // than at 3 on the 192x192x128 torus
-        if (L.occ) hipLaunchKernelGGL((k_update<true, 4, false, 0, true>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
-        else hipLaunchKernelGGL((k_update<true, 1, false, 0, true>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
-      } else {
-        if (L.occ) hipLaunchKernelGGL((k_update<true, 3>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
-        else hipLaunchKernelGGL((k_update<true, 1>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
+    // capped variants: 3 waves per SIMD; the mixed-precision row-aligned one 4
+    // (some registers spilled): 5 % faster than at 3 on the 192x192x128 torus
+    const auto go = [&](auto M, auto K) {
+      constexpr bool m = decltype(M)::value;
+      constexpr int k = decltype(K)::value;
+      if constexpr (k != GK_FLAT) {
+        if (uni) {
+          if (L.occ) hipLaunchKernelGGL((k_update<m, m ? 4 : 3, false, 0, true, k>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
+          else hipLaunchKernelGGL((k_update<m, 1, false, 0, true, k>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
+          return;
+        }
       }
-    } else {
-      if (uni) {
-        if (L.occ) hipLaunchKernelGGL((k_update<false, 3, false, 0, true>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
-        else hipLaunchKernelGGL((k_update<false, 1, false, 0, true>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
-      } else {
-        if (L.occ) hipLaunchKernelGGL((k_update<false, 3>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
-        else hipLaunchKernelGGL((k_update<false, 1>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
-      }
-    }
+      if (L.occ) hipLaunchKernelGGL((k_update<m, 3, false, 0, false, k>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
+      else hipLaunchKernelGGL((k_update<m, 1, false, 0, false, k>), grid, blk, 0, st, c->P, c->X, stage, b, T, G, lvl);
+    };
+    const auto kind = [&](auto M) {
+      if (c->P.gkind == GK_FLAT) go(M, std::integral_constant<int, GK_FLAT>());
+      else if (c->P.gkind == GK_KS) go(M, std::integral_constant<int, GK_KS>());
+      else go(M, std::integral_constant<int, GK_GEN>());
+    };
+    if (c->P.mixed) kind(std::true_type());
+    else kind(std::false_type());
   }
   // The autotuner times the conserved-update family as the whole predictor
   // update (split pair or fused kernel), which writes only arrays that the
@@ -1451,13 +989,8 @@ struct GpuBE {
     return hip_check(hipGetLastError(), "k_reset_words");
   }
   static int flux(hgpu_ctx* c, const double* src, int d) {
-    Box b = flux_box(c->P, d);
     Scope s(c, "flux");
-    const LaunchShape& L = priv(c)->shape[FAM_FLUX1 + d];
-    hipStream_t st = priv(c)->stream;
-    if (d == 0) launch_flux_dir<0>(c->P, c->X, L, src, b, st, c->pn, c->otf_stage);
-    else if (d == 1) launch_flux_dir<1>(c->P, c->X, L, src, b, st, c->pn, c->otf_stage);
-    else launch_flux_dir<2>(c->P, c->X, L, src, b, st, c->pn, c->otf_stage);
+    launch_flux_dir(d, c->P, c->X, priv(c)->shape[FAM_FLUX1 + d], src, priv(c)->stream, c->pn, c->otf_stage);
     return hip_check(hipGetLastError(), "k_flux");
   }
   static int emf(hgpu_ctx* c) {

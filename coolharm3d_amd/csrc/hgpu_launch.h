@@ -1,0 +1,190 @@
+// hgpu_launch.h -- launch shapes, the tile decomposition and the workgroup
+// reductions shared by the device translation units of the advance
+// (hgpu_kernels.hip, hgpu_flux.hip).
+#pragma once
+#include "hgpu_core.h"
+#include <hip/hip_runtime.h>
+#include <algorithm>
+#include <type_traits>
+
+namespace hgpu {
+
+constexpr int BLOCK = 256;
+
+// Launch shape of a stencil-kernel family (tile decomposition below).
+struct LaunchShape {
+  unsigned bs = 256;     // threads per workgroup: 64, 128 or 256
+  unsigned kc = 0;       // k-extent of a 2D tile, dividing bs; 0 = flat tiles
+  unsigned remap = 1;    // XCD-contiguous tile order
+  unsigned order = 0;    // 0: plane after plane; 1: x1 fastest (one (j,k) tile through consecutive planes)
+  unsigned occ = 0;      // 1: the register-capped kernel variant (flux, conserved update)
+  unsigned fused = 0;    // conserved update only: 1 = update and inversion in one kernel
+  unsigned fpt = 1;      // face fluxes only: faces per thread along the direction (1, 2, 4)
+  unsigned stage = 0;    // x3 face fluxes (FP64, PPM, fpt > 1): reconstruction from LDS-staged pencils
+};
+enum { FAM_FLUX1 = 0, FAM_FLUX2, FAM_FLUX3, FAM_EMF, FAM_CONS, FAM_INV, N_FAM };
+
+
+// --------------------------------------------------------------------------
+__device__ __forceinline__ int wave_sum(int v) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned long long o = __shfl_xor(v, off, 64);
+    v = (o > v) ? o : v;
+  }
+  return v;
+}
+
+// Writes the fail() tallies of a workgroup: per-zone nfail, and block totals of
+// nfailtot, the failure words and the fastest face speed (vmax_slot >= 0),
+// reduced in LDS so each status word receives at most one atomic per
+// workgroup.  Every thread of the block must call it.
+__device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, const FailRec& fr,
+                                            bool active, long long c, unsigned mask, int vmax_slot = -1,
+                                            bool zone_map = true) {
+  __shared__ unsigned s_cnt[N_NFAIL];
+  __shared__ unsigned s_flags;
+  __shared__ unsigned long long s_vmax;
+  const long long NT = P.nt;
+  const int tid = threadIdx.x;
+  if (tid < N_NFAIL) s_cnt[tid] = 0;
+  if (tid == 0) { s_flags = 0; s_vmax = 0; }
+  __syncthreads();
+  if (active) {
+    for (int l = 0; l < N_NFAIL; l++) {
+      if (!(mask & (1u << l))) continue;
+      const int v = fr.nf[l];
+      if (v) {
+        if (P.track_nfail && zone_map) X.nfail[l*NT + c] += v;
+        atomicAdd(&s_cnt[l], (unsigned)v);
+      }
+    }
+    if (fr.pflag) {
+      unsigned f = 1u | ((fr.pflag == PFLAG_INTERP_PRIM) ? 2u : 4u) | ((fr.boundary & 1) ? 8u : 0u) |
+                   ((fr.boundary & 2) ? 16u : 0u);
+      atomicOr(&s_flags, f);
+    }
+  }
+  if (vmax_slot >= 0) {
+    const unsigned long long m = wave_max_u64(active ? dbl_bits(fr.vmax) : 0ull);
+    if ((tid & 63) == 0 && m) atomicMax(&s_vmax, m);
+  }
+  __syncthreads();
+  if (tid < N_NFAIL && s_cnt[tid]) atomicAdd(&X.status[ST_NFAILTOT + tid], (unsigned long long)s_cnt[tid]);
+  if (tid == 0) {
+    const unsigned f = s_flags;
+    if (f) {
+      atomicOr(&X.status[ST_FAILURE_EXISTS], 1ull);
+      if (f & 2u) atomicOr(&X.status[ST_FAILTYPE_PRIM], 1ull);
+      if (f & 4u) atomicOr(&X.status[ST_FAILTYPE_V], 1ull);
+      if (f & 8u) atomicOr(&X.status[ST_BOUNDARY_PHYS], 1ull);
+      if (f & 16u) atomicOr(&X.status[ST_BOUNDARY_MPI], 1ull);
+    }
+    if (vmax_slot >= 0 && s_vmax) atomicMax(&X.status[ST_VMAX + vmax_slot], s_vmax);
+  }
+}
+
+// Work decomposition of the stencil kernels.  The index box is cut into
+// x1-planes of (j,k) and each plane into tiles of one workgroup: either bs
+// consecutive (j,k) points (k fastest; kc = 0), or kc k-points x bs/kc j-rows
+// (kc > 0).  Hardware dispatches workgroup p to XCD p % 8, and each XCD has its
+// own L2; with remap set, the logical tile of workgroup p is chosen so that
+// every XCD gets one contiguous range of tiles (whole x1-slabs), processed in
+// order, so the +-3-zone stencils of neighbouring tiles hit the same L2.  With
+// order = 1 consecutive workgroups take one (j,k) tile through consecutive
+// x1-planes, so an x1 stencil finds the planes it shares with the previous
+// workgroup in L2.  The shape of each kernel family is picked by the autotuner
+// (or set by the caller).
+struct Tiling {
+  unsigned ni, nj, nk;  // box extents
+  unsigned bs, kc, jr;  // tile: kc x jr (kc > 0) or bs consecutive points (kc = 0)
+  unsigned nkt;         // tiles along k (2D tiles)
+  unsigned X;           // tiles per plane
+  unsigned nblocks;     // X * ni, rounded up to a multiple of 8 when remapped
+  unsigned remap;
+  unsigned order;
+};
+
+static inline Tiling make_tiling(const Box& b, const LaunchShape& L = LaunchShape()) {
+  Tiling T;
+  T.nk = (unsigned)(b.hi[2] - b.lo[2] + 1);
+  T.nj = (unsigned)(b.hi[1] - b.lo[1] + 1);
+  T.ni = (unsigned)(b.hi[0] - b.lo[0] + 1);
+  T.bs = L.bs;
+  T.remap = L.remap;
+  T.order = L.order;
+  if (L.kc > 0 && L.kc < T.nk && L.bs % L.kc == 0) {
+    T.kc = L.kc;
+    T.jr = L.bs / L.kc;
+    T.nkt = (T.nk + T.kc - 1) / T.kc;
+    T.X = T.nkt * ((T.nj + T.jr - 1) / T.jr);
+  } else {
+    T.kc = 0;
+    T.jr = 0;
+    T.nkt = 0;
+    T.X = (T.nj * T.nk + T.bs - 1) / T.bs;
+  }
+  T.nblocks = T.X * T.ni;
+  if (T.remap) T.nblocks = ((T.nblocks + 7u) / 8u) * 8u;
+  return T;
+}
+
+__device__ __forceinline__ bool tile_index(const Box& b, const Tiling& T, int& i, int& j, int& k) {
+  const unsigned p = blockIdx.x;
+  const unsigned L = T.remap ? (p & 7u) * (T.nblocks >> 3) + (p >> 3) : p;
+  unsigned ii, t;
+  if (T.order == 0) {
+    ii = L / T.X;
+    t = L - ii * T.X;
+  } else {
+    t = L / T.ni;
+    ii = L - t * T.ni;
+    if (t >= T.X) return false;
+  }
+  if (ii >= T.ni) return false;
+  unsigned jj, kk;
+  if (T.kc == 0) {
+    const unsigned q = t * T.bs + threadIdx.x;
+    jj = q / T.nk;
+    kk = q - jj * T.nk;
+    if (jj >= T.nj) return false;
+  } else {
+    const unsigned tj = t / T.nkt;
+    const unsigned tk = t - tj * T.nkt;
+    const unsigned r = threadIdx.x / T.kc;
+    kk = tk * T.kc + (threadIdx.x - r * T.kc);
+    jj = tj * T.jr + r;
+    if (kk >= T.nk || jj >= T.nj) return false;
+  }
+  i = b.lo[0] + (int)ii;
+  j = b.lo[1] + (int)jj;
+  k = b.lo[2] + (int)kk;
+  return true;
+}
+
+constexpr unsigned MASK_GAMMA = 1u << NFAIL_GAMMA_CALC;
+constexpr unsigned MASK_ALL = (1u << N_NFAIL) - 1u;
+
+// Positions and velocities of a level's orbit record (the 12 values the
+// metric records read; not the time derivatives, which only the metric
+// derivatives need): the same address in every lane, read through the
+// scalar cache (constant address space) so they sit in SGPRs.
+__device__ __forceinline__ PnOrbit orbit_load(const PnOrbit* p) {
+  const __attribute__((address_space(4))) double* q = (const __attribute__((address_space(4))) double*)p;
+  PnOrbit o;
+  double* d = &o.y[0][0];
+#pragma unroll
+  for (int m = 0; m < 12; m++) d[m] = q[m];
+  return o;
+}
+
+
+// hgpu_flux.hip: face fluxes of direction d with launch shape L
+void launch_flux_dir(int d, const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, hipStream_t st,
+                     const PnGrid& G, int lvl);
+
+}  // namespace hgpu

@@ -67,14 +67,50 @@ struct StateF {
   float opu_t;     // 1 + u_t without cancellation
 };
 
-HD void lower_f(const float* v, const GeomF* g, float* w) {
+// The record's pointer may be a GeomView (its structure decides which terms are
+// formed: lower_f() and spatial_sq_f() below).  Both are restated here, inside
+// the region whose multiply-adds fuse.
+template <class GP>
+HD void lower_f(const float* v, GP g, float* w) {
+  constexpr int K = geom_kind<GP>::value;
+  if constexpr (K == GK_FLAT) {
+    w[0] = -v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
+  } else if constexpr (K == GK_KS) {
+    w[0] = g->gcov[0][0]*v[0] + g->gcov[0][1]*v[1] + g->gcov[0][3]*v[3];
+    w[1] = g->gcov[0][1]*v[0] + g->gcov[1][1]*v[1] + g->gcov[1][3]*v[3];
+    w[2] = g->gcov[2][2]*v[2];
+    w[3] = g->gcov[0][3]*v[0] + g->gcov[1][3]*v[1] + g->gcov[3][3]*v[3];
+  } else if constexpr (K == GK_DIAG) {
+    w[0] = g->gcov[0][0]*v[0] + g->gcov[0][1]*v[1] + g->gcov[0][2]*v[2] + g->gcov[0][3]*v[3];
+    w[1] = g->gcov[0][1]*v[0] + g->gcov[1][1]*v[1];
+    // the general sum fuses its last products into the rounded first one
+    w[2] = g->gcov[2][2]*v[2] + g->gcov[0][2]*v[0];
+    w[3] = g->gcov[3][3]*v[3] + g->gcov[0][3]*v[0];
+  } else {
 #pragma unroll
-  for (int m = 0; m < 4; m++) w[m] = g->gcov[m][0]*v[0] + g->gcov[m][1]*v[1] + g->gcov[m][2]*v[2] + g->gcov[m][3]*v[3];
+    for (int m = 0; m < 4; m++)
+      w[m] = g->gcov[m][0]*v[0] + g->gcov[m][1]*v[1] + g->gcov[m][2]*v[2] + g->gcov[m][3]*v[3];
+  }
+}
+template <class GP>
+HD float spatial_sq_f(const float* v, GP g) {
+  constexpr int K = geom_kind<GP>::value;
+  if constexpr (K == GK_FLAT) {
+    return v[0]*v[0] + v[1]*v[1] + v[2]*v[2];
+  } else if constexpr (K == GK_KS) {
+    return g->gcov[1][1]*v[0]*v[0] + g->gcov[2][2]*v[1]*v[1] + g->gcov[3][3]*v[2]*v[2]
+         + 2.f*(g->gcov[1][3]*v[0]*v[2]);
+  } else if constexpr (K == GK_DIAG) {
+    return g->gcov[1][1]*v[0]*v[0] + g->gcov[2][2]*v[1]*v[1] + g->gcov[3][3]*v[2]*v[2];
+  } else {
+    return g->gcov[1][1]*v[0]*v[0] + g->gcov[2][2]*v[1]*v[1] + g->gcov[3][3]*v[2]*v[2]
+         + 2.f*(g->gcov[1][2]*v[0]*v[1] + g->gcov[1][3]*v[0]*v[2] + g->gcov[2][3]*v[1]*v[2]);
+  }
 }
 
-HD int gamma_calc_f(const float* pr, const GeomF* g, float* gamma, float* qsq_out) {
-  float qsq = g->gcov[1][1]*pr[U1]*pr[U1] + g->gcov[2][2]*pr[U2]*pr[U2] + g->gcov[3][3]*pr[U3]*pr[U3]
-            + 2.f*(g->gcov[1][2]*pr[U1]*pr[U2] + g->gcov[1][3]*pr[U1]*pr[U3] + g->gcov[2][3]*pr[U2]*pr[U3]);
+template <class GP>
+HD int gamma_calc_f(const float* pr, GP g, float* gamma, float* qsq_out) {
+  float qsq = spatial_sq_f(pr + U1, g);
   if (qsq < 0.f) {
     if (fabsf(qsq) > 1.E-10f) { *gamma = 1.f; *qsq_out = 0.f; return 1; }
     qsq = 1.E-10f;
@@ -84,15 +120,32 @@ HD int gamma_calc_f(const float* pr, const GeomF* g, float* gamma, float* qsq_ou
   return 0;
 }
 
-HD int get_state_f(const float* pr, const GeomF* g, float gam, StateF* q) {
+template <class GP>
+HD int get_state_f(const float* pr, GP g, float gam, StateF* q) {
+  constexpr int K = geom_kind<GP>::value;
   float gamma, qsq;
   int fl = gamma_calc_f(pr, g, &gamma, &qsq);
-  q->opu_t = gamma*g->om_alpha - qsq*rcp_f(gamma + 1.f)
-           + (g->gcov[0][1]*pr[U1] + g->gcov[0][2]*pr[U2] + g->gcov[0][3]*pr[U3]);
-  q->ucon[0] = gamma*g->ncon[0];
-  q->ucon[1] = pr[U1] - q->ucon[0]*g->beta[0];
-  q->ucon[2] = pr[U2] - q->ucon[0]*g->beta[1];
-  q->ucon[3] = pr[U3] - q->ucon[0]*g->beta[2];
+  if constexpr (K == GK_FLAT) {
+    q->opu_t = -(qsq*rcp_f(gamma + 1.f));
+    q->ucon[0] = gamma;
+    q->ucon[1] = pr[U1];
+  } else {
+    if constexpr (K == GK_KS)
+      // the last product fused into the rounded first one, as in the general sum
+      q->opu_t = gamma*g->om_alpha - qsq*rcp_f(gamma + 1.f) + (g->gcov[0][3]*pr[U3] + g->gcov[0][1]*pr[U1]);
+    else
+      q->opu_t = gamma*g->om_alpha - qsq*rcp_f(gamma + 1.f)
+               + (g->gcov[0][1]*pr[U1] + g->gcov[0][2]*pr[U2] + g->gcov[0][3]*pr[U3]);
+    q->ucon[0] = gamma*g->ncon[0];
+    q->ucon[1] = pr[U1] - q->ucon[0]*g->beta[0];
+  }
+  if constexpr (K == GK_FLAT || K == GK_KS) {
+    q->ucon[2] = pr[U2];
+    q->ucon[3] = pr[U3];
+  } else {
+    q->ucon[2] = pr[U2] - q->ucon[0]*g->beta[1];
+    q->ucon[3] = pr[U3] - q->ucon[0]*g->beta[2];
+  }
   lower_f(q->ucon, g, q->ucov);
   float inv_ut = rcp_f(q->ucon[0]);
   q->bcon[0] = pr[B1]*q->ucov[1] + pr[B2]*q->ucov[2] + pr[B3]*q->ucov[3];
@@ -107,8 +160,8 @@ HD int get_state_f(const float* pr, const GeomF* g, float gam, StateF* q) {
   return fl;
 }
 
-template <int dir>
-HD void primtoflux_f(const float* pr, const StateF* q, const GeomF* g, float* flux) {
+template <int dir, class GP>
+HD void primtoflux_f(const float* pr, const StateF* q, GP g, float* flux) {
   const float eu = q->eta*q->ucon[dir], bd = q->bcon[dir];
   float mhd[4];
 #pragma unroll
@@ -124,19 +177,31 @@ HD void primtoflux_f(const float* pr, const StateF* q, const GeomF* g, float* fl
   flux[B1] = q->bcon[1]*q->ucon[dir] - q->bcon[dir]*q->ucon[1];
   flux[B2] = q->bcon[2]*q->ucon[dir] - q->bcon[dir]*q->ucon[2];
   flux[B3] = q->bcon[3]*q->ucon[dir] - q->bcon[dir]*q->ucon[3];
+  if constexpr (geom_kind<GP>::value != GK_FLAT) {
 #pragma unroll
-  for (int l = 0; l < NP; l++) flux[l] *= g->g;
+    for (int l = 0; l < NP; l++) flux[l] *= g->g;
+  }
 }
 
-template <int js>
-HD void vchar_f(const StateF* q, const GeomF* g, float gam, float* vmax, float* vmin) {
+template <int js, class GP>
+HD void vchar_f(const StateF* q, GP g, float gam, float* vmax, float* vmin) {
   float cms2 = (gam*q->p + q->bsq)*rcp_f(q->eta);
   if (cms2 < 0.f) cms2 = (float)SMALL;
   else if (cms2 > 1.f) cms2 = 1.f;
   const float Au2 = q->ucon[js]*q->ucon[js], Bu2 = q->ucon[0]*q->ucon[0], AuBu = q->ucon[js]*q->ucon[0];
-  const float A = Bu2 - (g->gcon[0][0] + Bu2)*cms2;
-  const float B = AuBu - (g->gcon[0][js] + AuBu)*cms2;
-  const float C = Au2 - (g->gcon[js][js] + Au2)*cms2;
+  constexpr int K = geom_kind<GP>::value;
+  float gtt, gtj = 0.f, gjj;
+  if constexpr (K == GK_FLAT) {
+    gtt = -1.f;
+    gjj = 1.f;
+  } else {
+    gtt = g->gcon[0][0];
+    gjj = g->gcon[js][js];
+    if constexpr (K != GK_KS || js == 1) gtj = g->gcon[0][js];
+  }
+  const float A = Bu2 - (gtt + Bu2)*cms2;
+  const float B = AuBu - ((K == GK_FLAT || (K == GK_KS && js != 1)) ? AuBu : gtj + AuBu)*cms2;
+  const float C = Au2 - (gjj + Au2)*cms2;
   float discr = B*B - A*C;
   if (discr < 0.f) discr = 0.f;
   discr = sqrt_f(discr);
@@ -326,9 +391,9 @@ HD void ppm_faces_mixed(const Params& P, const Ptrs& X, const double* __restrict
 
 // FP32 Riemann solve of face (i,j,k) from its two states; fluxes to X.Ff or
 // to out[8]
-template <int d>
+template <int d, class GP>
 HD void flux_riemann_mixed_g(const Params& P, const Ptrs& X, const float* pl, const float* pr,
-                             int i, int j, int k, FailRec& fr, float* out, const GeomF* g) {
+                             int i, int j, int k, FailRec& fr, float* out, GP g) {
   const long long NT = P.nt;
   constexpr int dim = d + 1;
   const float gam = (float)P.gam;
@@ -369,10 +434,11 @@ HD void flux_riemann_mixed_g(const Params& P, const Ptrs& X, const float* pl, co
   }
 }
 
-template <int d>
+template <int d, int K = GK_GEN>
 HD void flux_riemann_mixed(const Params& P, const Ptrs& X, const float* pl, const float* pr,
                            int i, int j, int k, FailRec& fr, float* out = nullptr) {
-  flux_riemann_mixed_g<d>(P, X, pl, pr, i, j, k, fr, out, X.geomf + geom_id(P, i, j, k, d));
+  flux_riemann_mixed_g<d>(P, X, pl, pr, i, j, k, fr, out,
+                          GeomView<K, const GeomF*>{X.geomf + geom_id(P, i, j, k, d)});
 }
 
 // Entropy flux of face (i,j,k) for fixup_entropy_eq() (src/fixup.c:363-398)
@@ -406,12 +472,12 @@ HD double entropy_face_mixed(const Params& P, const Ptrs& X, const double* __res
   return (double)Fs;
 }
 
-template <int d>
+template <int d, int K = GK_GEN>
 HD void flux_face_mixed(const Params& P, const Ptrs& X, const double* __restrict__ src,
                         int i, int j, int k, FailRec& fr) {
   float pl[NP], pr[NP];
   flux_recon_mixed<d>(P, X, src, i, j, k, pl, pr);
-  flux_riemann_mixed<d>(P, X, pl, pr, i, j, k, fr);
+  flux_riemann_mixed<d, K>(P, X, pl, pr, i, j, k, fr);
 }
 
 // Corner EMFs from the FP32 face fluxes (flux_ct_para_fast2(), src/flux_ct.c:780-846;

@@ -65,21 +65,95 @@ HD bool is_finite(double x) { return isfinite(x); }
 // pointer into the constant address space when every lane of the wavefront
 // reads the same record (its fields then load through the scalar cache).
 
-// Metric contractions, src/metric.c:338-383
-template <class GP>
-HD void lower(const double* ucon, GP g, double* ucov) {
-  ucov[0] = g->gcov[0][0]*ucon[0] + g->gcov[0][1]*ucon[1] + g->gcov[0][2]*ucon[2] + g->gcov[0][3]*ucon[3];
-  ucov[1] = g->gcov[1][0]*ucon[0] + g->gcov[1][1]*ucon[1] + g->gcov[1][2]*ucon[2] + g->gcov[1][3]*ucon[3];
-  ucov[2] = g->gcov[2][0]*ucon[0] + g->gcov[2][1]*ucon[1] + g->gcov[2][2]*ucon[2] + g->gcov[2][3]*ucon[3];
-  ucov[3] = g->gcov[3][0]*ucon[0] + g->gcov[3][1]*ucon[1] + g->gcov[3][2]*ucon[2] + g->gcov[3][3]*ucon[3];
+// GP may also be a GeomView, whose structure decides which terms are formed.
+
+// Metric contractions, src/metric.c:338-383.  T: double, or float for the
+// FP32 records.
+template <class GP, class T>
+HD void lower(const T* ucon, GP g, T* ucov) {
+  constexpr int K = geom_kind<GP>::value;
+  if constexpr (K == GK_FLAT) {
+    ucov[0] = -ucon[0]; ucov[1] = ucon[1]; ucov[2] = ucon[2]; ucov[3] = ucon[3];
+  } else if constexpr (K == GK_KS) {
+    ucov[0] = g->gcov[0][0]*ucon[0] + g->gcov[0][1]*ucon[1] + g->gcov[0][3]*ucon[3];
+    ucov[1] = g->gcov[0][1]*ucon[0] + g->gcov[1][1]*ucon[1] + g->gcov[1][3]*ucon[3];
+    ucov[2] = g->gcov[2][2]*ucon[2];
+    ucov[3] = g->gcov[0][3]*ucon[0] + g->gcov[1][3]*ucon[1] + g->gcov[3][3]*ucon[3];
+  } else if constexpr (K == GK_DIAG) {
+    ucov[0] = g->gcov[0][0]*ucon[0] + g->gcov[0][1]*ucon[1] + g->gcov[0][2]*ucon[2] + g->gcov[0][3]*ucon[3];
+    ucov[1] = g->gcov[0][1]*ucon[0] + g->gcov[1][1]*ucon[1];
+    ucov[2] = g->gcov[0][2]*ucon[0] + g->gcov[2][2]*ucon[2];
+    ucov[3] = g->gcov[0][3]*ucon[0] + g->gcov[3][3]*ucon[3];
+  } else {
+    ucov[0] = g->gcov[0][0]*ucon[0] + g->gcov[0][1]*ucon[1] + g->gcov[0][2]*ucon[2] + g->gcov[0][3]*ucon[3];
+    ucov[1] = g->gcov[1][0]*ucon[0] + g->gcov[1][1]*ucon[1] + g->gcov[1][2]*ucon[2] + g->gcov[1][3]*ucon[3];
+    ucov[2] = g->gcov[2][0]*ucon[0] + g->gcov[2][1]*ucon[1] + g->gcov[2][2]*ucon[2] + g->gcov[2][3]*ucon[3];
+    ucov[3] = g->gcov[3][0]*ucon[0] + g->gcov[3][1]*ucon[1] + g->gcov[3][2]*ucon[2] + g->gcov[3][3]*ucon[3];
+  }
 }
 template <class GP>
 HD void raise_v(const double* ucov, GP g, double* ucon) {
-  ucon[0] = g->gcon[0][0]*ucov[0] + g->gcon[0][1]*ucov[1] + g->gcon[0][2]*ucov[2] + g->gcon[0][3]*ucov[3];
-  ucon[1] = g->gcon[1][0]*ucov[0] + g->gcon[1][1]*ucov[1] + g->gcon[1][2]*ucov[2] + g->gcon[1][3]*ucov[3];
-  ucon[2] = g->gcon[2][0]*ucov[0] + g->gcon[2][1]*ucov[1] + g->gcon[2][2]*ucov[2] + g->gcon[2][3]*ucov[3];
-  ucon[3] = g->gcon[3][0]*ucov[0] + g->gcon[3][1]*ucov[1] + g->gcon[3][2]*ucov[2] + g->gcon[3][3]*ucov[3];
+  constexpr int K = geom_kind<GP>::value;
+  if constexpr (K == GK_FLAT) {
+    ucon[0] = -ucov[0]; ucon[1] = ucov[1]; ucon[2] = ucov[2]; ucon[3] = ucov[3];
+  } else if constexpr (K == GK_KS) {
+    ucon[0] = g->gcon[0][0]*ucov[0] + g->gcon[0][1]*ucov[1];
+    ucon[1] = g->gcon[0][1]*ucov[0] + g->gcon[1][1]*ucov[1] + g->gcon[1][3]*ucov[3];
+    ucon[2] = g->gcon[2][2]*ucov[2];
+    ucon[3] = g->gcon[1][3]*ucov[1] + g->gcon[3][3]*ucov[3];
+  } else {
+    ucon[0] = g->gcon[0][0]*ucov[0] + g->gcon[0][1]*ucov[1] + g->gcon[0][2]*ucov[2] + g->gcon[0][3]*ucov[3];
+    ucon[1] = g->gcon[1][0]*ucov[0] + g->gcon[1][1]*ucov[1] + g->gcon[1][2]*ucov[2] + g->gcon[1][3]*ucov[3];
+    ucon[2] = g->gcon[2][0]*ucov[0] + g->gcon[2][1]*ucov[1] + g->gcon[2][2]*ucov[2] + g->gcon[2][3]*ucov[3];
+    ucon[3] = g->gcon[3][0]*ucov[0] + g->gcon[3][1]*ucov[1] + g->gcon[3][2]*ucov[2] + g->gcon[3][3]*ucov[3];
+  }
 }
+// gamma_ij v^i v^j of the spatial vector v[0..2], in the order gamma_calc() and
+// Utoprim_new_body() sum it
+template <class GP, class T>
+HD T spatial_sq(const T* v, GP g) {
+  constexpr int K = geom_kind<GP>::value;
+  if constexpr (K == GK_FLAT) {
+    return v[0]*v[0] + v[1]*v[1] + v[2]*v[2];
+  } else if constexpr (K == GK_KS) {
+    return g->gcov[1][1]*v[0]*v[0] + g->gcov[2][2]*v[1]*v[1] + g->gcov[3][3]*v[2]*v[2]
+         + 2*(g->gcov[1][3]*v[0]*v[2]);
+  } else if constexpr (K == GK_DIAG) {
+    return g->gcov[1][1]*v[0]*v[0] + g->gcov[2][2]*v[1]*v[1] + g->gcov[3][3]*v[2]*v[2];
+  } else {
+    return g->gcov[1][1]*v[0]*v[0] + g->gcov[2][2]*v[1]*v[1] + g->gcov[3][3]*v[2]*v[2]
+         + 2*(g->gcov[1][2]*v[0]*v[1] + g->gcov[1][3]*v[0]*v[2] + g->gcov[2][3]*v[1]*v[2]);
+  }
+}
+// sqrt(-g), its inverse, lapse, n^t; v^i - u^t beta^i
+template <class GP> HD auto g_det(GP g) { if constexpr (geom_kind<GP>::value == GK_FLAT) return 1.; else return g->g; }
+template <class GP> HD auto g_detinv(GP g) { if constexpr (geom_kind<GP>::value == GK_FLAT) return 1.; else return g->g_inv; }
+template <class GP> HD auto g_alpha(GP g) { if constexpr (geom_kind<GP>::value == GK_FLAT) return 1.; else return g->alpha; }
+template <class GP> HD auto g_ncon0(GP g) { if constexpr (geom_kind<GP>::value == GK_FLAT) return 1.; else return g->ncon[0]; }
+template <class GP, class T>
+HD void shift_ucon(const T* v, GP g, T* ucon) {
+  constexpr int K = geom_kind<GP>::value;
+  if constexpr (K == GK_FLAT) ucon[1] = v[0];
+  else ucon[1] = v[0] - ucon[0]*g->beta[0];
+  if constexpr (K == GK_FLAT || K == GK_KS) {
+    ucon[2] = v[1];
+    ucon[3] = v[2];
+  } else {
+    ucon[2] = v[1] - ucon[0]*g->beta[1];
+    ucon[3] = v[2] - ucon[0]*g->beta[2];
+  }
+}
+// g^tt + x, g^{tj} + x and g^{jj} + x (the characteristic quadratic's coefficients)
+template <class GP, class T>
+HD T gtt_plus(GP g, T x) { if constexpr (geom_kind<GP>::value == GK_FLAT) return -1. + x; else return g->gcon[0][0] + x; }
+template <int js, class GP, class T>
+HD T gtj_plus(GP g, T x) {
+  constexpr int K = geom_kind<GP>::value;
+  if constexpr (K == GK_FLAT || (K == GK_KS && js != 1)) return x;
+  else return g->gcon[0][js] + x;
+}
+template <int js, class GP, class T>
+HD T gjj_plus(GP g, T x) { if constexpr (geom_kind<GP>::value == GK_FLAT) return 1. + x; else return g->gcon[js][js] + x; }
 HD double dot4(const double* a, const double* b) {
   return a[0]*b[0] + a[1]*b[1] + a[2]*b[2] + a[3]*b[3];
 }
@@ -87,12 +161,7 @@ HD double dot4(const double* a, const double* b) {
 // gamma_calc(), src/phys.c:244-268.  Returns 1 on failure (gamma = 1).
 template <class GP>
 HD int gamma_calc(const double* pr, GP g, double* gamma) {
-  double qsq = g->gcov[1][1]*pr[U1]*pr[U1]
-             + g->gcov[2][2]*pr[U2]*pr[U2]
-             + g->gcov[3][3]*pr[U3]*pr[U3]
-             + 2*(g->gcov[1][2]*pr[U1]*pr[U2]
-                + g->gcov[1][3]*pr[U1]*pr[U3]
-                + g->gcov[2][3]*pr[U2]*pr[U3]);
+  double qsq = spatial_sq(pr + U1, g);
   if (qsq < 0.) {
     if (fabs(qsq) > 1.E-10) { *gamma = 1.; return 1; }
     else qsq = 1.E-10;
@@ -107,10 +176,8 @@ template <class GP>
 HD int get_state(const double* pr, GP g, double gam, State* q) {
   double gamma;
   int fl = gamma_calc(pr, g, &gamma);
-  q->ucon[0] = gamma*g->ncon[0];
-  q->ucon[1] = pr[U1] - q->ucon[0]*g->beta[0];
-  q->ucon[2] = pr[U2] - q->ucon[0]*g->beta[1];
-  q->ucon[3] = pr[U3] - q->ucon[0]*g->beta[2];
+  q->ucon[0] = gamma*g_ncon0(g);
+  shift_ucon(pr + U1, g, q->ucon);
   lower(q->ucon, g, q->ucov);
   double inv_ut = 1./q->ucon[0];
   q->bcon[0] = pr[B1]*q->ucov[1] + pr[B2]*q->ucov[2] + pr[B3]*q->ucov[3];
@@ -149,20 +216,21 @@ HD void primtoflux(const double* pr, const State* q, int dir, GP g, double* flux
   flux[B1] = q->bcon[1]*q->ucon[dir] - q->bcon[dir]*q->ucon[1];
   flux[B2] = q->bcon[2]*q->ucon[dir] - q->bcon[dir]*q->ucon[2];
   flux[B3] = q->bcon[3]*q->ucon[dir] - q->bcon[dir]*q->ucon[3];
-  for (int l = 0; l < NP; l++) flux[l] *= g->g;
+  for (int l = 0; l < NP; l++) flux[l] *= g_det(g);
 }
 
 // vchar_fast(), src/phys.c:432-501
-HD void vchar_fast(const State* q, const Geom* g, int js, double gam, double* vmax, double* vmin) {
+template <int js, class GP>
+HD void vchar_fast(const State* q, GP g, double gam, double* vmax, double* vmin) {
   double cms2 = (gam * q->p + q->bsq) / q->eta;
   if (cms2 < 0.) cms2 = SMALL;
   else if (cms2 > 1.) cms2 = 1.;
   double Au2 = q->ucon[js]*q->ucon[js];
   double Bu2 = q->ucon[0]*q->ucon[0];
   double AuBu = q->ucon[js]*q->ucon[0];
-  double A = Bu2 - (g->gcon[0][0] + Bu2)*cms2;
-  double B = AuBu - (g->gcon[0][js] + AuBu)*cms2;
-  double C = Au2 - (g->gcon[js][js] + Au2)*cms2;
+  double A = Bu2 - gtt_plus(g, Bu2)*cms2;
+  double B = AuBu - gtj_plus<js>(g, AuBu)*cms2;
+  double C = Au2 - gjj_plus<js>(g, Au2)*cms2;
   double discr = B*B - A*C;
   if (discr < 0.) discr = 0.;   // both branches of src/phys.c:473-484 set 0
   discr = sqrt(discr);
@@ -346,8 +414,8 @@ struct U2dAux {
 template <class GP>
 HD int u2d_prepare(const double* U, GP geom, double gmog, double* prim, U2d& s, U2dAux& aux) {
   if (U[0] <= 0.) return -100;
-  double inv_gdet = geom->g_inv;
-  double alpha = geom->alpha;
+  double inv_gdet = g_detinv(geom);
+  double alpha = g_alpha(geom);
   double geomfactor = alpha * inv_gdet;
   prim[B1] = U[B1] * inv_gdet;
   prim[B2] = U[B2] * inv_gdet;
@@ -365,12 +433,7 @@ HD int u2d_prepare(const double* U, GP geom, double gmog, double* prim, U2d& s, 
   s.gmog = gmog;
   double* Bcon = aux.Bcon;
   Bcon[0] = 0.; Bcon[1] = Ut[B1]; Bcon[2] = Ut[B2]; Bcon[3] = Ut[B3];
-  s.Bsq = geom->gcov[1][1]*Bcon[1]*Bcon[1]
-        + geom->gcov[2][2]*Bcon[2]*Bcon[2]
-        + geom->gcov[3][3]*Bcon[3]*Bcon[3]
-        + 2*(geom->gcov[1][2]*Bcon[1]*Bcon[2]
-           + geom->gcov[1][3]*Bcon[1]*Bcon[3]
-           + geom->gcov[2][3]*Bcon[2]*Bcon[3]);
+  s.Bsq = spatial_sq(Bcon + 1, geom);
   double Qcov[4] = {Ut[UU], Ut[U1], Ut[U2], Ut[U3]};
   raise_v(Qcov, geom, aux.Qcon);
   aux.QdotB = Qcov[1]*Bcon[1] + Qcov[2]*Bcon[2] + Qcov[3]*Bcon[3];
@@ -380,7 +443,16 @@ HD int u2d_prepare(const double* U, GP geom, double gmog, double* prim, U2d& s, 
   s.Qtsq = Qsq + s.Qdotn*s.Qdotn;
   s.D = Ut[RHO];
   s.half_Bsq = 0.5*s.Bsq;
-  for (int l = 0; l < 4; l++) aux.ncon[l] = geom->ncon[l];
+  if constexpr (geom_kind<GP>::value == GK_FLAT) {
+    aux.ncon[0] = 1.;
+    aux.ncon[1] = aux.ncon[2] = aux.ncon[3] = 0.;
+  } else if constexpr (geom_kind<GP>::value == GK_KS) {
+    aux.ncon[0] = geom->ncon[0];
+    aux.ncon[1] = geom->ncon[1];
+    aux.ncon[2] = aux.ncon[3] = 0.;
+  } else {
+    for (int l = 0; l < 4; l++) aux.ncon[l] = geom->ncon[l];
+  }
   return 0;
 }
 
@@ -405,12 +477,7 @@ HD void u2d_guess_w(const U2d& s, double W_last, double* x2d, double vsq_guess =
 // (src/utoprim_2d_fast.c:302-330).  Returns 2 when their u~^2 is unusable.
 template <class GP>
 HD int u2d_guess(const U2d& s, GP geom, double gam, const double* prim, double* x2d) {
-  double utsq = geom->gcov[1][1]*prim[U1]*prim[U1]
-              + geom->gcov[2][2]*prim[U2]*prim[U2]
-              + geom->gcov[3][3]*prim[U3]*prim[U3]
-              + 2*(geom->gcov[1][2]*prim[U1]*prim[U2]
-                 + geom->gcov[1][3]*prim[U1]*prim[U3]
-                 + geom->gcov[2][3]*prim[U2]*prim[U3]);
+  double utsq = spatial_sq(prim + U1, geom);
   if ((utsq < 0.) && (fabs(utsq) < 1.0e-13)) utsq = fabs(utsq);
   if (utsq < 0. || utsq > UTSQ_TOO_BIG) return 2;
   double gammasq = 1. + utsq;
@@ -432,6 +499,8 @@ HD int u2d_setup(const double* U, GP geom, double gam, double gmog, double* prim
 }
 
 // Utoprim_new_body() after the Newton solve (src/utoprim_2d_fast.c:345-408).
+// K: the geometry's structure (which components of n^i are zero).
+template <int K = GK_GEN>
 HD int u2d_finish(const U2d& s, const U2dAux& aux, double gam, const double* x2d, int retval, double* prim,
                   double* gamma_out, double* bsq_out) {
   double W = x2d[0];
@@ -451,9 +520,15 @@ HD int u2d_finish(const U2d& s, const U2dAux& aux, double gam, const double* x2d
   double g_o_WBsq = gamma/(W + s.Bsq);
   double QdB_o_W = aux.QdotB / W;
   *bsq_out = s.Bsq * (1. - vsq) + QdB_o_W*QdB_o_W;
-  prim[U1] = g_o_WBsq * (aux.Qcon[1] + aux.ncon[1] * s.Qdotn + QdB_o_W*aux.Bcon[1]);
-  prim[U2] = g_o_WBsq * (aux.Qcon[2] + aux.ncon[2] * s.Qdotn + QdB_o_W*aux.Bcon[2]);
-  prim[U3] = g_o_WBsq * (aux.Qcon[3] + aux.ncon[3] * s.Qdotn + QdB_o_W*aux.Bcon[3]);
+  if constexpr (K == GK_FLAT) prim[U1] = g_o_WBsq * (aux.Qcon[1] + QdB_o_W*aux.Bcon[1]);
+  else prim[U1] = g_o_WBsq * (aux.Qcon[1] + aux.ncon[1] * s.Qdotn + QdB_o_W*aux.Bcon[1]);
+  if constexpr (K == GK_FLAT || K == GK_KS) {
+    prim[U2] = g_o_WBsq * (aux.Qcon[2] + QdB_o_W*aux.Bcon[2]);
+    prim[U3] = g_o_WBsq * (aux.Qcon[3] + QdB_o_W*aux.Bcon[3]);
+  } else {
+    prim[U2] = g_o_WBsq * (aux.Qcon[2] + aux.ncon[2] * s.Qdotn + QdB_o_W*aux.Bcon[2]);
+    prim[U3] = g_o_WBsq * (aux.Qcon[3] + aux.ncon[3] * s.Qdotn + QdB_o_W*aux.Bcon[3]);
+  }
   return 0;
 }
 
@@ -473,7 +548,7 @@ HD int utoprim_2d_fast(const double* U, GP geom, double gam, double gmog, double
   int rc = u2d_setup(U, geom, gam, gmog, prim, s, aux, x2d);
   if (rc) return rc;
   int retval = u2d_newton(s, x2d, iters, n_extra);
-  return u2d_finish(s, aux, gam, x2d, retval, prim, gamma_out, bsq_out);
+  return u2d_finish<geom_kind<GP>::value>(s, aux, gam, x2d, retval, prim, gamma_out, bsq_out);
 }
 
 // ---------------------------------------------------------------------------
