@@ -51,7 +51,6 @@ struct hgpu_ctx {
   int otf_stage = 0;               // level of the running stage (binary metric evaluated in kernels)
   long long n_geom = 0, n_conn = 0;
   int n1_conn = 0;
-  std::vector<double> stage;       // host staging buffer
   void* be = nullptr;              // backend-private data
   unsigned long long host_status[hgpu::ST_WORDS];
   double host_scal[hgpu::SC_WORDS];
@@ -403,23 +402,12 @@ struct Api {
 
   static int upload_prims(hgpu_ctx* c, int which, const double* host) {
     if (!c || !host) return set_error(-1, "null argument");
-    const long long NT = c->P.nt;
-    c->stage.resize(NP * NT);
-    aos_to_soa(host, c->stage.data(), NT, NP);
-    double* dst = which ? c->X.ph : c->X.p;
-    int rc = BE::h2d(c, dst, c->stage.data(), sizeof(double) * NP * NT);
-    return rc ? rc : BE::sync(c);
+    return BE::upload_state(c, which ? c->X.ph : c->X.p, host, c->P.nt);
   }
 
   static int download_prims(hgpu_ctx* c, int which, double* host) {
     if (!c || !host) return set_error(-1, "null argument");
-    const long long NT = c->P.nt;
-    c->stage.resize(NP * NT);
-    const double* src = which ? c->X.ph : c->X.p;
-    int rc = BE::d2h(c, c->stage.data(), src, sizeof(double) * NP * NT);
-    if (rc) return rc;
-    soa_to_aos(c->stage.data(), host, NT, NP);
-    return 0;
+    return BE::download_state(c, host, which ? c->X.ph : c->X.p, c->P.nt);
   }
 
   static int set_time(hgpu_ctx* c, double t, double dt) {

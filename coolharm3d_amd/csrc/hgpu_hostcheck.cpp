@@ -43,6 +43,8 @@ struct HostBE {
   static void release(hgpu_ctx*, void* p) { free(p); }
   static int h2d(hgpu_ctx*, void* d, const void* h, size_t bytes) { memcpy(d, h, bytes); return 0; }
   static int d2h(hgpu_ctx*, void* h, const void* d, size_t bytes) { memcpy(h, d, bytes); return 0; }
+  static int download_state(hgpu_ctx*, double* h, const double* S, long long nt) { soa_to_aos(S, h, nt, NP); return 0; }
+  static int upload_state(hgpu_ctx*, double* S, const double* h, long long nt) { aos_to_soa(h, S, nt, NP); return 0; }
   static int zero(hgpu_ctx*, void* p, size_t bytes) { memset(p, 0, bytes); return 0; }
   static int sync(hgpu_ctx*) { return 0; }
   static int mark(hgpu_ctx*, const char*, int) { return 0; }

@@ -6,6 +6,7 @@
 // the stencil kernels map workgroups to tiles XCD by XCD (Tiling below).
 // Failure counters are summed across the wavefront before one atomic per wave.
 #include "hgpu_launch.h"
+#include "hgpu_xfer.h"
 
 namespace hgpu {
 
@@ -24,6 +25,7 @@ struct GpuPriv {
   std::map<std::string, hipEvent_t> open;   // mark() begin events
   void* box_stage = nullptr;           // staging of hgpu_download_box / hgpu_upload_box
   size_t box_bytes = 0;
+  XferRing ring;                       // pinned chunks of the copies to and from the host
 };
 
 static inline GpuPriv* priv(hgpu_ctx* c) { return static_cast<GpuPriv*>(c->be); }
@@ -596,6 +598,7 @@ struct GpuBE {
     if (!g) return;
     if (g->stream) (void)hipStreamSynchronize(g->stream);
     if (g->step_exec) (void)hipGraphExecDestroy(g->step_exec);
+    g->ring.release();
     if (g->box_stage) (void)hipFree(g->box_stage);
     if (g->stream) (void)hipStreamDestroy(g->stream);
     for (auto& pe : g->pending) { (void)hipEventDestroy(pe.a); (void)hipEventDestroy(pe.b); }
@@ -615,8 +618,35 @@ struct GpuBE {
            hip_check(hipStreamSynchronize(priv(c)->stream), "hipStreamSynchronize");
   }
   static int d2h(hgpu_ctx* c, void* h, const void* d, size_t bytes) {
-    return hip_check(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, priv(c)->stream), "hipMemcpy D2H") |
-           hip_check(hipStreamSynchronize(priv(c)->stream), "hipStreamSynchronize");
+    GpuPriv* g = priv(c);
+    if (bytes >= 4 && bytes % 4 == 0 && reinterpret_cast<uintptr_t>(d) % 16 == 0) {
+      const char* src = static_cast<const char*>(d);
+      return hip_check(xfer_to_host(g->ring, g->stream, h, bytes, [&](size_t off, size_t len, char* chunk) {
+        const long long n32 = (long long)(len / 4);
+        const unsigned nb = (unsigned)std::min<long long>((n32 / 4 + XFER_B - 1) / XFER_B + 1, 512);
+        hipLaunchKernelGGL(k_copy_words, dim3(nb), dim3(XFER_B), 0, g->stream,
+                           reinterpret_cast<const unsigned*>(src + off), n32, reinterpret_cast<unsigned*>(chunk));
+      }), "copy to host");
+    }
+    return hip_check(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, g->stream), "hipMemcpy D2H") |
+           hip_check(hipStreamSynchronize(g->stream), "hipStreamSynchronize");
+  }
+  // a state array S ([8][nt]) to or from the host's [nt][8]
+  static int download_state(hgpu_ctx* c, double* h, const double* S, long long nt) {
+    GpuPriv* g = priv(c);
+    return hip_check(xfer_to_host(g->ring, g->stream, h, sizeof(double) * NP * nt, [&](size_t off, size_t len, char* chunk) {
+      const long long z0 = (long long)(off / (sizeof(double) * NP)), nz = (long long)(len / (sizeof(double) * NP));
+      hipLaunchKernelGGL(k_soa_to_aos, dim3((unsigned)((nz + XFER_B - 1) / XFER_B)), dim3(XFER_B), 0, g->stream, S, nt,
+                         z0, nz, reinterpret_cast<double*>(chunk));
+    }), "state to host");
+  }
+  static int upload_state(hgpu_ctx* c, double* S, const double* h, long long nt) {
+    GpuPriv* g = priv(c);
+    return hip_check(xfer_to_device(g->ring, g->stream, h, sizeof(double) * NP * nt, [&](size_t off, size_t len, const char* chunk) {
+      const long long z0 = (long long)(off / (sizeof(double) * NP)), nz = (long long)(len / (sizeof(double) * NP));
+      hipLaunchKernelGGL(k_aos_to_soa, dim3((unsigned)((nz + XFER_B - 1) / XFER_B)), dim3(XFER_B), 0, g->stream,
+                         reinterpret_cast<const double*>(chunk), nt, z0, nz, S);
+    }), "state to device");
   }
   // zero fill with a kernel (no memset nodes on the stream)
   static int zero(hgpu_ctx* c, void* p, size_t bytes) {
