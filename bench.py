@@ -497,6 +497,9 @@ def main():
 
     tag = "fp64" if args.precision == "fp64" else "mixed"
     units = units_per_launch(n1, n2, n3)
+    # faces of a step's two stages and three directions over its flux launches (one a stage, or
+    # one per direction)
+    units["flux"] *= 6.0 * args.prof_steps / max(kern["flux"][1], 1)
     model = ALGO_BYTES if tag == "fp64" else ALGO_BYTES_MIXED
     per_launch_s = {k: kern[k][0] / max(kern[k][1], 1) / 1e3 for k in ("flux", "emf", "update")}
     workload = f"torus{n1}x{n2}x{n3}_{tag}"

@@ -477,7 +477,7 @@ struct Api {
       X.cent_lvl = stage;
       c->otf_stage = stage;
     }
-    for (int d = 0; d < 3; d++) rc |= BE::flux(c, src, d);
+    rc |= BE::flux_stage(c, src);
     rc |= BE::emf(c);
     rc |= BE::update(c, stage, false);   // begin_stage() emptied the slow-zone queue
     if (c->P.dyn) { X.geom = X.geom_new; X.cent_lvl = stage + 1; }

@@ -78,6 +78,11 @@ struct HostBE {
     for (int l = 0; l < N_NFAIL; l++) c->X.status[ST_NFAILTOT + l] = 0;
     return 0;
   }
+  static int flux_stage(hgpu_ctx* c, const double* src) {
+    int rc = 0;
+    for (int d = 0; d < 3; d++) rc |= flux(c, src, d);
+    return rc;
+  }
   static int flux(hgpu_ctx* c, const double* src, int d) {
     Box b = flux_box(c->P, d);
     for (long long t = 0; t < b.count(); t++) {

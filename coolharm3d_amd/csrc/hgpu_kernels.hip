@@ -19,6 +19,7 @@ struct GpuPriv {
   bool graph = false;                  // replay captured steps
   hipGraphExec_t step_exec = nullptr;  // one step_ch(), captured on first use
   LaunchShape shape[N_FAM];            // per kernel family
+  bool flux_all = true;                // the three face-flux directions in one launch
   std::vector<ProfEvent> pending;
   std::vector<hipEvent_t> pool;
   std::map<std::string, std::pair<double, long long>> acc;
@@ -798,6 +799,7 @@ struct GpuBE {
     if (int rc = check_shape(L)) return rc;
     int rc = invalidate_graph(c);
     priv(c)->shape[fam] = L;
+    if (fam <= FAM_FLUX3) priv(c)->flux_all = false;
     return rc;
   }
   static int get_shape(hgpu_ctx* c, int fam, int* bs, int* kc, int* remap) {
@@ -988,6 +990,23 @@ struct GpuBE {
         report[fam*4 + 3] = best_ms;
       }
     }
+    // the face fluxes in one launch, or the tuned launch per direction
+    if (!rc && flux_all_possible(c->P)) {
+      float ms[2] = {1e30f, 1e30f};
+      for (int round = 0; round < 2 && !rc; round++)
+        for (int all = 0; all < 2; all++) {
+          g->flux_all = all != 0;
+          rc |= flux_stage(c, c->X.p);
+          rc |= hip_check(hipEventRecord(e0, st), "hipEventRecord");
+          for (int r = 0; r < 3 * reps; r++) rc |= flux_stage(c, c->X.p);
+          rc |= hip_check(hipEventRecord(e1, st), "hipEventRecord");
+          rc |= hip_check(hipEventSynchronize(e1), "hipEventSynchronize");
+          float t = 0.f;
+          rc |= hip_check(hipEventElapsedTime(&t, e0, e1), "hipEventElapsedTime");
+          ms[all] = std::min(ms[all], t);
+        }
+      g->flux_all = ms[1] < ms[0];
+    }
     g->pool.push_back(e0);
     g->pool.push_back(e1);
     g->prof = prof;
@@ -1017,6 +1036,19 @@ struct GpuBE {
   static int reset_nfailtot(hgpu_ctx* c) {
     hipLaunchKernelGGL(k_reset_words, dim3(1), dim3(64), 0, priv(c)->stream, c->X, (int)ST_NFAILTOT, N_NFAIL);
     return hip_check(hipGetLastError(), "k_reset_words");
+  }
+  // every direction of a stage: one launch unless the caller or the autotuner
+  // chose shapes per direction
+  static int flux_stage(hgpu_ctx* c, const double* src) {
+    GpuPriv* g = priv(c);
+    if (g->flux_all && flux_all_possible(c->P)) {
+      Scope s(c, "flux");
+      launch_flux_all(c->P, c->X, src, g->stream, c->pn, c->otf_stage);
+      return hip_check(hipGetLastError(), "k_flux_all");
+    }
+    int rc = 0;
+    for (int d = 0; d < 3; d++) rc |= flux(c, src, d);
+    return rc;
   }
   static int flux(hgpu_ctx* c, const double* src, int d) {
     Scope s(c, "flux");

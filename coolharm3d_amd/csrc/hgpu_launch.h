@@ -100,9 +100,10 @@ __device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, cons
 // workgroup in L2.  The shape of each kernel family is picked by the autotuner
 // (or set by the caller).
 struct Tiling {
-  unsigned ni, nj, nk;  // box extents
+  unsigned ni, nj, nk;  // box extents (ni: rows of tiles, i.e. x1-planes, or groups of pp of them)
   unsigned bs, kc, jr;  // tile: kc x jr (kc > 0) or bs consecutive points (kc = 0)
   unsigned nkt;         // tiles along k (2D tiles)
+  unsigned pp, np;      // x1-planes per flat tile (small planes), x1-planes in all
   unsigned X;           // tiles per plane
   unsigned nblocks;     // X * ni, rounded up to a multiple of 8 when remapped
   unsigned remap;
@@ -113,7 +114,8 @@ static inline Tiling make_tiling(const Box& b, const LaunchShape& L = LaunchShap
   Tiling T;
   T.nk = (unsigned)(b.hi[2] - b.lo[2] + 1);
   T.nj = (unsigned)(b.hi[1] - b.lo[1] + 1);
-  T.ni = (unsigned)(b.hi[0] - b.lo[0] + 1);
+  T.ni = T.np = (unsigned)(b.hi[0] - b.lo[0] + 1);
+  T.pp = 1;
   T.bs = L.bs;
   T.remap = L.remap;
   T.order = L.order;
@@ -127,27 +129,27 @@ static inline Tiling make_tiling(const Box& b, const LaunchShape& L = LaunchShap
     T.jr = 0;
     T.nkt = 0;
     T.X = (T.nj * T.nk + T.bs - 1) / T.bs;
+    // planes smaller than a tile: several to a tile (a 1D grid's planes hold a
+    // handful of points, and a workgroup per plane left 250 of 256 threads idle)
+    T.pp = std::max(1u, T.bs / (T.nj * T.nk));
+    T.ni = (T.np + T.pp - 1) / T.pp;
   }
   T.nblocks = T.X * T.ni;
   if (T.remap) T.nblocks = ((T.nblocks + 7u) / 8u) * 8u;
   return T;
 }
 
-__device__ __forceinline__ bool tile_index(const Box& b, const Tiling& T, int& i, int& j, int& k) {
-  const unsigned p = blockIdx.x;
-  const unsigned L = T.remap ? (p & 7u) * (T.nblocks >> 3) + (p >> 3) : p;
-  unsigned ii, t;
-  if (T.order == 0) {
-    ii = L / T.X;
-    t = L - ii * T.X;
-  } else {
-    t = L / T.ni;
-    ii = L - t * T.ni;
-    if (t >= T.X) return false;
-  }
-  if (ii >= T.ni) return false;
+// point (i, j, k) of this thread in tile t of tile row ii
+__device__ __forceinline__ bool tile_point(const Box& b, const Tiling& T, unsigned ii, unsigned t, int& i, int& j,
+                                           int& k) {
   unsigned jj, kk;
-  if (T.kc == 0) {
+  if (T.pp > 1) {        // X = 1
+    const unsigned np = T.nj * T.nk, di = threadIdx.x / np, q = threadIdx.x - di * np;
+    ii = ii * T.pp + di;
+    if (di >= T.pp || ii >= T.np) return false;
+    jj = q / T.nk;
+    kk = q - jj * T.nk;
+  } else if (T.kc == 0) {
     const unsigned q = t * T.bs + threadIdx.x;
     jj = q / T.nk;
     kk = q - jj * T.nk;
@@ -164,6 +166,22 @@ __device__ __forceinline__ bool tile_index(const Box& b, const Tiling& T, int& i
   j = b.lo[1] + (int)jj;
   k = b.lo[2] + (int)kk;
   return true;
+}
+
+__device__ __forceinline__ bool tile_index(const Box& b, const Tiling& T, int& i, int& j, int& k) {
+  const unsigned p = blockIdx.x;
+  const unsigned L = T.remap ? (p & 7u) * (T.nblocks >> 3) + (p >> 3) : p;
+  unsigned ii, t;
+  if (T.order == 0) {
+    ii = L / T.X;
+    t = L - ii * T.X;
+  } else {
+    t = L / T.ni;
+    ii = L - t * T.ni;
+    if (t >= T.X) return false;
+  }
+  if (ii >= T.ni) return false;
+  return tile_point(b, T, ii, t, i, j, k);
 }
 
 constexpr unsigned MASK_GAMMA = 1u << NFAIL_GAMMA_CALC;
@@ -186,5 +204,9 @@ __device__ __forceinline__ PnOrbit orbit_load(const PnOrbit* p) {
 // hgpu_flux.hip: face fluxes of direction d with launch shape L
 void launch_flux_dir(int d, const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, hipStream_t st,
                      const PnGrid& G, int lvl);
+// The three directions in one launch (flux_all_possible(); 2 faces per thread,
+// or one where flux_all_multi() says no)
+bool flux_all_possible(const Params& P);
+void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStream_t st, const PnGrid& G, int lvl);
 
 }  // namespace hgpu

@@ -141,6 +141,8 @@ int hgpu_set_graph(hgpu_ctx *ctx, int on);
  * sharing each zone's parabola, bit 6 (family 2, FP64, 2 or 4 faces per
  * thread): the reconstruction reads LDS-staged x3 pencils (each wavefront's
  * zones loaded once, coalesced, into LDS) instead of per-lane stencil loads.
+ * The three face-flux directions run in one launch until a shape of families
+ * 0-2 is set by hand or hgpu_autotune() finds a launch per direction faster.
  * hgpu_autotune() times every candidate of families 0-4 on the current state
  * (reps launches each; family 4 as the whole predictor update, split or fused)
  * and keeps the fastest; report (NULL or [5][4]) gets
