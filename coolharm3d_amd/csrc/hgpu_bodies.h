@@ -20,8 +20,11 @@ struct FaceOtf {
 // Zone-centre record at the level X.geom describes: read, or (binary metric
 // evaluated in the kernels, P.otf) evaluated into buf from the orbit of level
 // X.cent_lvl.
+// OTF: 0 or 1 fixes the choice when a kernel is compiled (a pointer that may be
+// either keeps the record in scratch memory), -1 takes it from P.
+template <int OTF = -1>
 HD const Geom* cent_rec(const Params& P, const Ptrs& X, int i, int j, int k, Geom& buf) {
-  if (P.otf) {
+  if (OTF < 0 ? P.otf != 0 : OTF != 0) {
     pn_zone_geom(P, X.pn, X.orbit[X.cent_lvl], i, j, k, CENT, &buf);
     return &buf;
   }
@@ -55,21 +58,25 @@ HD void flux_recon(const Params& P, const Ptrs& X, const double* __restrict__ sr
     if (P.degen[0]) ii = NG;
     if (P.degen[1]) jj = NG;
     if (P.degen[2]) kk = NG;
+    // every primitive's stencil is loaded before any limiter runs, so their
+    // loads are in flight together (their branches keep the compiler from
+    // moving loads across them)
     if (P.recon == RECON_PPM_MC) {
-      long long c0 = cidx(P, ii - 3*di, jj - 3*dj, kk - 3*dk);
-      long long st = cidx(P, di, dj, dk) - cidx(P, 0, 0, 0);
+      const long long c0 = cidx(P, ii - 3*di, jj - 3*dj, kk - 3*dk);
+      const long long st = cidx(P, di, dj, dk) - cidx(P, 0, 0, 0);
+      double y[NP][6];
+#pragma unroll
+      for (int v = 0; v < NP; v++)
+#pragma unroll
+        for (int m = 0; m < 6; m++) y[v][m] = src[v*NT + c0 + m*st];
+#pragma unroll
       for (int v = 0; v < NP; v++) {
-        double y[6];
+#pragma unroll
         for (int m = 0; m < 6; m++) {
-          double x = src[v*NT + c0 + m*st];
-          if (d == 0) {
-            x *= X.rscale[rs_slot(v)*P.n1t + (ii - 3 + m)];
-          } else {
-            x = rt_val(P, X, v, ii, x);
-          }
-          y[m] = x;
+          if (d == 0) y[v][m] *= X.rscale[rs_slot(v)*P.n1t + (ii - 3 + m)];
+          else y[v][m] = rt_val(P, X, v, ii, y[v][m]);
         }
-        ppm_interface(y, &pl[v], &pr[v]);
+        ppm_interface(y[v], &pl[v], &pr[v]);
         if (d == 0) {
           double f = X.irscale[(3 + rs_slot(v))*P.n1t + i];
           pl[v] *= f;
@@ -78,23 +85,24 @@ HD void flux_recon(const Params& P, const Ptrs& X, const double* __restrict__ sr
       }
     } else {
       // MC slopes, src/recon.c:960-986
-      long long c0 = cidx(P, ii - 2*di, jj - 2*dj, kk - 2*dk);
-      long long st = cidx(P, di, dj, dk) - cidx(P, 0, 0, 0);
+      const long long c0 = cidx(P, ii - 2*di, jj - 2*dj, kk - 2*dk);
+      const long long st = cidx(P, di, dj, dk) - cidx(P, 0, 0, 0);
+      double y[NP][4];
+#pragma unroll
+      for (int v = 0; v < NP; v++)
+#pragma unroll
+        for (int m = 0; m < 4; m++) y[v][m] = src[v*NT + c0 + m*st];
+#pragma unroll
       for (int v = 0; v < NP; v++) {
-        double y[4];
+#pragma unroll
         for (int m = 0; m < 4; m++) {
-          double x = src[v*NT + c0 + m*st];
-          if (d == 0) {
-            x *= X.rscale[rs_slot(v)*P.n1t + (ii - 2 + m)];
-          } else {
-            x = rt_val(P, X, v, ii, x);
-          }
-          y[m] = x;
+          if (d == 0) y[v][m] *= X.rscale[rs_slot(v)*P.n1t + (ii - 2 + m)];
+          else y[v][m] = rt_val(P, X, v, ii, y[v][m]);
         }
-        double dql = 0.5*mc_slope(y[0], y[1], y[2]);
-        double dqr = 0.5*mc_slope(y[1], y[2], y[3]);
-        pl[v] = y[1] + dql;
-        pr[v] = y[2] - dqr;
+        double dql = 0.5*mc_slope(y[v][0], y[v][1], y[v][2]);
+        double dqr = 0.5*mc_slope(y[v][1], y[v][2], y[v][3]);
+        pl[v] = y[v][1] + dql;
+        pr[v] = y[v][2] - dqr;
         if (d == 0) {
           double f = X.irscale[(3 + rs_slot(v))*P.n1t + i];
           pl[v] *= f;
@@ -542,23 +550,33 @@ HD double entropy_flux(const Params& P, const Ptrs& X, const double* src, int d,
   }
 }
 
+// Entropy flux of face f of zone (i,j,k): f = 2 d lower, 2 d + 1 upper face along d
+template <bool MIXED>
+HD double entropy_face(const Params& P, const Ptrs& X, const double* src, int f, int i, int j, int k,
+                       const FaceOtf* fo) {
+  return entropy_flux<MIXED>(P, X, src, f >> 1, i + (f == 1), j + (f == 3), k + (f == 5), fo);
+}
+
 // fixup_entropy_eq(), src/fixup.c:335-454
 template <bool MIXED>
 HD int fixup_entropy_eq(const Params& P, const Ptrs& X, int i, int j, int k, double Dt,
                         const double* prim_old, double* prim, const Geom* g, const double* U,
-                        double* gamma_out, const double* src, const FaceOtf* fo, FailRec& fr) {
+                        double* gamma_out, const double* src, const FaceOtf* fo, FailRec& fr,
+                        const double* Fs = nullptr, int fs_stride = 0) {
   double prim_backup[NP];
   for (int l = 0; l < NP; l++) prim_backup[l] = prim[l];
   double gamma;
   gamma_calc(prim_old, g, &gamma);
   double S_old = g->g * (P.gam - 1.)*prim_old[UU]*gamma / (g->alpha * pow(prim_old[RHO], (P.gam - 1.)));
-  const double Fm0 = entropy_flux<MIXED>(P, X, src, 0, i, j, k, fo), Fp0 = entropy_flux<MIXED>(P, X, src, 0, i + 1, j, k, fo);
-  const double Fm1 = entropy_flux<MIXED>(P, X, src, 1, i, j, k, fo), Fp1 = entropy_flux<MIXED>(P, X, src, 1, i, j + 1, k, fo);
-  const double Fm2 = entropy_flux<MIXED>(P, X, src, 2, i, j, k, fo), Fp2 = entropy_flux<MIXED>(P, X, src, 2, i, j, k + 1, fo);
+  // the six entropy face fluxes: the caller's (face f of the zone, entropy_face(),
+  // at Fs[f*fs_stride]), or evaluated here
+  double Ff[6];
+#pragma unroll
+  for (int f = 0; f < 6; f++) Ff[f] = Fs ? Fs[f*fs_stride] : entropy_face<MIXED>(P, X, src, f, i, j, k, fo);
   double S = S_old + Dt*(
-      - (Fp0 - Fm0) * P.invdx[1]
-      - (Fp1 - Fm1) * P.invdx[2]
-      - (Fp2 - Fm2) * P.invdx[3]);
+      - (Ff[1] - Ff[0]) * P.invdx[1]
+      - (Ff[3] - Ff[2]) * P.invdx[2]
+      - (Ff[5] - Ff[4]) * P.invdx[3]);
   int ret = utoprim_1d_ee(U, S, g, P.gam, prim, &gamma);
   if ((!ret) && (check_gamma(gamma) == 2)) {
     for (int l = 0; l < NP; l++) prim[l] = prim_backup[l];
@@ -579,34 +597,76 @@ HD int fixup_entropy_eq(const Params& P, const Ptrs& X, int i, int j, int k, dou
 }
 
 // --------------------------------------------------------------------------
-// recover_primitives(), src/step_ch.c:801-1024 (FIXUP_TREE 3, entropy fix on)
-// src: the stage's reconstruction source, for the entropy face fluxes.
-template <bool MIXED>
-HD void recover_primitives(const Params& P, const Ptrs& X, int i, int j, int k, double Dt,
-                           double* pf, const double* U, const double* p_old, const Geom* g,
-                           double rhoflr, double uuflr, double* p_gamma, const double* src, const FaceOtf* fo,
-                           FailRec& fr) {
-  double pg[NP], pf2[NP];
-  for (int l = 0; l < NP; l++) pg[l] = pf[l];
-  double gamma = 1., bsq = 0.;
-  int ret = utoprim_2d_fast(U, g, P.gam, P.gam_m1_o_gam, pf, &gamma, &bsq, nullptr);
-  if ((!ret) && (check_gamma(gamma) == 2)) {
-    for (int l = 0; l < B1; l++) pf[l] = pg[l];
-    ret = 1;
-    gamma = 1.;
+// recover_primitives(), src/step_ch.c:801-1024 (FIXUP_TREE 3, entropy fix on),
+// in two parts so that the device can form the entropy face fluxes beside the
+// first: the inversions (recover_invert()), then the entropy fix, floors and
+// ceilings (recover_finish()).
+struct RecoverState {
+  double pf[NP], pg[NP];   // primitives after the inversions; the guess
+  double gamma, bsq;
+  int ret;                 // 0: an inversion succeeded
+};
+// The 1D inversion of a zone from its guess, as recover_invert() falls back to
+// it; it needs nothing of the 2D one, so the device runs both side by side.
+struct Recover1d {
+  double pf[NP];
+  double gamma, bsq;       // set when ret == 0
+  int ret;
+};
+HD void recover_1d(const Params& P, const double* U, const Geom* g, const double* guess, Recover1d& r) {
+  for (int l = 0; l < NP; l++) r.pf[l] = guess[l];
+  r.gamma = 1.;
+  r.bsq = 0.;
+  r.ret = utoprim_1d(U, g, P.gam, r.pf, &r.gamma, &r.bsq);
+}
+HD void recover_2d(const Params& P, const double* U, const Geom* g, RecoverState& s) {
+  for (int l = 0; l < NP; l++) s.pg[l] = s.pf[l];
+  s.gamma = 1.;
+  s.bsq = 0.;
+  s.ret = utoprim_2d_fast(U, g, P.gam, P.gam_m1_o_gam, s.pf, &s.gamma, &s.bsq, nullptr);
+  if ((!s.ret) && (check_gamma(s.gamma) == 2)) {
+    for (int l = 0; l < B1; l++) s.pf[l] = s.pg[l];
+    s.ret = 1;
+    s.gamma = 1.;
   }
-  if (ret) {
-    ret = utoprim_1d(U, g, P.gam, pf, &gamma, &bsq);
-    if ((!ret) && (check_gamma(gamma) == 2)) {
-      for (int l = 0; l < B1; l++) pf[l] = pg[l];
-      ret = 1;
+}
+// the 1D result in place of a failed 2D one
+HD void recover_take_1d(const Recover1d& r, RecoverState& s) {
+  for (int l = 0; l < NP; l++) s.pf[l] = r.pf[l];
+  s.ret = r.ret;
+  if (!r.ret) {
+    s.gamma = r.gamma;
+    s.bsq = r.bsq;
+    if (check_gamma(s.gamma) == 2) {
+      for (int l = 0; l < B1; l++) s.pf[l] = s.pg[l];
+      s.ret = 1;
     }
-    if (ret) gamma = 1.;
   }
+  if (s.ret) s.gamma = 1.;
+}
+HD void recover_invert(const Params& P, const double* U, const Geom* g, RecoverState& s) {
+  recover_2d(P, U, g, s);
+  if (s.ret) {
+    Recover1d r;
+    recover_1d(P, U, g, s.pg, r);
+    recover_take_1d(r, s);
+  }
+}
+// src: the stage's reconstruction source, for the entropy face fluxes (Fs: the
+// fluxes themselves, face f at Fs[f*fs_stride])
+template <bool MIXED>
+HD void recover_finish(const Params& P, const Ptrs& X, int i, int j, int k, double Dt, RecoverState& s,
+                       const double* U, const double* p_old, const Geom* g, double rhoflr, double uuflr,
+                       double* p_gamma, const double* src, const FaceOtf* fo, FailRec& fr,
+                       const double* Fs = nullptr, int fs_stride = 0) {
+  double pf2[NP];
+  double* pf = s.pf;
+  double gamma = s.gamma;
+  const int ret = s.ret;
   *p_gamma = gamma;
 
   int use_ee = 0;
-  if (ret || (pf[UU] < BETA_MIN * bsq) || (pf[RHO] < BETA_MIN * bsq)) use_ee = 1;
+  if (ret || (pf[UU] < BETA_MIN * s.bsq) || (pf[RHO] < BETA_MIN * s.bsq)) use_ee = 1;
 
   if (!use_ee) {
     if (!ret) fail_set(P, fr, NFAIL_USE_FULL_INV, 0, i, j, k);
@@ -614,8 +674,8 @@ HD void recover_primitives(const Params& P, const Ptrs& X, int i, int j, int k, 
   } else {
     if (!ret) { for (int l = 0; l < NP; l++) pf2[l] = pf[l]; }
     else fail_set(P, fr, NFAIL_UTOPRIM, 0, i, j, k);
-    for (int l = 0; l < B1; l++) pf[l] = pg[l];
-    int ret_ee = fixup_entropy_eq<MIXED>(P, X, i, j, k, Dt, p_old, pf, g, U, &gamma, src, fo, fr);
+    for (int l = 0; l < B1; l++) pf[l] = s.pg[l];
+    int ret_ee = fixup_entropy_eq<MIXED>(P, X, i, j, k, Dt, p_old, pf, g, U, &gamma, src, fo, fr, Fs, fs_stride);
     if (ret_ee) {
       if (ret) {
         fail_set(P, fr, NFAIL_UTOPRIM_EE, 1, i, j, k);
@@ -790,25 +850,34 @@ HD void store_zone(const Params& P, const Ptrs& X, int stage, long long c, const
   if (fr.pflag) X.pflag[c] = fr.pflag;
 }
 
-// Full recover_primitives() tree for a zone whose U^{n+1} is known.
-// fo: the stage's face records are evaluated (binary metric) for the
-// entropy fluxes.
-template <bool MIXED>
-HD void recover_zone(const Params& P, const Ptrs& X, int stage, double dt, int i, int j, int k, const double* U,
-                     FailRec& fr, const FaceOtf* fo = nullptr) {
+// Full recover_primitives() tree for a zone whose U^{n+1} is known (s: after
+// the inversions).  fo: the stage's face records are evaluated (binary metric) for the
+// entropy fluxes; Fs, fs_stride: those fluxes, when the caller has formed them.
+template <bool MIXED, int OTF = -1>
+HD void recover_zone_end(const Params& P, const Ptrs& X, int stage, double dt, int i, int j, int k, const double* U,
+                         RecoverState& s, FailRec& fr, const FaceOtf* fo, const double* Fs = nullptr,
+                         int fs_stride = 0) {
   const long long NT = P.nt;
   const long long c = cidx(P, i, j, k);
   const double Dt = (stage == 0) ? 0.5*dt : dt;
   Geom gb;
-  const Geom* g = cent_rec(P, X, i, j, k, gb);
-  double pf[NP], p_raw[NP];
-  zone_guess(P, X, stage, i, c, pf);
+  const Geom* g = cent_rec<OTF>(P, X, i, j, k, gb);
+  double p_raw[NP];
 #pragma unroll
   for (int v = 0; v < NP; v++) p_raw[v] = X.p[v*NT + c];
   double pgam = 1.;
-  recover_primitives<MIXED>(P, X, i, j, k, Dt, pf, U, p_raw, g, floor_rho(P, X, i, c), floor_uu(P, X, i, c),
-                            &pgam, (stage == 0) ? X.p : X.ph, fo, fr);
-  store_zone(P, X, stage, c, pf, pgam, fr);
+  recover_finish<MIXED>(P, X, i, j, k, Dt, s, U, p_raw, g, floor_rho(P, X, i, c), floor_uu(P, X, i, c), &pgam,
+                        (stage == 0) ? X.p : X.ph, fo, fr, Fs, fs_stride);
+  store_zone(P, X, stage, c, s.pf, pgam, fr);
+}
+template <bool MIXED>
+HD void recover_zone(const Params& P, const Ptrs& X, int stage, double dt, int i, int j, int k, const double* U,
+                     FailRec& fr, const FaceOtf* fo = nullptr) {
+  RecoverState s;
+  Geom gb;
+  zone_guess(P, X, stage, i, cidx(P, i, j, k), s.pf);
+  recover_invert(P, U, cent_rec(P, X, i, j, k, gb), s);
+  recover_zone_end<MIXED>(P, X, stage, dt, i, j, k, U, s, fr, fo);
 }
 
 // Whole zone in one pass (the host build's sequence; the device runs the two

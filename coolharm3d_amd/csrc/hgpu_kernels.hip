@@ -111,7 +111,7 @@ __device__ __forceinline__ void mtot_wave_part(const Ptrs& X, double v) {
 }
 // every thread of every workgroup of the grid
 __device__ __forceinline__ void mtot_level2(const Ptrs& X) {
-  __shared__ double s_w[BLOCK / 64];
+  __shared__ double s_w[16];
   const unsigned n = (unsigned)X.status[ST_MPARTS];
   const unsigned G = gridDim.x * blockDim.x;
   double s = 0.;
@@ -253,34 +253,80 @@ __global__ __launch_bounds__(BLOCK, W) void k_update(Params P, Ptrs X, int stage
 }
 
 // Full con-to-prim tree for the queued zones: a fixed grid strides over the
-// queue, so every wave works on queued zones only.
-// G, lvl: with P.otf, the entropy fix's face records are evaluated from the
+// queue, 64 zones to a workgroup of 8 wavefronts.  Few zones take the tree (a
+// few thousandths of a torus), so the launch lasts as long as one zone's serial
+// chain, and the chain is cut by what can run side by side: wavefronts 0-5 form
+// the zones' six entropy face fluxes (one face each: reconstruction and two
+// face states), wavefront 6 runs the 2D inversion and wavefront 7 the 1D one
+// (used where the 2D one fails); then wavefront 6 goes on to the entropy solve
+// with their results from LDS.  One thread per zone took 0.10 ms a stage on every
+// torus (0.20 ms a step at 192x192x128, 0.19 at 67x45x33); this takes 0.14 and
+// 0.08 ms a step, a launch being as long as its slowest zone.
+// G, lvl: with OTF, the entropy fix's face records are evaluated from the
 // orbit of level lvl.
-template <bool MIXED>
-__global__ __launch_bounds__(BLOCK) void k_recover(Params P, Ptrs X, int stage, PnGrid G, int lvl) {
+constexpr int REC_Z = 64, REC_T = 8 * REC_Z;
+template <bool MIXED, int OTF>
+__global__ __launch_bounds__(REC_T) void k_recover(Params P, Ptrs X, int stage, PnGrid G, int lvl) {
+  __shared__ double sF[6 * REC_Z];
+  __shared__ double s1[(NP + 2) * REC_Z];
+  __shared__ int sR[REC_Z];
   mtot_level2(X);   // the update's M_tot parts
   const unsigned n = (unsigned)X.status[ST_SLOW];
-  const unsigned stride = gridDim.x * BLOCK;
+  const unsigned stride = gridDim.x * REC_Z;
   const unsigned rounds = (n + stride - 1) / stride;
   const double dt = X.scal[SC_DT];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   for (unsigned r = 0; r < rounds; r++) {
-    const unsigned slot = r * stride + blockIdx.x * BLOCK + threadIdx.x;
+    const unsigned slot = r * stride + blockIdx.x * REC_Z + lane;
     const bool active = slot < n;
     FailRec fr; fr.clear();
+    RecoverState rs;
+    double U[NP];
     long long c = 0;
+    int i = 0, j = 0, k = 0;
+    FaceOtf fo;
+    if constexpr (OTF) { fo.G = G; fo.o = X.orbit + lvl; }
     if (active) {
       c = X.slow_idx[slot];
-      const int k = (int)(c % P.n3t);
-      const int j = (int)((c / P.n3t) % P.n2t);
-      const int i = (int)(c / ((long long)P.n3t * P.n2t));
-      double U[NP];
+      k = (int)(c % P.n3t);
+      j = (int)((c / P.n3t) % P.n2t);
+      i = (int)(c / ((long long)P.n3t * P.n2t));
+      if (wv < 6) {
+        sF[wv*REC_Z + lane] = entropy_face<MIXED>(P, X, (stage == 0) ? X.p : X.ph, wv, i, j, k, OTF ? &fo : nullptr);
+      } else {
+        Geom gb;
+        const Geom* g = cent_rec<OTF>(P, X, i, j, k, gb);
 #pragma unroll
-      for (int l = 0; l < NP; l++) U[l] = X.Uslow[l*P.nt + c];
-      FaceOtf fo;
-      if (P.otf) { fo.G = G; fo.o = X.orbit + lvl; }
-      recover_zone<MIXED>(P, X, stage, dt, i, j, k, U, fr, P.otf ? &fo : nullptr);
+        for (int l = 0; l < NP; l++) U[l] = X.Uslow[l*P.nt + c];
+        zone_guess(P, X, stage, i, c, rs.pf);
+        if (wv == 6) {
+          recover_2d(P, U, g, rs);
+        } else {
+          Recover1d r1;
+          recover_1d(P, U, g, rs.pf, r1);
+#pragma unroll
+          for (int l = 0; l < NP; l++) s1[l*REC_Z + lane] = r1.pf[l];
+          s1[NP*REC_Z + lane] = r1.gamma;
+          s1[(NP + 1)*REC_Z + lane] = r1.bsq;
+          sR[lane] = r1.ret;
+        }
+      }
     }
-    commit_fail(P, X, fr, active, c, MASK_ALL);
+    __syncthreads();
+    const bool finish = active && wv == 6;
+    if (finish) {
+      if (rs.ret) {
+        Recover1d r1;
+#pragma unroll
+        for (int l = 0; l < NP; l++) r1.pf[l] = s1[l*REC_Z + lane];
+        r1.gamma = s1[NP*REC_Z + lane];
+        r1.bsq = s1[(NP + 1)*REC_Z + lane];
+        r1.ret = sR[lane];
+        recover_take_1d(r1, rs);
+      }
+      recover_zone_end<MIXED, OTF>(P, X, stage, dt, i, j, k, U, rs, fr, OTF ? &fo : nullptr, sF + lane, REC_Z);
+    }
+    commit_fail(P, X, fr, finish, c, MASK_ALL);   // its barriers also keep the LDS until every zone has read it
   }
 }
 
@@ -1094,11 +1140,15 @@ struct GpuBE {
   static int recover_queued(hgpu_ctx* c, int stage) {
     Scope s(c, "recover");
     const long long nint = (long long)c->P.n1 * c->P.n2 * c->P.n3;
-    const unsigned nb = (unsigned)std::min<long long>((nint + BLOCK - 1) / BLOCK, 1024);
-    if (c->P.mixed)
-      hipLaunchKernelGGL(k_recover<true>, dim3(nb), dim3(BLOCK), 0, priv(c)->stream, c->P, c->X, stage, c->pn, stage);
-    else
-      hipLaunchKernelGGL(k_recover<false>, dim3(nb), dim3(BLOCK), 0, priv(c)->stream, c->P, c->X, stage, c->pn, stage);
+    const unsigned nb = (unsigned)std::min<long long>((nint + REC_Z - 1) / REC_Z, 1024);
+    const auto go = [&](auto M, auto O) {
+      hipLaunchKernelGGL((k_recover<decltype(M)::value, decltype(O)::value>), dim3(nb), dim3(REC_T), 0,
+                         priv(c)->stream, c->P, c->X, stage, c->pn, stage);
+    };
+    typedef std::integral_constant<int, 0> Stored;
+    typedef std::integral_constant<int, 1> Evaluated;
+    if (c->P.mixed) { if (c->P.otf) go(std::true_type(), Evaluated()); else go(std::true_type(), Stored()); }
+    else { if (c->P.otf) go(std::false_type(), Evaluated()); else go(std::false_type(), Stored()); }
     return hip_check(hipGetLastError(), "k_recover");
   }
   static int bounds_dir(hgpu_ctx* c, double* S, int dir, int skip_mpi, bool mtot = false) {
