@@ -938,11 +938,12 @@ HD double update_zone(const Params& P, const Ptrs& X, int stage, double dt, int 
 // Boundary conditions, src/bounds.c:31-579 (BC_CARTESIAN_OUTFLOW :58-133,
 // BC_SPHERICAL_OUTFLOW3 :492-579) and inflow_check(), src/bounds.c:2304-2380.
 
+template <int OTF = -1>
 HD void inflow_check(const Params& P, const Ptrs& X, double* pr, int ii, int jj, int kk, int type,
                      FailRec& fr) {
   const int dir = 1;
   Geom gb;
-  const Geom* g = cent_rec(P, X, ii, jj, kk, gb);
+  const Geom* g = cent_rec<OTF>(P, X, ii, jj, kk, gb);
   double gamma;
   if (gamma_calc(pr, g, &gamma)) fr.nf[NFAIL_GAMMA_CALC]++;
   double ucon[4];
@@ -969,39 +970,67 @@ HD void inflow_check(const Params& P, const Ptrs& X, double* pr, int ii, int jj,
   }
 }
 
-// One ghost zone of direction dir.  t enumerates (g, transverse...) for the
-// lower (side 0) and upper (side 1) faces.
-HD void bound_zone(const Params& P, const Ptrs& X, double* S, int dir, int side, int g, int a, int b,
-                   int do_pflag, FailRec& fr) {
-  // a face shared with another block gets its ghosts from that block
-  if ((P.bc_nbr >> (2*dir + side)) & 1) return;
+// Source index of ghost index d along a direction of n interior zones (lower
+// side: side 0): copy of the edge zone, reflection or the periodic image
+HD int bound_src(int d, int n, int side, bool copy, bool periodic) {
+  const int e = n + NG - 1;                                    // last interior zone
+  const int g = side ? d - e - 1 : NG - 1 - d;                 // layer, counted from the face
+  if (copy) return side ? e : NG;
+  if (periodic) return side ? NG + g : e - g;
+  return side ? e - g : NG + g;
+}
+
+// One ghost zone (i,j,k) of bounds(): the x1, x2, x3 fills, each of which reads
+// what the ones before it wrote, as one map from the zone to where its values
+// come from -- x3's image first, then x2's (with the reflected signs), then
+// x1's (with inflow_check()).  Faces shared with another block are not filled:
+// there the chain ends, at the zone itself (nothing to do) or at a ghost zone
+// that no direction writes.  So no zone this writes is read by another.
+// fr counts inflow_check()'s failures of the x1 ghost itself.
+// OTF: as cent_rec().
+template <int OTF = -1>
+HD void bound_zone(const Params& P, const Ptrs& X, double* S, int i, int j, int k, int do_pflag, FailRec& fr) {
   const long long NT = P.nt;
-  const int n1e = P.n1 + NG - 1, n2e = P.n2 + NG - 1, n3e = P.n3 + NG - 1;
-  int di, dj, dk, si, sj, sk;
-  bool reflect = false;
-  if (dir == 0) {
-    // a = j in [N2S,N2E], b = k in [N3S,N3E]
-    dj = sj = a; dk = sk = b;
-    di = side ? (n1e + 1 + g) : (NG - 1 - g);
-    si = side ? n1e : NG;
-  } else if (dir == 1) {
-    // a = i (all), b = k in [N3S,N3E]
-    di = si = a; dk = sk = b;
-    dj = side ? (n2e + 1 + g) : (NG - 1 - g);
-    if (P.bc == BC_SPHERICAL_OUTFLOW3) { sj = side ? (n2e - g) : (NG + g); reflect = true; }
-    else sj = side ? n2e : NG;
-  } else {
-    // a = i (all), b = j (all)
-    di = si = a; dj = sj = b;
-    dk = side ? (n3e + 1 + g) : (NG - 1 - g);
-    if (P.bc == BC_SPHERICAL_OUTFLOW3) sk = side ? (NG + g) : (n3e - g);
-    else sk = side ? n3e : NG;
+  const bool sph = P.bc == BC_SPHERICAL_OUTFLOW3;
+  int si = i, sj = j, sk = k;
+  bool reflect = false, inflow = false, open = true;
+  int side1 = 0;
+  if (k < NG || k >= NG + P.n3) {
+    const int side = k >= NG;
+    if ((P.bc_nbr >> (4 + side)) & 1) return;
+    sk = bound_src(k, P.n3, side, !sph, true);
   }
-  const long long cd = cidx(P, di, dj, dk), cs = cidx(P, si, sj, sk);
+  if (j < NG || j >= NG + P.n2) {
+    const int side = j >= NG;
+    if ((P.bc_nbr >> (2 + side)) & 1) {
+      if (sk == k) return;
+      open = false;
+    } else {
+      sj = bound_src(j, P.n2, side, !sph, false);
+      reflect = sph;
+    }
+  }
+  if (open && (i < NG || i >= NG + P.n1)) {
+    side1 = i >= NG;
+    if ((P.bc_nbr >> side1) & 1) {
+      if (sk == k && sj == j) return;
+    } else {
+      si = bound_src(i, P.n1, side1, true, false);
+      inflow = sph;
+    }
+  }
+  const long long cd = cidx(P, i, j, k), cs = cidx(P, si, sj, sk);
   double pr[NP];
+#pragma unroll
   for (int v = 0; v < NP; v++) pr[v] = S[v*NT + cs];
+  if (inflow) {
+    FailRec own;
+    own.clear();
+    const bool mine = sj == j && sk == k;   // the edges' copies of this ghost do not count again
+    inflow_check<OTF>(P, X, pr, i, sj, sk, side1, mine ? fr : own);
+  }
   if (reflect) { pr[U2] *= -1; pr[B2] *= -1; }
-  if (dir == 0 && P.bc == BC_SPHERICAL_OUTFLOW3) inflow_check(P, X, pr, di, dj, dk, side, fr);
+#pragma unroll
   for (int v = 0; v < NP; v++) S[v*NT + cd] = pr[v];
   if (do_pflag) X.pflag[cd] = X.pflag[cs];
 }
@@ -1250,15 +1279,39 @@ HD Box interior_box(const Params& P) {
   b.hi[0] = NG + P.n1 - 1; b.hi[1] = NG + P.n2 - 1; b.hi[2] = NG + P.n3 - 1;
   return b;
 }
-// ghost layers of direction dir, both sides: (side, g, a, b) flattened as
-// lo = {0, 0, a0, b0}: index box over (side*NG + g, a, b)
-HD Box ghost_box(const Params& P, int dir) {
-  Box b;
-  b.lo[0] = 0; b.hi[0] = 2*NG - 1;
-  if (dir == 0) { b.lo[1] = NG; b.hi[1] = NG + P.n2 - 1; b.lo[2] = NG; b.hi[2] = NG + P.n3 - 1; }
-  else if (dir == 1) { b.lo[1] = 0; b.hi[1] = P.n1t - 1; b.lo[2] = NG; b.hi[2] = NG + P.n3 - 1; }
-  else { b.lo[1] = 0; b.hi[1] = P.n1t - 1; b.lo[2] = 0; b.hi[2] = P.n2t - 1; }
-  return b;
+// Every ghost zone once, in three groups: x1 ghosts of the interior (j,k); x2
+// ghosts at every i, interior k; x3 ghosts at every (i,j).  t < ghost_count()
+// -> (i,j,k).  Along x3 the 2 NG layers are the fastest index, so a
+// wavefront's accesses stay within the rows' ends rather than one cache line per
+// lane.
+HD long long ghost_count(const Params& P, int group) {
+  if (group == 0) return 2LL*NG * P.n2 * P.n3;
+  if (group == 1) return 2LL*NG * P.n1t * P.n3;
+  return 2LL*NG * P.n1t * P.n2t;
+}
+HD void ghost_at(const Params& P, long long t, int& i, int& j, int& k) {
+  const long long n0 = ghost_count(P, 0), n1 = ghost_count(P, 1);
+  if (t < n0) {
+    k = NG + (int)(t % P.n3);
+    const long long r = t / P.n3;
+    j = NG + (int)(r % P.n2);
+    const int s = (int)(r / P.n2);
+    i = (s < NG) ? s : P.n1 + s;
+  } else if (t < n0 + n1) {
+    t -= n0;
+    k = NG + (int)(t % P.n3);
+    const long long r = t / P.n3;
+    i = (int)(r % P.n1t);
+    const int s = (int)(r / P.n1t);
+    j = (s < NG) ? s : P.n2 + s;
+  } else {
+    t -= n0 + n1;
+    const int s = (int)(t % (2*NG));
+    k = (s < NG) ? s : P.n3 + s;
+    const long long r = t / (2*NG);
+    j = (int)(r % P.n2t);
+    i = (int)(r / P.n2t);
+  }
 }
 // interior corners for div B: (N1S+1..N1E, ...) so that all 8 zones are interior
 HD Box divb_box(const Params& P) {

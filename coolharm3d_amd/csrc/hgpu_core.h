@@ -436,11 +436,10 @@ struct Api {
 
   // bounds(prim, skip_mpi): skip_mpi = 0 always applies the physical BCs;
   // skip_mpi = 1 only if boundary_phys_pflag (src/bounds.c:56)
-  // after_update: the first bounds after an update (it completes M_tot)
-  static int bounds(hgpu_ctx* c, double* S, int skip_mpi, bool after_update = false) {
-    int rc = 0;
-    for (int dir = 0; dir < 3; dir++) rc |= BE::bounds_dir(c, S, dir, skip_mpi, after_update && dir == 0);
-    return rc;
+  // after_update: the first bounds after an update (it completes M_tot);
+  // last: the step's last launch, which also takes the new time step
+  static int bounds(hgpu_ctx* c, double* S, int skip_mpi, bool after_update = false, bool last = false) {
+    return BE::bounds(c, S, skip_mpi, after_update, last);
   }
 
   // One advance() stage plus its boundaries and fixups (src/step_ch.c:92-121,
@@ -489,10 +488,10 @@ struct Api {
   // The rest of the stage after bounds(prim,0) (src/step_ch.c:105-114,
   // :171-180): the interpolating fixups, bounds(prim,1) where the boundary
   // flags ask for it, the flags cleared.
-  static int stage_fixup(hgpu_ctx* c, int stage) {
+  static int stage_fixup(hgpu_ctx* c, int stage, bool last = false) {
     double* dst = (stage == 0) ? c->X.ph : c->X.p;
     int rc = BE::fixup_interp(c, dst);   // fixup_interp_v(), then fixup_interp_prim()
-    rc |= bounds(c, dst, 1);   // the boundary flags are cleared when the next stage starts
+    rc |= bounds(c, dst, 1, false, last);   // the boundary flags are cleared when the next stage starts
     return rc;
   }
 
@@ -619,8 +618,7 @@ struct Api {
     rc |= stage_fixup(c, 0);
     rc |= BE::begin_stage(c);         // src/step_ch.c:117-121
     rc |= substep(c, 1);
-    rc |= stage_fixup(c, 1);
-    rc |= BE::timestep(c);            // src/step_ch.c:218-223
+    rc |= stage_fixup(c, 1, true);    // with timestep(), src/step_ch.c:218-223
     if (c->P.dyn) {
       // the state is now at t + dt: level 2 (centres) describes it
       c->X.geom = c->X.geom_n = c->X.geom_new = c->lev[2];

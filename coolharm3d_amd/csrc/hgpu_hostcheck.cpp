@@ -136,18 +136,17 @@ struct HostBE {
     c->X.scal[SC_MTOT] = mtot;
     return 0;
   }
-  static int bounds_dir(hgpu_ctx* c, double* S, int dir, int skip_mpi, bool = false) {
+  static int bounds(hgpu_ctx* c, double* S, int skip_mpi, bool = false, bool tstep = false) {
+    if (tstep) timestep_update(c->P, c->X);
     if (skip_mpi && !c->X.status[ST_BOUNDARY_PHYS]) return 0;
     const int do_pflag = c->X.status[ST_FAILURE_EXISTS] ? 1 : 0;
-    Box b = ghost_box(c->P, dir);
-    const int n1e = c->P.n1 + NG - 1;
-    for (long long t = 0; t < b.count(); t++) {
-      int sg, a, bb;
-      b.at(t, sg, a, bb);
-      const int side = sg / NG, g = sg % NG;
+    const long long n = ghost_count(c->P, 0) + ghost_count(c->P, 1) + ghost_count(c->P, 2);
+    for (long long t = n - 1; t >= 0; t--) {   // any order will do
+      int i, j, k;
+      ghost_at(c->P, t, i, j, k);
       FailRec fr; fr.clear();
-      bound_zone(c->P, c->X, S, dir, side, g, a, bb, do_pflag, fr);
-      if (dir == 0) host_commit(c->P, c->X, fr, cidx(c->P, side ? (n1e + 1 + g) : (NG - 1 - g), a, bb), true);
+      bound_zone(c->P, c->X, S, i, j, k, do_pflag, fr);
+      host_commit(c->P, c->X, fr, cidx(c->P, i, j, k), true);
     }
     return 0;
   }

@@ -43,12 +43,14 @@ __global__ __launch_bounds__(64) void k_orbit(Ptrs X, PnBinary B, PnOrbit* out) 
 }
 
 __global__ __launch_bounds__(BLOCK) void k_emf(Params P, Ptrs X, Box b, Tiling T) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) X.status[ST_PFDIRTY] = 0;   // k_begin_stage has used it
   int i, j, k;
   if (!tile_index(b, T, i, j, k)) return;
   emf_edge(P, X, i, j, k);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_emf_mixed(Params P, Ptrs X, Box b, Tiling T) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) X.status[ST_PFDIRTY] = 0;
   int i, j, k;
   if (!tile_index(b, T, i, j, k)) return;
   emf_edge_mixed(P, X, i, j, k);
@@ -330,17 +332,20 @@ __global__ __launch_bounds__(REC_T) void k_recover(Params P, Ptrs X, int stage, 
   }
 }
 
-// mtot: the first boundary kernel after an update, whose first workgroup
-// completes that update's M_tot.  One kernel per direction: only x1 runs
-// inflow_check() (its geometry record and registers), so the x2 and x3 fills
-// are lean copies.
-template <int DIR>
-__global__ __launch_bounds__(BLOCK) void k_bounds(Params P, Ptrs X, double* S, int skip_mpi, Box b, int mtot) {
-  constexpr int dir = DIR;
+// bounds(): every ghost zone in one launch (bound_zone()).  Both of a stage's
+// bounds, three launches each before: 0.135 -> 0.081 ms a step at 192x192x128,
+// 0.079 -> 0.030 on small grids, where a launch costs more than its zones.
+// mtot: after an update, whose M_tot the first workgroup completes.
+// tstep: the step's last launch, whose first thread also takes the new time step
+// (it needs the fluxes' speeds and the fixups' counters, not the ghosts).
+template <int OTF>
+__global__ __launch_bounds__(BLOCK) void k_bounds(Params P, Ptrs X, double* S, int skip_mpi, long long n, int mtot,
+                                                  int tstep) {
   if (mtot && blockIdx.x == 0) mtot_level3(X);
+  if (tstep && blockIdx.x == 0 && threadIdx.x == 0) timestep_update(P, X);
   if (skip_mpi && !X.status[ST_BOUNDARY_PHYS]) return;
   const int do_pflag = X.status[ST_FAILURE_EXISTS] ? 1 : 0;
-  const long long n = b.count(), stride = (long long)gridDim.x * BLOCK;
+  const long long stride = (long long)gridDim.x * BLOCK;
   const long long rounds = (n + stride - 1) / stride;   // the same in every workgroup (barriers)
   for (long long rd = 0; rd < rounds; rd++) {
     const long long t = rd * stride + (long long)blockIdx.x * BLOCK + threadIdx.x;
@@ -348,26 +353,12 @@ __global__ __launch_bounds__(BLOCK) void k_bounds(Params P, Ptrs X, double* S, i
     FailRec fr; fr.clear();
     long long c = 0;
     if (active) {
-      int sg, a, bb;
-      if (dir == 2) {
-        // x3 ghosts: the 2 NG layers of one (i, j) row are the fastest index, so
-        // a wavefront's accesses stay within the rows' ends rather than one
-        // cache line per lane
-        const int nsg = b.hi[0] - b.lo[0] + 1, nb = b.hi[2] - b.lo[2] + 1;
-        sg = b.lo[0] + (int)(t % nsg);
-        const long long r = t / nsg;
-        bb = b.lo[2] + (int)(r % nb);
-        a = b.lo[1] + (int)(r / nb);
-      } else {
-        b.at(t, sg, a, bb);
-      }
-      const int side = sg / NG, g = sg % NG;
-      bound_zone(P, X, S, dir, side, g, a, bb, do_pflag, fr);
-      // nfail of inflow_check() belongs to the ghost zone
-      const int n1e = P.n1 + NG - 1;
-      if (dir == 0) c = cidx(P, side ? (n1e + 1 + g) : (NG - 1 - g), a, bb);
+      int i, j, k;
+      ghost_at(P, t, i, j, k);
+      bound_zone<OTF>(P, X, S, i, j, k, do_pflag, fr);
+      c = cidx(P, i, j, k);   // nfail of inflow_check() belongs to the ghost zone
     }
-    commit_fail(P, X, fr, active && dir == 0, c, MASK_GAMMA);
+    commit_fail(P, X, fr, active, c, MASK_GAMMA);
   }
 }
 
@@ -409,24 +400,27 @@ __global__ __launch_bounds__(BLOCK) void k_fixup_init(Params P, Ptrs X, Box b) {
   commit_fail(P, X, fr, active, c, MASK_ALL);
 }
 
-__global__ __launch_bounds__(BLOCK) void k_clear_pflag(Ptrs X, long long nt) {
-  if (!X.status[ST_FAILURE_EXISTS]) return;
+// Start of a stage, one launch: the flag map cleared if a zone was flagged
+// since it last was (a word of its own says so: the first workgroup may reset
+// the others before the last one has started; k_emf clears it, after this
+// kernel and before anything can flag a zone again), and the words a stage
+// starts from: failure words, boundary flags, fastest speeds, an empty
+// slow-zone queue.
+__global__ __launch_bounds__(BLOCK) void k_begin_stage(Ptrs X, long long nt) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) {
+      X.status[ST_FAILURE_EXISTS] = 0;
+      X.status[ST_FAILTYPE_V] = 0;
+      X.status[ST_FAILTYPE_PRIM] = 0;
+      X.status[ST_BOUNDARY_PHYS] = 0;
+      X.status[ST_BOUNDARY_MPI] = 0;
+      X.status[ST_SLOW] = 0;
+    }
+    if (threadIdx.x < 4) X.status[ST_VMAX + threadIdx.x] = 0;
+  }
+  if (!X.status[ST_PFDIRTY]) return;
   const long long stride = (long long)gridDim.x * BLOCK;
   for (long long t = (long long)blockIdx.x * BLOCK + threadIdx.x; t < nt; t += stride) X.pflag[t] = 0;
-}
-
-// the words a stage starts from: failure words, boundary flags, fastest
-// speeds, an empty slow-zone queue
-__global__ void k_reset_stage_words(Ptrs X) {
-  if (threadIdx.x == 0) {
-    X.status[ST_FAILURE_EXISTS] = 0;
-    X.status[ST_FAILTYPE_V] = 0;
-    X.status[ST_FAILTYPE_PRIM] = 0;
-    X.status[ST_BOUNDARY_PHYS] = 0;
-    X.status[ST_BOUNDARY_MPI] = 0;
-    X.status[ST_SLOW] = 0;
-  }
-  if (threadIdx.x < 4) X.status[ST_VMAX + threadIdx.x] = 0;
 }
 
 __global__ void k_reset_words(Ptrs X, int first, int n) {
@@ -1151,18 +1145,16 @@ struct GpuBE {
     else { if (c->P.otf) go(std::false_type(), Evaluated()); else go(std::false_type(), Stored()); }
     return hip_check(hipGetLastError(), "k_recover");
   }
-  static int bounds_dir(hgpu_ctx* c, double* S, int dir, int skip_mpi, bool mtot = false) {
-    Box b = ghost_box(c->P, dir);
+  static int bounds(hgpu_ctx* c, double* S, int skip_mpi, bool mtot = false, bool tstep = false) {
     Scope s(c, "bounds");
+    const long long n = ghost_count(c->P, 0) + ghost_count(c->P, 1) + ghost_count(c->P, 2);
     // bounds(prim,0) has work every time: one zone per thread; bounds(prim,1)
     // mostly finds its flag clear: a strided grid
-    const unsigned nb = skip_mpi ? std::min(nblocks(b.count()), priv(c)->flag_grid) : nblocks(b.count());
-    if (dir == 0)
-      hipLaunchKernelGGL(k_bounds<0>, dim3(nb), dim3(BLOCK), 0, priv(c)->stream, c->P, c->X, S, skip_mpi, b, mtot ? 1 : 0);
-    else if (dir == 1)
-      hipLaunchKernelGGL(k_bounds<1>, dim3(nb), dim3(BLOCK), 0, priv(c)->stream, c->P, c->X, S, skip_mpi, b, mtot ? 1 : 0);
+    const unsigned nb = skip_mpi ? std::min(nblocks(n), priv(c)->flag_grid) : nblocks(n);
+    if (c->P.otf)
+      hipLaunchKernelGGL(k_bounds<1>, dim3(nb), dim3(BLOCK), 0, priv(c)->stream, c->P, c->X, S, skip_mpi, n, mtot, tstep);
     else
-      hipLaunchKernelGGL(k_bounds<2>, dim3(nb), dim3(BLOCK), 0, priv(c)->stream, c->P, c->X, S, skip_mpi, b, mtot ? 1 : 0);
+      hipLaunchKernelGGL(k_bounds<0>, dim3(nb), dim3(BLOCK), 0, priv(c)->stream, c->P, c->X, S, skip_mpi, n, mtot, tstep);
     return hip_check(hipGetLastError(), "k_bounds");
   }
   static int fixup_interp(hgpu_ctx* c, double* S) {
@@ -1216,10 +1208,9 @@ struct GpuBE {
   // before each stage: flag map, failure words and boundary flags cleared,
   // fastest speeds reset, the slow-zone queue emptied
   static int begin_stage(hgpu_ctx* c) {
-    hipLaunchKernelGGL(k_clear_pflag, dim3(std::min(nblocks(c->P.nt), priv(c)->flag_grid)), dim3(BLOCK), 0,
+    hipLaunchKernelGGL(k_begin_stage, dim3(std::min(nblocks(c->P.nt), priv(c)->flag_grid)), dim3(BLOCK), 0,
                        priv(c)->stream, c->X, c->P.nt);
-    hipLaunchKernelGGL(k_reset_stage_words, dim3(1), dim3(64), 0, priv(c)->stream, c->X);
-    return hip_check(hipGetLastError(), "k_reset_stage_words");
+    return hip_check(hipGetLastError(), "k_begin_stage");
   }
   static int timestep(hgpu_ctx* c) {
     hipLaunchKernelGGL(k_timestep, dim3(1), dim3(64), 0, priv(c)->stream, c->P, c->X);

@@ -79,6 +79,7 @@ __device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, cons
     const unsigned f = s_flags;
     if (f) {
       atomicOr(&X.status[ST_FAILURE_EXISTS], 1ull);
+      atomicOr(&X.status[ST_PFDIRTY], 1ull);
       if (f & 2u) atomicOr(&X.status[ST_FAILTYPE_PRIM], 1ull);
       if (f & 4u) atomicOr(&X.status[ST_FAILTYPE_V], 1ull);
       if (f & 8u) atomicOr(&X.status[ST_BOUNDARY_PHYS], 1ull);

@@ -126,7 +126,8 @@ enum {
   ST_CRASH_NBAD = 29,        // its n_bad
   ST_MPARTS = 30,            // M_tot parts of the last update (one per wavefront)
   ST_MPARTS2 = 31,           // their second-level parts (one per k_recover workgroup)
-  ST_WORDS = 32
+  ST_PFDIRTY = 32,           // a flagged zone since the flag map was last cleared
+  ST_WORDS = 33
 };
 
 // Device scalars of the integrator (t, dt ... of src/globals.h:380-390).
