@@ -261,9 +261,8 @@ struct HostBE {
     for (int i = NG; i < NG + P.n1; i++)
       for (int j = NG; j < NG + P.n2; j++)
         for (int k = NG; k < NG + P.n3; k++) {
-          double Xc[4], dg[PN_NDG];
-          zone_X(P, c->pn, i, j, k, CENT, Xc);
-          pn_metric_dg(c->pn.B, c->orbit[tsel], Xc[1], Xc[2], Xc[3], dg);
+          double dg[PN_NDG];
+          pn_zone_dg(P, c->pn, c->orbit[tsel], i, j, k, dg);
           const long long cid = conn_id(P, i, j, k);
           for (int l = 0; l < PN_NDG; l++) dst[l * P.nconn + cid] = dg[l];
         }

@@ -215,8 +215,7 @@ __global__ __launch_bounds__(BLOCK, W) void k_update(Params P, Ptrs X, int stage
     if constexpr (OTF) {
       // the stage's record for U^n in the predictor (the corrector reads U^n,
       // and the source terms come precomputed by k_source_otf: evaluating the
-      // metric derivatives here, by forward-mode differentiation, needs ~200
-      // VGPRs on top of the update's), then the result's record for the
+      // metric derivatives here needs their registers on top of the update's), then the result's record for the
       // inversion
       {
         Geom gs;
@@ -524,10 +523,8 @@ __global__ __launch_bounds__(BLOCK) void k_fill_conn(Params P, Ptrs X, PnGrid G,
   const int k = NG + (int)(z % P.n3);
   const int j = NG + (int)((z / P.n3) % P.n2);
   const int i = NG + (int)(z / ((long long)P.n3 * P.n2));
-  double Xc[4];
-  zone_X(P, G, i, j, k, CENT, Xc);
   double dg[PN_NDG];
-  pn_metric_dg(G.B, X.orbit[tsel], Xc[1], Xc[2], Xc[3], dg);
+  pn_zone_dg(P, G, X.orbit[tsel], i, j, k, dg);
   const long long cid = conn_id(P, i, j, k);
   for (int l = 0; l < PN_NDG; l++) dst[l * P.nconn + cid] = dg[l];   // structure-of-arrays levels
 }
@@ -564,10 +561,8 @@ __global__ __launch_bounds__(BLOCK, 2) void k_source_otf(Params P, Ptrs X, PnGri
       source_dyn_state(P, X, phz, GeomView<GK_DIAG, const Geom*>{&gs}, i, sd);
       gdet = gs.g;
     }
-    double Xc[4];
-    zone_X(P, G, i, j, k, CENT, Xc);
     double dg[PN_NDG], dU[NP];
-    pn_metric_dg(G.B, o, Xc[1], Xc[2], Xc[3], dg);
+    pn_zone_dg(P, G, o, i, j, k, dg);
     source_dyn_finish(P, sd, dg, 1, gdet, dU);
     fr.nf[NFAIL_GAMMA_CALC] += sd.gfail;
     const long long cid = conn_id(P, i, j, k);

@@ -25,10 +25,10 @@
 //   coordinates is J^T g_harmonic J with J = d(t, x, y, z)/d(t, X1, X2, X3),
 //   which for this conformally flat spatial metric and orthogonal map has a
 //   closed form (pn_gcov_num()).
-// * Everything is templated on the scalar: double for values, Dual4 for values
-//   and the four partial derivatives d/d(t, X1, X2, X3) (forward-mode
-//   differentiation), from which the connection Gamma^a_bc, including the
-//   time derivatives of the moving metric, is formed exactly.
+// * The metric's first derivatives, time derivatives of the moving metric
+//   included, are closed-form (pn_metric_dg_coords()); the connection Gamma^a_bc
+//   is formed from them.  The orbit's time derivatives come from forward-mode
+//   numbers (Dual4), once per time level.
 #pragma once
 #include "hgpu_types.h"
 #include <math.h>
@@ -240,6 +240,15 @@ HD void pn_coord2(const PnBinary& B, const T& X2, T* st, T* ct, T* dth) {
   *ct = cos(th);
   if (fabs(value(*st)) < 1.E-16) set_value(*st, value(*st) >= 0. ? 1.E-16 : -1.E-16);   // trigvalues(), src/metric.c:29-40
 }
+// d2theta/dX2^2 (the derivative of pn_coord2()'s dtheta/dX2)
+HD double pn_ddtheta(const PnBinary& B, double X2) {
+  if (B.coords == 4) {
+    const double f = 2. * seesaw_unit(X2) - 1.;
+    const int n = B.diag3_exponent;
+    return 2. * M_PI * n * (n - 1) * B.diag3_factor * ::pow(f, (double)(n - 2));
+  }
+  return -4. * M_PI * M_PI * B.h_slope * ::sin(2. * M_PI * X2);
+}
 template <class T>
 HD void pn_coord3(const T& X3, T* sp, T* cp) {
   *sp = sin(X3);
@@ -300,26 +309,121 @@ HD void pn_gcomp(int m, int* a, int* b) {
 }
 constexpr int PN_NDG = 4 * PN_NG;   // dg[nu * PN_NG + m] = d g_{ab(m)} / dx^nu, x = (t, X1, X2, X3)
 
-// First derivatives of the numerical metric at (X1, X2, X3) and the level of
-// orbit o, by forward-mode differentiation with the orbit's time derivatives.
+// First derivatives of the numerical metric from the coordinate functions (ddth:
+// d2theta/dX2^2) at the level of orbit o, in closed form.  The potentials depend
+// on the point only through the distances and projections to the two holes, so
+// each derivative is a few scalars per hole: with d = x - y, q = 1/|d| and the
+// columns J_n of the map along the orthogonal unit vectors e_r, e_theta, e_phi,
+//   d_n q = -q^3 d.J_n,  d_t q = q^3 d.ydot,  nv = q d.v,
+//   d_n nv = q (v.J_n - nv q d.J_n),  d_t nv = q (d.vdot - ydot.v) + nv q^2 d.ydot.
+// Forward-mode numbers (four partial derivatives carried through every
+// operation, most of them zeros) took ~2500 FP64 operations and 200 registers
+// for the 28 values; this takes ~350.  Source kernel of the binary disk,
+// 120x64x160: 125 -> 76 us a stage (capped at 3 wavefronts per SIMD: the same).
+HD void pn_metric_dg_coords(const PnBinary& B, const PnOrbit& o, const PnCoords<double>& C, double ddth, double* dg) {
+  const double er[3] = {C.st*C.cp, C.st*C.sp, C.ct}, et[3] = {C.ct*C.cp, C.ct*C.sp, -C.st}, ep[2] = {-C.sp, C.cp};
+  const double R = C.r*C.dth, rs = C.r*C.st;
+  const double sc[3] = {C.dr, R, rs};          // |J_n|
+  const double x[3] = {C.r*er[0], C.r*er[1], C.r*er[2]};
+  const double m[2] = {B.m1, B.m2};
+  double q[2], dq[2][4], vJ[2][3], aJ[2][3];   // 1/r, its derivatives (t, 1, 2, 3), v.J_n, vdot.J_n
+  double r2[2], nv[2], dnv[2][4], vsq[2], dvsq[2], D[2][3], dyd[2];
+  for (int a = 0; a < 2; a++) {
+    const double *y = o.y[a], *v = o.v[a], *yd = o.ydot[a], *vd = o.vdot[a];
+    const double d[3] = {x[0] - y[0], x[1] - y[1], x[2] - y[2]};
+    r2[a] = d[0]*d[0] + d[1]*d[1] + d[2]*d[2];
+    q[a] = 1./::sqrt(r2[a]);
+    D[a][0] = sc[0]*(d[0]*er[0] + d[1]*er[1] + d[2]*er[2]);
+    D[a][1] = sc[1]*(d[0]*et[0] + d[1]*et[1] + d[2]*et[2]);
+    D[a][2] = sc[2]*(d[0]*ep[0] + d[1]*ep[1]);
+    vJ[a][0] = sc[0]*(v[0]*er[0] + v[1]*er[1] + v[2]*er[2]);
+    vJ[a][1] = sc[1]*(v[0]*et[0] + v[1]*et[1] + v[2]*et[2]);
+    vJ[a][2] = sc[2]*(v[0]*ep[0] + v[1]*ep[1]);
+    aJ[a][0] = sc[0]*(vd[0]*er[0] + vd[1]*er[1] + vd[2]*er[2]);
+    aJ[a][1] = sc[1]*(vd[0]*et[0] + vd[1]*et[1] + vd[2]*et[2]);
+    aJ[a][2] = sc[2]*(vd[0]*ep[0] + vd[1]*ep[1]);
+    const double q3 = q[a]*q[a]*q[a];
+    dyd[a] = d[0]*yd[0] + d[1]*yd[1] + d[2]*yd[2];
+    nv[a] = q[a]*(d[0]*v[0] + d[1]*v[1] + d[2]*v[2]);
+    vsq[a] = v[0]*v[0] + v[1]*v[1] + v[2]*v[2];
+    dvsq[a] = 2.*(v[0]*vd[0] + v[1]*vd[1] + v[2]*vd[2]);
+    dq[a][0] = q3*dyd[a];
+    dnv[a][0] = q[a]*((d[0]*vd[0] + d[1]*vd[1] + d[2]*vd[2]) - (yd[0]*v[0] + yd[1]*v[1] + yd[2]*v[2]))
+              + nv[a]*q[a]*q[a]*dyd[a];
+    for (int n = 0; n < 3; n++) {
+      dq[a][1 + n] = -q3*D[a][n];
+      dnv[a][1 + n] = q[a]*(vJ[a][n] - nv[a]*q[a]*D[a][n]);
+    }
+  }
+  const double e[3] = {o.y[0][0] - o.y[1][0], o.y[0][1] - o.y[1][1], o.y[0][2] - o.y[1][2]};
+  const double ed[3] = {o.ydot[0][0] - o.ydot[1][0], o.ydot[0][1] - o.ydot[1][1], o.ydot[0][2] - o.ydot[1][2]};
+  const double b2 = e[0]*e[0] + e[1]*e[1] + e[2]*e[2], ib = 1./::sqrt(b2), ib3 = ib*ib*ib;
+  const double eed = e[0]*ed[0] + e[1]*ed[1] + e[2]*ed[2];
+  const double dib = -eed*ib3, dib3 = 3.*ib*ib*dib;   // d_t of 1/b and 1/b^3
+  const double mm = m[0]*m[1];
+  // potentials and their derivatives along nu = t, 1, 2, 3
+  double U = m[0]*q[0] + m[1]*q[1];
+  double dU[4], dV[4] = {0., 0., 0., 0.};
+  for (int nu = 0; nu < 4; nu++) dU[nu] = m[0]*dq[0][nu] + m[1]*dq[1][nu];
+  for (int a = 0; a < 2; a++) {
+    const int b = 1 - a;
+    const double A = 1. + 2.*vsq[a] - 0.5*nv[a]*nv[a];
+    const double Cc = r2[b] - r2[a] - b2;
+    const double f = m[a]*A - mm*ib + 0.25*mm*Cc*ib3;   // V = sum_a q_a f_a
+    for (int nu = 0; nu < 4; nu++) {
+      double df;
+      if (nu == 0) {
+        const double dC = 2.*(dyd[a] - dyd[b]) - 2.*eed;
+        df = m[a]*(2.*dvsq[a] - nv[a]*dnv[a][0]) - mm*dib + 0.25*mm*(dC*ib3 + Cc*dib3);
+      } else {
+        const double dC = 2.*(D[b][nu - 1] - D[a][nu - 1]);
+        df = -m[a]*nv[a]*dnv[a][nu] + 0.25*mm*dC*ib3;
+      }
+      dV[nu] += dq[a][nu]*f + q[a]*df;
+    }
+  }
+  // V_i J^i_n / |J_n|: the vector potential along the unit vectors
+  double w[3];
+  const double vr[3] = {m[0]*q[0]*o.v[0][0] + m[1]*q[1]*o.v[1][0], m[0]*q[0]*o.v[0][1] + m[1]*q[1]*o.v[1][1],
+                        m[0]*q[0]*o.v[0][2] + m[1]*q[1]*o.v[1][2]};
+  w[0] = vr[0]*er[0] + vr[1]*er[1] + vr[2]*er[2];
+  w[1] = vr[0]*et[0] + vr[1]*et[1] + vr[2]*et[2];
+  w[2] = vr[0]*ep[0] + vr[1]*ep[1];
+  // V_i d_nu J^i_n
+  const double dJ[4][3] = {{0., 0., 0.},
+                           {C.dr*w[0], C.dr*C.dth*w[1], C.dr*C.st*w[2]},
+                           {C.dr*C.dth*w[1], C.r*ddth*w[1] - R*C.dth*w[0], R*C.ct*w[2]},
+                           {C.dr*C.st*w[2], R*C.ct*w[2], -rs*(C.st*w[0] + C.ct*w[1])}};
+  const double A = 1. + 2.*U;
+  const double g11 = C.dr*C.dr, g22 = R*R, g33 = rs*rs;
+  for (int nu = 0; nu < 4; nu++) {
+    double* g = dg + nu*PN_NG;
+    g[0] = 2.*dV[nu] - 4.*U*dU[nu];
+    for (int n = 0; n < 3; n++) {
+      double s = m[0]*vJ[0][n]*dq[0][nu] + m[1]*vJ[1][n]*dq[1][nu];
+      if (nu == 0) s += m[0]*aJ[0][n]*q[0] + m[1]*aJ[1][n]*q[1];
+      else s += dJ[nu][n];
+      g[1 + n] = -4.*s;
+    }
+    g[4] = 2.*dU[nu]*g11;
+    g[5] = 2.*dU[nu]*g22;
+    g[6] = 2.*dU[nu]*g33;
+  }
+  // the scale factors' own derivatives: dr along 1; R and r sin(theta) along 1 and 2
+  dg[1*PN_NG + 4] += 2.*A*g11;
+  dg[1*PN_NG + 5] += 2.*A*R*C.dr*C.dth;
+  dg[2*PN_NG + 5] += 2.*A*R*C.r*ddth;
+  dg[1*PN_NG + 6] += 2.*A*rs*C.dr*C.st;
+  dg[2*PN_NG + 6] += 2.*A*rs*R*C.ct;
+}
+
+// The same at numerical coordinates.
 HD void pn_metric_dg(const PnBinary& B, const PnOrbit& o, double X1, double X2, double X3, double* dg) {
-  Dual4 yd[2][3], vd[2][3];
-  for (int a = 0; a < 2; a++)
-    for (int i = 0; i < 3; i++) {
-      yd[a][i] = dc(o.y[a][i]); yd[a][i].d[0] = o.ydot[a][i];
-      vd[a][i] = dc(o.v[a][i]); vd[a][i].d[0] = o.vdot[a][i];
-    }
-  Dual4 g[4][4];
-  pn_gcov_num_pot(B, dvar(X1, 1), dvar(X2, 2), dvar(X3, 3), g,
-                  [&](const Dual4 x[3], Dual4& U, Dual4& V, Dual4 Vi[3]) {
-                    pn_potentials_yv<Dual4>(B, yd, vd, x, U, V, Vi);
-                  });
-  for (int nu = 0; nu < 4; nu++)
-    for (int m = 0; m < PN_NG; m++) {
-      int a, b;
-      pn_gcomp(m, &a, &b);
-      dg[nu * PN_NG + m] = g[a][b].d[nu];
-    }
+  PnCoords<double> C;
+  pn_coord1(B, X1, &C.r, &C.dr);
+  pn_coord2(B, X2, &C.st, &C.ct, &C.dth);
+  pn_coord3(X3, &C.sp, &C.cp);
+  pn_metric_dg_coords(B, o, C, pn_ddtheta(B, X2), dg);
 }
 
 // Inverse and determinant of a 4x4 matrix by the Laplace expansion in 2x2
@@ -396,7 +500,7 @@ HD void pn_geom_orb(const PnBinary& B, const PnOrbit& o, double X1, double X2, d
 
 // Binary and grid of a context whose metric is the binary's: the numerical
 // coordinates of zone (i,j,k) at position pos (coord(), src/coord.c:182-228).
-HD long long pn_tab_size(const Params& P) { return 2LL * (2 * P.n1t + 3 * P.n2t + 2 * P.n3t); }
+HD long long pn_tab_size(const Params& P) { return 2LL * (2 * P.n1t + 4 * P.n2t + 2 * P.n3t); }
 HD void zone_X(const Params& P, const PnGrid& G, int i, int j, int k, int pos, double* X) {
   const double h1 = (pos == FACE1 || pos == CORN) ? 0. : 0.5;
   const double h2 = (pos == FACE2 || pos == CORN) ? 0. : 0.5;
@@ -412,8 +516,8 @@ HD void pn_zone_coords(const Params& P, const PnGrid& G, int i, int j, int k, in
   const int h2 = (pos == FACE2 || pos == CORN) ? 0 : 1;
   const int h3 = (pos == FACE3 || pos == CORN) ? 0 : 1;
   const double* t1 = G.tab + 2 * (h1 * P.n1t + i);
-  const double* t2 = G.tab + 4 * P.n1t + 3 * (h2 * P.n2t + j);
-  const double* t3 = G.tab + 4 * P.n1t + 6 * P.n2t + 2 * (h3 * P.n3t + k);
+  const double* t2 = G.tab + 4 * P.n1t + 4 * (h2 * P.n2t + j);
+  const double* t3 = G.tab + 4 * P.n1t + 8 * P.n2t + 2 * (h3 * P.n3t + k);
   C.r = t1[0]; C.dr = t1[1];
   C.st = t2[0]; C.ct = t2[1]; C.dth = t2[2];
   C.sp = t3[0]; C.cp = t3[1];
@@ -428,18 +532,27 @@ HD void pn_tab_entry(const Params& P, const PnGrid& G, double* tab, long long e)
   e -= 2LL * P.n1t;
   if (e < 2LL * P.n2t) {
     const int h = (int)(e / P.n2t), j = (int)(e % P.n2t);
-    double* t = tab + 4 * P.n1t + 3 * e;
-    pn_coord2(G.B, G.x0[2] + (j + G.gpos[1] + 0.5 * h) * P.dx[2], &t[0], &t[1], &t[2]);
+    double* t = tab + 4 * P.n1t + 4 * e;
+    const double X2 = G.x0[2] + (j + G.gpos[1] + 0.5 * h) * P.dx[2];
+    pn_coord2(G.B, X2, &t[0], &t[1], &t[2]);
+    t[3] = pn_ddtheta(G.B, X2);
     return;
   }
   e -= 2LL * P.n2t;
   if (e < 2LL * P.n3t) {
     const int h = (int)(e / P.n3t), k = (int)(e % P.n3t);
-    double* t = tab + 4 * P.n1t + 6 * P.n2t + 2 * e;
+    double* t = tab + 4 * P.n1t + 8 * P.n2t + 2 * e;
     pn_coord3(G.x0[3] + (k + G.gpos[2] + 0.5 * h) * P.dx[3], &t[0], &t[1]);
   }
 }
 HD long long pn_tab_entries(const Params& P) { return 2LL * (P.n1t + P.n2t + P.n3t); }
+// Metric derivatives at the centre of zone (i,j,k) and the level of orbit o, from
+// the tables
+HD void pn_zone_dg(const Params& P, const PnGrid& G, const PnOrbit& o, int i, int j, int k, double* dg) {
+  PnCoords<double> C;
+  pn_zone_coords(P, G, i, j, k, CENT, C);
+  pn_metric_dg_coords(G.B, o, C, G.tab[4 * P.n1t + 4 * (P.n2t + j) + 3], dg);
+}
 
 // FP32 geometry record of zone (i,j,k) at position pos and the level of orbit
 // o, evaluated in FP32 from the tables (for the FP32 face solve).  1 - alpha

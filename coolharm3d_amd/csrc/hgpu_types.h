@@ -182,8 +182,8 @@ struct PnBinary {
 };
 // Binary and grid of a context whose metric is the binary's; x0: startx.
 // tab: the coordinate functions at every zone's lower face (h = 0) and centre
-// (h = 1) along each direction, [2][N1T][2] (r, dr), then [2][N2T][3]
-// (sin theta, cos theta, dtheta/dX2), then [2][N3T][2] (sin phi, cos phi);
+// (h = 1) along each direction, [2][N1T][2] (r, dr), then [2][N2T][4]
+// (sin theta, cos theta, dtheta/dX2, d2theta/dX2^2), then [2][N3T][2] (sin phi, cos phi);
 // null: evaluate them.
 struct PnGrid {
   PnBinary B;
