@@ -83,6 +83,9 @@ HD void ks_record_rth(double a, double r, double th, Geom* G) {
   geom_finish(G);
 }
 
+// The record with its structure, for the solve
+typedef GeomView<GK_KS, const Geom*> KsView;
+
 // Sampling ranges of the batched inversion workload.
 constexpr double C2P_R_MIN = 1.3, C2P_R_MAX = 100., C2P_TH_PAD = 0.05;
 constexpr double C2P_GAMMA_MAX = 50.;
@@ -305,7 +308,8 @@ HD void c2p_start_learned(C2pCell& c, int rc_plain, const float* y);
 // plain_guess == 0), written with B from U and the plain guess's rho, u, u~ --
 // what the zone holds if no attempt succeeds.  Returns an early return code of
 // Utoprim_2d_fast() (-100, 2) or C2P_RUNNING.
-HD int c2p_begin(const double* U, const Geom* geom, double gam, double gmog, const float* mlp, int plain_guess,
+template <class GP>
+HD int c2p_begin(const double* U, GP geom, double gam, double gmog, const float* mlp, int plain_guess,
                  double* prim, C2pCell& c) {
   c.total = 0;
   c.attempt = 0;
@@ -333,7 +337,8 @@ HD int c2p_begin(const double* U, const Geom* geom, double gam, double gmog, con
 // C2P_RUNNING, with *rc_plain the plain guess's code; f may be null when the
 // outputs are already known); c2p_start_learned()
 // starts the Newton iteration from the network's outputs y.
-HD int c2p_prepare_learned(const double* U, const Geom* geom, double gam, double gmog, int plain_guess,
+template <class GP>
+HD int c2p_prepare_learned(const double* U, GP geom, double gam, double gmog, int plain_guess,
                            double* prim, C2pCell& c, int* rc_plain, float* f) {
   c.total = 0;
   c.attempt = 0;
@@ -367,7 +372,7 @@ HD int c2p_advance(C2pCell& c, double gam, int budget, double* prim, double* gam
     if (keep) continue;
     const int retval = u2d_newton_result(c.it);
     double bsq = 0.;
-    const int ret = u2d_finish(c.s, c.aux, gam, c.it.x, retval, prim, gamma, &bsq);
+    const int ret = u2d_finish<GK_KS>(c.s, c.aux, gam, c.it.x, retval, prim, gamma, &bsq);
     if (ret == 0 || !c.has_fallback || c.attempt == 1) return ret;
     c.attempt = 1;
     u2d_newton_init(c.it, c.x_plain);
@@ -378,6 +383,7 @@ HD int c2p_advance(C2pCell& c, double gam, int budget, double* prim, double* gam
 // Parked-zone record of the compaction queue: 19 doubles + 2 ints, stored
 // structure-of-arrays (field f of slot q at d[f*cap + q]).
 constexpr int C2P_QD = 19;
+static_assert(MAX_NEWT_ITER <= 32, "n_iter and stop have 5 bits each");
 struct C2pQueue {
   double* d;        // [C2P_QD][cap]
   int* cell;        // [cap]
@@ -398,8 +404,7 @@ HD void c2p_park(const C2pQueue& Q, long long q, int cell, const C2pCell& c) {
   d[15*K + q] = c.it.x[0]; d[16*K + q] = c.it.x[1];
   d[17*K + q] = c.x_plain[0]; d[18*K + q] = c.x_plain[1];
   Q.cell[q] = cell;
-  Q.meta[q] = c.it.n_iter | (c.it.i_extra << 6) | (c.it.doing_extra << 9) | (c.attempt << 10) |
-              (c.has_fallback << 11) | (c.total << 12);
+  Q.meta[q] = c.it.n_iter | (c.it.stop << 5) | (c.attempt << 10) | (c.has_fallback << 11) | (c.total << 12);
 }
 
 HD int c2p_unpark(const C2pQueue& Q, long long q, double gmog, C2pCell& c) {
@@ -418,14 +423,14 @@ HD int c2p_unpark(const C2pQueue& Q, long long q, double gmog, C2pCell& c) {
   c.it.x[0] = d[15*K + q]; c.it.x[1] = d[16*K + q];
   c.x_plain[0] = d[17*K + q]; c.x_plain[1] = d[18*K + q];
   const int m = Q.meta[q];
-  c.it.n_iter = m & 63;
-  c.it.i_extra = (m >> 6) & 7;
-  c.it.doing_extra = (m >> 9) & 1;
+  c.it.n_iter = m & 31;
+  c.it.stop = (m >> 5) & 31;
   c.it.n_extra = EXTRA_NEWT_ITER;
   c.attempt = (m >> 10) & 1;
   c.has_fallback = (m >> 11) & 1;
   c.total = m >> 12;
-  c.it.f = c.it.df = c.it.errx = 1.;   // recomputed by the next iteration before use
+  c.it.r0 = c.it.r1 = 1.;   // recomputed by the next iteration before use
+  c.it.conv = 0;
   return Q.cell[q];
 }
 
@@ -456,7 +461,7 @@ HD bool c2p_first_zone(const C2pArgs& A, const float* mlp, long long t, int budg
   Geom G;
   ks_record_rth(A.a, A.rth[t], A.rth[n + t], &G);
   double gm = 1.;
-  int rc = c2p_begin(u, &G, A.gam, A.gmog, mlp, A.plain_guess, pr, c);
+  int rc = c2p_begin(u, KsView{&G}, A.gam, A.gmog, mlp, A.plain_guess, pr, c);
   if (rc == C2P_RUNNING) rc = c2p_advance(c, A.gam, budget, pr, &gm);
   for (int l = 0; l < NP; l++) A.prim[l*n + t] = pr[l];
   if (rc == C2P_RUNNING) return true;

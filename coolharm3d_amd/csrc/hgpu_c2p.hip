@@ -114,10 +114,11 @@ constexpr int NL_SIZE = NL_TAIL + 3 * MLP_OUT;
 constexpr int NL_FEAT = MLP_IN + 1;             // padded feature row of one zone
 
 // gelu() with the hardware's single-instruction exp2 and reciprocal (about 1
-// ulp each), for the guess network's inference: x sigma(k (x + c x^3)).
+// ulp each), for the guess network's inference: x / (1 + exp2(x (c1 + c2 x^2)))
+// with c1 = -k log2(e), c2 = c c1.
 __device__ __forceinline__ float gelu_hw(float x) {
-  const float z = GELU_K * (x + GELU_C * x * x * x);
-  return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
+  constexpr float c1 = -1.4426950408889634f * GELU_K, c2 = c1 * GELU_C;
+  return x * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(x * fmaf(x * x, c2, c1)));
 }
 
 // Every thread of the workgroup: the parameters into LDS.
@@ -158,7 +159,8 @@ __device__ void mlp_forward_wave(const float* nl, const float* f, float* y, floa
   for (int mt = 0; mt < 4; mt++)
 #pragma unroll
     for (int nt = 0; nt < 4; nt++) {
-      mfma_f4 acc = {0.f, 0.f, 0.f, 0.f};
+      // the sum starts from the bias of the element's unit, 16 mt + 4 g + r
+      mfma_f4 acc = *reinterpret_cast<const mfma_f4*>(&nl[NL_B1 + 16 * mt + 4 * g]);
 #pragma unroll
       for (int s = 0; s < MLP_IN / 4; s++) {
         const float a = nl[NL_W1 + (4 * s + g) * MLP_H + 16 * mt + c];
@@ -166,7 +168,7 @@ __device__ void mlp_forward_wave(const float* nl, const float* f, float* y, floa
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
       }
 #pragma unroll
-      for (int r = 0; r < 4; r++) acc[r] = gelu_hw(acc[r] + nl[NL_B1 + 16 * mt + 4 * g + r]);
+      for (int r = 0; r < 4; r++) acc[r] = gelu_hw(acc[r]);
       h1[mt][nt] = acc;
     }
   float o0[4], o1[4];
@@ -176,7 +178,7 @@ __device__ void mlp_forward_wave(const float* nl, const float* f, float* y, floa
   for (int ot = 0; ot < 4; ot++) {
     mfma_f4 acc[4];
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) acc[nt] = (mfma_f4){0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < 4; nt++) acc[nt] = *reinterpret_cast<const mfma_f4*>(&nl[NL_B2 + 16 * ot + 4 * g]);
 #pragma unroll
     for (int mt = 0; mt < 4; mt++) {
       // W2^T[out 16 ot + c][in 16 mt + 4 g + r], r = 0..3: four consecutive floats
@@ -192,7 +194,7 @@ __device__ void mlp_forward_wave(const float* nl, const float* f, float* y, floa
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int u = 16 * ot + 4 * g + r;
-        const float h = gelu_hw(acc[nt][r] + nl[NL_B2 + u]);
+        const float h = gelu_hw(acc[nt][r]);
         o0[nt] = fmaf(h, nl[NL_W3 + u * MLP_OUT + 0], o0[nt]);
         o1[nt] = fmaf(h, nl[NL_W3 + u * MLP_OUT + 1], o1[nt]);
       }
@@ -233,7 +235,7 @@ __global__ __launch_bounds__(CB) void k_c2p_guess(C2pArgs A, const float* __rest
       ks_record_rth(A.a, A.rth[t], A.rth[n + t], &G);
       C2pCell c;
       int rc_plain = 0;
-      if (c2p_prepare_learned(u, &G, A.gam, A.gmog, A.plain_guess, pr, c, &rc_plain, f) != C2P_RUNNING)
+      if (c2p_prepare_learned(u, KsView{&G}, A.gam, A.gmog, A.plain_guess, pr, c, &rc_plain, f) != C2P_RUNNING)
         for (int i = 0; i < MLP_IN; i++) f[i] = 0.f;
     }
     mlp_forward_wave(nl, f, y, featbuf + (threadIdx.x >> 6) * 64 * NL_FEAT);
@@ -244,7 +246,13 @@ __global__ __launch_bounds__(CB) void k_c2p_guess(C2pArgs A, const float* __rest
   }
 }
 
-// First pass; with MLP the network's outputs come from k_c2p_guess.
+// First pass; with MLP the network's outputs come from k_c2p_guess.  Bound by
+// FP64 issue (2^24 zones move 2.6 GB in 1.30 ms; ~150 VALU instructions an
+// iteration, as many iterations as the wavefront's slowest zone): the
+// convergence test compares without dividing, one counter holds the stopping
+// rule, sin and cos share their reduction and the Kerr-Schild zeros are left out
+// (1.42 ms before).  At 4 wavefronts per SIMD (128 VGPRs) spills cost more than
+// they hide: 1.36 ms.
 template <bool MLP>
 __global__ __launch_bounds__(CB) void k_c2p_first(C2pArgs A, int budget, C2pQueue Q, unsigned* count) {
   const long long stride = (long long)gridDim.x * CB;
@@ -262,7 +270,7 @@ __global__ __launch_bounds__(CB) void k_c2p_first(C2pArgs A, int budget, C2pQueu
         Geom G;
         ks_record_rth(A.a, A.rth[t], A.rth[n + t], &G);
         int rc_plain = 0;
-        const int rc = c2p_prepare_learned(u, &G, A.gam, A.gmog, A.plain_guess, pr, c, &rc_plain, nullptr);
+        const int rc = c2p_prepare_learned(u, KsView{&G}, A.gam, A.gmog, A.plain_guess, pr, c, &rc_plain, nullptr);
         park = c2p_first_zone_finish(A, t, budget, rc, rc_plain, y, pr, c);
       } else {
         park = c2p_first_zone(A, nullptr, t, budget, c);
@@ -302,7 +310,7 @@ __global__ __launch_bounds__(CB) void k_mlp_features(long long n, double a, doub
   U2d s;
   U2dAux aux;
   float f[MLP_IN];
-  if (u2d_prepare(u, &G, (gam - 1.)/gam, pr, s, aux) == 0) mlp_features(s, f);
+  if (u2d_prepare(u, KsView{&G}, (gam - 1.)/gam, pr, s, aux) == 0) mlp_features(s, f);
   else for (int i = 0; i < MLP_IN; i++) f[i] = 0.f;
   for (int i = 0; i < MLP_IN; i++) feat[i*n + t] = f[i];
   if (prim && target) {

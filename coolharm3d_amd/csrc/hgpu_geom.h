@@ -76,8 +76,12 @@ inline void x_of_xp(const CoordParams& C, const double* xp, double* x, double J[
 
 // trigvalues(), src/metric.c:29-40 (COORDSINGFIX)
 HD void trigvalues(double th, double* cth, double* sth) {
+#ifdef __HIP_DEVICE_COMPILE__
+  sincos(th, sth, cth);   // one argument reduction for both
+#else
   *sth = sin(th);
   *cth = cos(th);
+#endif
   if (fabs(*sth) < 1.E-16) {
     if ((*sth) >= 0) *sth = 1.E-16;
     if ((*sth) < 0) *sth = -1.E-16;
@@ -120,8 +124,7 @@ HD void ks_metric_rth(double a, double M, double r, double th, double gcov[4][4]
     gcon[3][3] = t8/t14;
   }
   {
-    double cth, sth;
-    trigvalues(th, &cth, &sth);
+    const double cth = t4, sth = t12;
     double cos_2th = (cth - sth)*(cth + sth);
     double a2 = asq, r2 = r*r;
     *gdet = r2*fabs(sth)*(1. + 0.5*(a2/r2)*(1. + cos_2th));

@@ -321,7 +321,7 @@ HD double u2d_x1_of_x0(const U2d& s, double x0) {
   return (vsq > 1.) ? (1.0 - dv) : vsq;
 }
 
-HD void u2d_func_vsq(const U2d& s, const double* x, double* dx, double* f, double* df) {
+HD void u2d_func_vsq(const U2d& s, const double* x, double* dx, double* r0, double* r1) {
   double W = x[0], vsq = x[1];
   double ftmp = 1. - vsq;
   double gtmp = sqrt(ftmp);
@@ -342,9 +342,17 @@ HD void u2d_func_vsq(const U2d& s, const double* x, double* dx, double* f, doubl
   dx[0] = -(t2*t11 + t4*t18)*t21;
   double t40 = -2*(vsq + t24)*t3;
   dx[1] = -(-t25*t11 + t40*t18)*t21;
-  double r0 = t11, r1 = t18;
-  *df = -r0*r0 - r1*r1;
-  *f = -0.5 * (*df);
+  *r0 = t11;
+  *r1 = t18;
+}
+
+// |a|/|b| <= tol as the rounded quotient decides it, without the division
+// unless |a| lies within 2^-49 of tol |b| (the quotient and the product round by at
+// most 2^-53 each), tol |b| is too small for that, or something is not a number.
+HD bool ratio_within(double a, double b, double tol) {
+  const double p = tol*fabs(b), t = fabs(a) - p;
+  if (fabs(t) > 1.7763568394002505e-15*p + 1e-290) return t < 0.;
+  return fabs(a/b) <= tol;
 }
 
 // general_newton_raphson(), src/utoprim_2d_fast.c:489-592, as a resumable
@@ -353,44 +361,45 @@ HD void u2d_func_vsq(const U2d& s, const double* x, double* dx, double* f, doubl
 // cells; u2d_newton() runs it to completion.
 struct NewtonIter {
   double x[2];
-  double f, df, errx;
-  int n_iter, i_extra, doing_extra;
+  double r0, r1;           // residuals of the last iteration (f = (r0^2 + r1^2)/2, df = -2 f)
+  int conv;                // its step was within the tolerance (errx <= NEWT_TOL)
+  int n_iter;
+  int stop;      // index of the last iteration: MAX_NEWT_ITER - 1, or n_extra after the first converged one
   int n_extra;   // confirming iterations after convergence (EXTRA_NEWT_ITER)
 };
 
 HD void u2d_newton_init(NewtonIter& it, const double* x, int n_extra = EXTRA_NEWT_ITER) {
   it.x[0] = x[0]; it.x[1] = x[1];
-  it.f = 1.; it.df = 1.; it.errx = 1.;
-  it.n_iter = 0; it.i_extra = 0; it.doing_extra = 0;
+  it.r0 = it.r1 = 1.;
+  it.conv = 0;
+  it.n_iter = 0;
+  it.stop = MAX_NEWT_ITER - 1;
   it.n_extra = n_extra;
 }
 
 HD bool u2d_newton_step(const U2d& s, NewtonIter& it) {
   const double dv = (1. - 1.e-15);
   double dx[2], x_old[2];
-  u2d_func_vsq(s, it.x, dx, &it.f, &it.df);
-  it.errx = 0.;
+  u2d_func_vsq(s, it.x, dx, &it.r0, &it.r1);
   x_old[0] = it.x[0]; x_old[1] = it.x[1];
   it.x[0] += dx[0];
   it.x[1] += dx[1];
-  it.errx = (it.x[0] == 0.) ? fabs(dx[0]) : fabs(dx[0]/it.x[0]);
+  it.conv = (it.x[0] == 0.) ? (fabs(dx[0]) <= NEWT_TOL) : ratio_within(dx[0], it.x[0], NEWT_TOL);
   if (it.x[0] < 0.) { it.x[0] = fabs(it.x[0]); }
   else { if (it.x[0] > W_TOO_BIG) { it.x[0] = x_old[0]; } }
   if (it.x[1] < 0.) { it.x[1] = 0.; }
   else { if (it.x[1] > 1.) { it.x[1] = dv; } }
-  if ((fabs(it.errx) <= NEWT_TOL) && (it.doing_extra == 0) && (it.n_extra > 0)) it.doing_extra = 1;
-  if (it.doing_extra == 1) it.i_extra++;
-  bool keep = !(((fabs(it.errx) <= NEWT_TOL) && (it.doing_extra == 0)) || (it.i_extra > it.n_extra) ||
-                (it.n_iter >= (MAX_NEWT_ITER - 1)));
-  it.n_iter++;
-  return keep;
+  // the loop ends n_extra iterations after the first converged one (later ones
+  // would end it later), or at the iteration limit
+  if (it.conv && it.n_iter + it.n_extra < it.stop) it.stop = it.n_iter + it.n_extra;
+  return it.n_iter++ < it.stop;
 }
 
+// (MIN_NEWT_TOL equals NEWT_TOL, so the step's size decides once)
 HD int u2d_newton_result(const NewtonIter& it) {
-  if ((!is_finite(it.f)) || (!is_finite(it.df))) return 2;
-  if (fabs(it.errx) <= NEWT_TOL) return 0;
-  else if ((fabs(it.errx) <= MIN_NEWT_TOL) && (fabs(it.errx) > NEWT_TOL)) return 0;
-  return 1;
+  static_assert(MIN_NEWT_TOL == NEWT_TOL, "one tolerance");
+  if (!is_finite(-it.r0*it.r0 - it.r1*it.r1)) return 2;
+  return it.conv ? 0 : 1;
 }
 
 HD int u2d_newton(const U2d& s, double* x, int* iters, int n_extra = EXTRA_NEWT_ITER) {
