@@ -322,7 +322,7 @@ struct Api {
     rc |= dalloc(c, (void**)&X.slow_idx, sizeof(unsigned) * nint);
     rc |= dalloc(c, (void**)&X.pflag, sizeof(int) * NT);
     rc |= dalloc(c, (void**)&X.nfail, sizeof(int) * (P.track_nfail ? N_NFAIL * NT : 1));
-    rc |= dalloc(c, (void**)&X.status, sizeof(unsigned long long) * ST_WORDS);
+    rc |= dalloc(c, (void**)&X.status, sizeof(unsigned long long) * ST_ALLOC);
     rc |= dalloc(c, (void**)&X.scal, sizeof(double) * SC_WORDS);
     // at most n1 (n2 n3 / 64 + n2 + n3 + 2) + 8 workgroups of at most 4
     // wavefronts over the interior, for any tile of 64 to 256 threads
@@ -363,7 +363,7 @@ struct Api {
     rc |= BE::zero(c, X.gamma, sizeof(double) * NT);
     rc |= BE::zero(c, X.pflag, sizeof(int) * NT);
     rc |= BE::zero(c, X.nfail, sizeof(int) * (P.track_nfail ? N_NFAIL * NT : 1));
-    rc |= BE::zero(c, X.status, sizeof(unsigned long long) * ST_WORDS);
+    rc |= BE::zero(c, X.status, sizeof(unsigned long long) * ST_ALLOC);
     double sc[SC_WORDS] = {0};
     sc[SC_T] = cfg->startx[0];
     sc[SC_DT] = cfg->dx[0];

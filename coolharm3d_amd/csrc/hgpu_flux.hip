@@ -17,7 +17,8 @@ __global__ __launch_bounds__(BLOCK, W) void k_flux(Params P, Ptrs X, const doubl
     flux_face<D, K>(P, X, src, i, j, k, fr);
     c = cidx(P, i, j, k);
   }
-  commit_fail(P, X, fr, active, c, MASK_GAMMA, D + 1);
+  if (P.track_nfail && active && fr.nf[NFAIL_GAMMA_CALC]) X.nfail[NFAIL_GAMMA_CALC*P.nt + c] += fr.nf[NFAIL_GAMMA_CALC];
+  commit_flux(X, fr, active, D + 1);
 }
 
 template <int D, int W, int K>
@@ -31,7 +32,8 @@ __global__ __launch_bounds__(BLOCK, W) void k_flux_mixed(Params P, Ptrs X, const
     flux_face_mixed<D, K>(P, X, src, i, j, k, fr);
     c = cidx(P, i, j, k);
   }
-  commit_fail(P, X, fr, active, c, MASK_GAMMA, D + 1);
+  if (P.track_nfail && active && fr.nf[NFAIL_GAMMA_CALC]) X.nfail[NFAIL_GAMMA_CALC*P.nt + c] += fr.nf[NFAIL_GAMMA_CALC];
+  commit_flux(X, fr, active, D + 1);
 }
 
 __device__ __forceinline__ long long wave_min_ll(long long v) {
@@ -47,6 +49,16 @@ __device__ __forceinline__ long long wave_max_ll(long long v) {
     v = (o > v) ? o : v;
   }
   return v;
+}
+
+// Orders LDS accesses of a wavefront to a buffer of its own: its LDS operations
+// complete in order, so a wavefront-scope fence (no workgroup barrier) puts
+// one lane's stores before the other lanes' reads, and those before the next
+// stores.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // LDS capacity (doubles) of one primitive's x3 pencil of a wavefront: 64 face
@@ -110,12 +122,7 @@ __device__ void ppm_faces_x3_staged(const Params& P, const Ptrs& X, const double
         }
       }
     }
-    // the wavefront's own buffer: LDS operations of one wavefront complete in
-    // order, so a wavefront-scope fence (no workgroup barrier) orders the
-    // stores before the other lanes' reads
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_order();
     if (active) {
       const int s = rs_slot(v);
       const double ra = X.rscale[s * P.n1t + ii], ri = X.irscale[s * P.n1t + ii];
@@ -229,16 +236,16 @@ __device__ __forceinline__ void flux_multi_block(const Params& P, const Ptrs& X,
 #pragma unroll
     for (int l = 0; l < NP; l++) {
       if (l == B3) continue;   // the normal field's flux: never read
-      __syncthreads();
+      wave_lds_order();
 #pragma unroll
       for (int f = 0; f < F; f++) wbuf[lane*F + f] = fo[f][l];
-      __syncthreads();
+      wave_lds_order();
 #pragma unroll
       for (int s = 0; s < F; s++)
         if (ok[s]) Fa[(2*NFLUX + l)*(long long)P.nt + cs[s]] = wbuf[s*64 + lane];
     }
   }
-  commit_fail(P, X, fr, active, 0, MASK_GAMMA, D + 1, false);
+  commit_flux(X, fr, active, D + 1);
 }
 
 template <int D, int F, int W, bool MIXED, int K, bool OTF = false, bool STG = false>
@@ -340,7 +347,8 @@ __device__ __forceinline__ void flux_one_block(const Params& P, const Ptrs& X, c
     else flux_face<D, K>(P, X, src, i, j, k, fr);
     c = cidx(P, i, j, k);
   }
-  commit_fail(P, X, fr, active, c, MASK_GAMMA, D + 1);
+  if (P.track_nfail && active && fr.nf[NFAIL_GAMMA_CALC]) X.nfail[NFAIL_GAMMA_CALC*P.nt + c] += fr.nf[NFAIL_GAMMA_CALC];
+  commit_flux(X, fr, active, D + 1);
 }
 template <int W, bool MIXED, int K>
 __global__ __launch_bounds__(BLOCK, W) void k_flux_all_one(Params P, Ptrs X, const double* __restrict__ src,

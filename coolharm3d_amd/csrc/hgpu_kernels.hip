@@ -43,14 +43,14 @@ __global__ __launch_bounds__(64) void k_orbit(Ptrs X, PnBinary B, PnOrbit* out) 
 }
 
 __global__ __launch_bounds__(BLOCK) void k_emf(Params P, Ptrs X, Box b, Tiling T) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) X.status[ST_PFDIRTY] = 0;   // k_begin_stage has used it
+  if (blockIdx.x == T.nblocks) { fold_flux_words(X); return; }   // a workgroup of its own, beside the edges'
   int i, j, k;
   if (!tile_index(b, T, i, j, k)) return;
   emf_edge(P, X, i, j, k);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_emf_mixed(Params P, Ptrs X, Box b, Tiling T) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) X.status[ST_PFDIRTY] = 0;
+  if (blockIdx.x == T.nblocks) { fold_flux_words(X); return; }
   int i, j, k;
   if (!tile_index(b, T, i, j, k)) return;
   emf_edge_mixed(P, X, i, j, k);
@@ -416,6 +416,7 @@ __global__ __launch_bounds__(BLOCK) void k_begin_stage(Ptrs X, long long nt) {
       X.status[ST_SLOW] = 0;
     }
     if (threadIdx.x < 4) X.status[ST_VMAX + threadIdx.x] = 0;
+    for (int w = threadIdx.x; w < VS_LINE * N_VSLOT; w += BLOCK) X.status[VS_FIRST + w] = 0;
   }
   if (!X.status[ST_PFDIRTY]) return;
   const long long stride = (long long)gridDim.x * BLOCK;
@@ -1094,8 +1095,8 @@ struct GpuBE {
     Box b = edge_box(c->P);
     Scope s(c, "emf");
     const Tiling T = make_tiling(b, priv(c)->shape[FAM_EMF]);
-    if (c->P.mixed) hipLaunchKernelGGL(k_emf_mixed, dim3(T.nblocks), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
-    else hipLaunchKernelGGL(k_emf, dim3(T.nblocks), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
+    if (c->P.mixed) hipLaunchKernelGGL(k_emf_mixed, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
+    else hipLaunchKernelGGL(k_emf, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
     return hip_check(hipGetLastError(), "k_emf");
   }
   // reset_slow: empty the slow-zone queue first (the stage's update finds it

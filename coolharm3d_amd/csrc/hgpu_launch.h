@@ -40,26 +40,23 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
 }
 
 // Writes the fail() tallies of a workgroup: per-zone nfail, and block totals of
-// nfailtot, the failure words and the fastest face speed (vmax_slot >= 0),
-// reduced in LDS so each status word receives at most one atomic per
-// workgroup.  Every thread of the block must call it.
+// nfailtot and the failure words, reduced in LDS so each status word receives
+// at most one atomic per workgroup.  Every thread of the block must call it.
 __device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, const FailRec& fr,
-                                            bool active, long long c, unsigned mask, int vmax_slot = -1,
-                                            bool zone_map = true) {
+                                            bool active, long long c, unsigned mask) {
   __shared__ unsigned s_cnt[N_NFAIL];
   __shared__ unsigned s_flags;
-  __shared__ unsigned long long s_vmax;
   const long long NT = P.nt;
   const int tid = threadIdx.x;
   if (tid < N_NFAIL) s_cnt[tid] = 0;
-  if (tid == 0) { s_flags = 0; s_vmax = 0; }
+  if (tid == 0) s_flags = 0;
   __syncthreads();
   if (active) {
     for (int l = 0; l < N_NFAIL; l++) {
       if (!(mask & (1u << l))) continue;
       const int v = fr.nf[l];
       if (v) {
-        if (P.track_nfail && zone_map) X.nfail[l*NT + c] += v;
+        if (P.track_nfail) X.nfail[l*NT + c] += v;
         atomicAdd(&s_cnt[l], (unsigned)v);
       }
     }
@@ -68,10 +65,6 @@ __device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, cons
                    ((fr.boundary & 2) ? 16u : 0u);
       atomicOr(&s_flags, f);
     }
-  }
-  if (vmax_slot >= 0) {
-    const unsigned long long m = wave_max_u64(active ? dbl_bits(fr.vmax) : 0ull);
-    if ((tid & 63) == 0 && m) atomicMax(&s_vmax, m);
   }
   __syncthreads();
   if (tid < N_NFAIL && s_cnt[tid]) atomicAdd(&X.status[ST_NFAILTOT + tid], (unsigned long long)s_cnt[tid]);
@@ -85,7 +78,36 @@ __device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, cons
       if (f & 8u) atomicOr(&X.status[ST_BOUNDARY_PHYS], 1ull);
       if (f & 16u) atomicOr(&X.status[ST_BOUNDARY_MPI], 1ull);
     }
-    if (vmax_slot >= 0 && s_vmax) atomicMax(&X.status[ST_VMAX + vmax_slot], s_vmax);
+  }
+}
+
+// The face fluxes' tallies, wavefront by wavefront without a barrier: the
+// GAMMA_CALC failures (rare) and the fastest face speed, into the workgroup's line.
+__device__ __forceinline__ void commit_flux(const Ptrs& X, const FailRec& fr, bool active, int vmax_slot) {
+  const int v = active ? fr.nf[NFAIL_GAMMA_CALC] : 0;
+  const bool first = (threadIdx.x & 63) == 0;
+  if (__ballot(v != 0)) {
+    const int n = wave_sum(v);
+    if (first) atomicAdd(&X.status[ST_NFAILTOT + NFAIL_GAMMA_CALC], (unsigned long long)n);
+  }
+  const unsigned long long m = wave_max_u64(active ? dbl_bits(fr.vmax) : 0ull);
+  if (first && m) atomicMax(&X.status[VS_FIRST + VS_LINE * (blockIdx.x & (N_VSLOT - 1)) + vmax_slot], m);
+}
+
+// ST_VMAX of the stage from the workgroups' lines, by one wavefront; the
+// failure words' dirty mark goes down here too, after k_begin_stage's use.
+__device__ __forceinline__ void fold_flux_words(const Ptrs& X) {
+  if (threadIdx.x >= 64) return;
+  unsigned long long m[3] = {0, 0, 0};
+  for (int s = threadIdx.x; s < N_VSLOT; s += 64)
+    for (int d = 0; d < 3; d++) {
+      const unsigned long long o = X.status[VS_FIRST + VS_LINE * s + 1 + d];
+      m[d] = o > m[d] ? o : m[d];
+    }
+  for (int d = 0; d < 3; d++) m[d] = wave_max_u64(m[d]);
+  if (threadIdx.x == 0) {
+    for (int d = 0; d < 3; d++) X.status[ST_VMAX + 1 + d] = m[d];
+    X.status[ST_PFDIRTY] = 0;
   }
 }
 

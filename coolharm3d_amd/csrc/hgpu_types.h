@@ -127,7 +127,14 @@ enum {
   ST_MPARTS = 30,            // M_tot parts of the last update (one per wavefront)
   ST_MPARTS2 = 31,           // their second-level parts (one per k_recover workgroup)
   ST_PFDIRTY = 32,           // a flagged zone since the flag map was last cleared
-  ST_WORDS = 33
+  ST_WORDS = 33,
+  // Behind the words, the fastest face speeds of the stage's workgroups, one
+  // 128-byte line for every N_VSLOT-th workgroup (words 1..3: the directions):
+  // atomics on one address take about 8 ns each whoever issues them, so one
+  // word for all of them bounded the kernel.  k_begin_stage clears the lines,
+  // k_emf takes their maximum into ST_VMAX.
+  VS_FIRST = 48, VS_LINE = 16, N_VSLOT = 128,
+  ST_ALLOC = VS_FIRST + VS_LINE * N_VSLOT
 };
 
 // Device scalars of the integrator (t, dt ... of src/globals.h:380-390).
