@@ -271,14 +271,19 @@ struct FluxAll {
   unsigned per, nblocks;     // workgroups per slab, in all
   unsigned remap;            // XCD-contiguous slabs
 };
-static FluxAll make_flux_all(const Params& P, unsigned F, const LaunchShape& L) {
+static FluxAll make_flux_all(const Params& P, unsigned F, LaunchShape& L) {
   FluxAll A;
+  long long points = 0;
   bool small = false;
   for (int d = 0; d < 3; d++) {
     const Box b = flux_box(P, d);
     A.bg[d] = b;
     A.hi[d] = b.hi[d];
     A.bg[d].hi[d] = b.lo[d] + (b.hi[d] - b.lo[d] + (int)F) / (int)F - 1;
+    points += A.bg[d].count();
+  }
+  L = spread_shape(L, A.bg[0], points);
+  for (int d = 0; d < 3; d++) {
     A.T[d] = make_tiling(A.bg[d], L);
     small = small || A.T[d].pp > 1;
   }
@@ -358,13 +363,13 @@ __global__ __launch_bounds__(BLOCK, W) void k_flux_all_one(Params P, Ptrs X, con
   if (!flux_all_slot(A, d, ii, t)) return;
   int i = 0, j = 0, k = 0;
   if (d == 0) {
-    const bool active = tile_point(A.bg[0], A.T[0], ii, t, i, j, k);
+    const bool active = tile_point<true>(A.bg[0], A.T[0], ii, t, i, j, k);
     flux_one_block<0, MIXED, K>(P, X, src, active, i, j, k);
   } else if (d == 1) {
-    const bool active = tile_point(A.bg[1], A.T[1], ii, t, i, j, k);
+    const bool active = tile_point<true>(A.bg[1], A.T[1], ii, t, i, j, k);
     flux_one_block<1, MIXED, K>(P, X, src, active, i, j, k);
   } else {
-    const bool active = tile_point(A.bg[2], A.T[2], ii, t, i, j, k);
+    const bool active = tile_point<true>(A.bg[2], A.T[2], ii, t, i, j, k);
     flux_one_block<2, MIXED, K>(P, X, src, active, i, j, k);
   }
 }
@@ -464,6 +469,7 @@ void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStrea
   LaunchShape L;
   L.remap = 0;
   const bool multi = flux_all_multi(P);
+  L.spread = !multi;
   const FluxAll A = make_flux_all(P, multi ? 2u : 1u, L);
   const dim3 grid(A.nblocks), blk(L.bs);
   if (multi) {

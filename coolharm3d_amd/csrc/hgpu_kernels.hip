@@ -45,14 +45,14 @@ __global__ __launch_bounds__(64) void k_orbit(Ptrs X, PnBinary B, PnOrbit* out) 
 __global__ __launch_bounds__(BLOCK) void k_emf(Params P, Ptrs X, Box b, Tiling T) {
   if (blockIdx.x == T.nblocks) { fold_flux_words(X); return; }   // a workgroup of its own, beside the edges'
   int i, j, k;
-  if (!tile_index(b, T, i, j, k)) return;
+  if (!tile_index<true>(b, T, i, j, k)) return;
   emf_edge(P, X, i, j, k);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_emf_mixed(Params P, Ptrs X, Box b, Tiling T) {
   if (blockIdx.x == T.nblocks) { fold_flux_words(X); return; }
   int i, j, k;
-  if (!tile_index(b, T, i, j, k)) return;
+  if (!tile_index<true>(b, T, i, j, k)) return;
   emf_edge_mixed(P, X, i, j, k);
 }
 
@@ -202,7 +202,7 @@ template <bool MIXED, int W, bool OTF = false, int MET = 0, bool UNI = false, in
 __global__ __launch_bounds__(BLOCK, W) void k_update(Params P, Ptrs X, int stage, Box b, Tiling T, PnGrid G,
                                                      int lvl) {
   int i, j, k;
-  const bool active = tile_index(b, T, i, j, k);
+  const bool active = tile_index<true>(b, T, i, j, k);
   FailRec fr; fr.clear();
   long long c = 0;
   bool queue = false;
@@ -615,6 +615,7 @@ struct GpuBE {
     g->shape[FAM_FLUX2].occ = 1;
     g->shape[FAM_FLUX2].remap = 1;
     g->shape[FAM_EMF].order = mixed ? 1u : 0u;
+    g->shape[FAM_EMF].spread = g->shape[FAM_CONS].spread = 1;
     g->shape[FAM_CONS].fused = 1;
     g->shape[FAM_CONS].remap = 0;
     g->shape[FAM_CONS].occ = 1;
@@ -1094,7 +1095,7 @@ struct GpuBE {
   static int emf(hgpu_ctx* c) {
     Box b = edge_box(c->P);
     Scope s(c, "emf");
-    const Tiling T = make_tiling(b, priv(c)->shape[FAM_EMF]);
+    const Tiling T = make_tiling(b, spread_shape(priv(c)->shape[FAM_EMF], b, b.count()));
     if (c->P.mixed) hipLaunchKernelGGL(k_emf_mixed, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
     else hipLaunchKernelGGL(k_emf, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
     return hip_check(hipGetLastError(), "k_emf");
@@ -1112,7 +1113,9 @@ struct GpuBE {
     }
     Box b = interior_box(c->P);
     Scope s(c, "update");
-    const Tiling T = make_tiling(b, priv(c)->shape[FAM_CONS]);
+    LaunchShape L = priv(c)->shape[FAM_CONS];
+    if (L.fused || c->P.otf) L = spread_shape(L, b, b.count());
+    const Tiling T = make_tiling(b, L);
     const Tiling T2 = make_tiling(b, priv(c)->shape[FAM_INV]);
     if ((long long)T.nblocks * (T.bs / 64) > c->mpart_cap) return set_error(-3, "update grid exceeds the M_tot parts buffer");
     if (reset_slow) hipLaunchKernelGGL(k_reset_words, dim3(1), dim3(64), 0, priv(c)->stream, c->X, (int)ST_SLOW, 1);

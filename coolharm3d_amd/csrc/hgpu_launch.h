@@ -21,6 +21,8 @@ struct LaunchShape {
   unsigned fused = 0;    // conserved update only: 1 = update and inversion in one kernel
   unsigned fpt = 1;      // face fluxes only: faces per thread along the direction (1, 2, 4)
   unsigned stage = 0;    // x3 face fluxes (FP64, PPM, fpt > 1): reconstruction from LDS-staged pencils
+  unsigned spread = 0;   // 1: small grids are spread over more wavefronts (spread_shape)
+  unsigned sp = 0;       // only the first 64 >> sp lanes of a wavefront take a point
 };
 enum { FAM_FLUX1 = 0, FAM_FLUX2, FAM_FLUX3, FAM_EMF, FAM_CONS, FAM_INV, N_FAM };
 
@@ -124,7 +126,8 @@ __device__ __forceinline__ void fold_flux_words(const Ptrs& X) {
 // (or set by the caller).
 struct Tiling {
   unsigned ni, nj, nk;  // box extents (ni: rows of tiles, i.e. x1-planes, or groups of pp of them)
-  unsigned bs, kc, jr;  // tile: kc x jr (kc > 0) or bs consecutive points (kc = 0)
+  unsigned bs, kc, jr;  // threads; tile: kc x jr (kc > 0) or bs >> sp consecutive points (kc = 0)
+  unsigned sp;          // only the first 64 >> sp lanes of a wavefront take a point
   unsigned nkt;         // tiles along k (2D tiles)
   unsigned pp, np;      // x1-planes per flat tile (small planes), x1-planes in all
   unsigned X;           // tiles per plane
@@ -133,6 +136,24 @@ struct Tiling {
   unsigned order;
 };
 
+// Small grids whose rows along x3 are shorter than a cache line (1D grids, 2D
+// ones in x1 and x2): the 64 lanes of a wavefront touch a line each with every
+// load, about 60 loads one after the other on one compute unit, and most compute
+// units have no wavefront at all.  Workgroups of one wavefront with 64 >> sp
+// points each spread them, as long as that makes no more than SPREAD_WAVES
+// wavefronts.  1024-zone shock tube: update 21 -> 10 us a launch, step 0.097 ->
+// 0.074 ms (0.075 up to 1024 wavefronts, 0.081 up to 2048, where the dispatch of
+// the workgroups takes over).  Longer rows share their lines between lanes and lose:
+// 24x24x16, spread twofold 0.170 -> 0.172 ms, fourfold 0.187.
+constexpr long long SPREAD_WAVES = 512;
+static inline LaunchShape spread_shape(LaunchShape L, const Box& b, long long points) {
+  if (!L.spread || L.kc || b.hi[2] - b.lo[2] + 1 >= 8) return L;
+  const long long waves = (points + 63) / 64;
+  while (L.sp < 4 && (waves << (L.sp + 1)) <= SPREAD_WAVES) L.sp++;
+  if (L.sp) L.bs = 64;
+  return L;
+}
+
 static inline Tiling make_tiling(const Box& b, const LaunchShape& L = LaunchShape()) {
   Tiling T;
   T.nk = (unsigned)(b.hi[2] - b.lo[2] + 1);
@@ -140,9 +161,11 @@ static inline Tiling make_tiling(const Box& b, const LaunchShape& L = LaunchShap
   T.ni = T.np = (unsigned)(b.hi[0] - b.lo[0] + 1);
   T.pp = 1;
   T.bs = L.bs;
+  T.sp = L.sp;
+  const unsigned pts = L.bs >> L.sp;
   T.remap = L.remap;
   T.order = L.order;
-  if (L.kc > 0 && L.kc < T.nk && L.bs % L.kc == 0) {
+  if (L.kc > 0 && L.kc < T.nk && L.bs % L.kc == 0 && L.sp == 0) {
     T.kc = L.kc;
     T.jr = L.bs / L.kc;
     T.nkt = (T.nk + T.kc - 1) / T.kc;
@@ -151,10 +174,10 @@ static inline Tiling make_tiling(const Box& b, const LaunchShape& L = LaunchShap
     T.kc = 0;
     T.jr = 0;
     T.nkt = 0;
-    T.X = (T.nj * T.nk + T.bs - 1) / T.bs;
+    T.X = (T.nj * T.nk + pts - 1) / pts;
     // planes smaller than a tile: several to a tile (a 1D grid's planes hold a
     // handful of points, and a workgroup per plane left 250 of 256 threads idle)
-    T.pp = std::max(1u, T.bs / (T.nj * T.nk));
+    T.pp = std::max(1u, pts / (T.nj * T.nk));
     T.ni = (T.np + T.pp - 1) / T.pp;
   }
   T.nblocks = T.X * T.ni;
@@ -162,18 +185,25 @@ static inline Tiling make_tiling(const Box& b, const LaunchShape& L = LaunchShap
   return T;
 }
 
-// point (i, j, k) of this thread in tile t of tile row ii
+// point (i, j, k) of this thread in tile t of tile row ii.  SP: the kernel may be
+// launched with spread tiles.
+template <bool SP = false>
 __device__ __forceinline__ bool tile_point(const Box& b, const Tiling& T, unsigned ii, unsigned t, int& i, int& j,
                                            int& k) {
-  unsigned jj, kk;
+  unsigned jj, kk, r0 = threadIdx.x;
+  if (SP && T.sp) {
+    const unsigned lanes = 64u >> T.sp, lane = r0 & 63u;
+    if (lane >= lanes) return false;
+    r0 = (r0 >> 6) * lanes + lane;
+  }
   if (T.pp > 1) {        // X = 1
-    const unsigned np = T.nj * T.nk, di = threadIdx.x / np, q = threadIdx.x - di * np;
+    const unsigned np = T.nj * T.nk, di = r0 / np, q = r0 - di * np;
     ii = ii * T.pp + di;
     if (di >= T.pp || ii >= T.np) return false;
     jj = q / T.nk;
     kk = q - jj * T.nk;
   } else if (T.kc == 0) {
-    const unsigned q = t * T.bs + threadIdx.x;
+    const unsigned q = t * (SP ? T.bs >> T.sp : T.bs) + r0;
     jj = q / T.nk;
     kk = q - jj * T.nk;
     if (jj >= T.nj) return false;
@@ -191,6 +221,7 @@ __device__ __forceinline__ bool tile_point(const Box& b, const Tiling& T, unsign
   return true;
 }
 
+template <bool SP = false>
 __device__ __forceinline__ bool tile_index(const Box& b, const Tiling& T, int& i, int& j, int& k) {
   const unsigned p = blockIdx.x;
   const unsigned L = T.remap ? (p & 7u) * (T.nblocks >> 3) + (p >> 3) : p;
@@ -204,7 +235,7 @@ __device__ __forceinline__ bool tile_index(const Box& b, const Tiling& T, int& i
     if (t >= T.X) return false;
   }
   if (ii >= T.ni) return false;
-  return tile_point(b, T, ii, t, i, j, k);
+  return tile_point<SP>(b, T, ii, t, i, j, k);
 }
 
 constexpr unsigned MASK_GAMMA = 1u << NFAIL_GAMMA_CALC;
