@@ -44,6 +44,11 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
 // Writes the fail() tallies of a workgroup: per-zone nfail, and block totals of
 // nfailtot and the failure words, reduced in LDS so each status word receives
 // at most one atomic per workgroup.  Every thread of the block must call it.
+// The LDS addresses carry a zero that the compiler cannot see through: it turns
+// atomics of a wavefront on one address into a loop over its lanes on the
+// scalar unit (most zones count USE_FULL_INV), the LDS unit adds them faster.
+// Corrector update of 24x24x16: 0.9 us of 13; k_recover on the 192x192x128 torus
+// 68 -> 65 us.
 __device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, const FailRec& fr,
                                             bool active, long long c, unsigned mask) {
   __shared__ unsigned s_cnt[N_NFAIL];
@@ -54,18 +59,20 @@ __device__ __forceinline__ void commit_fail(const Params& P, const Ptrs& X, cons
   if (tid == 0) s_flags = 0;
   __syncthreads();
   if (active) {
+    unsigned z;
+    asm("v_mov_b32 %0, 0" : "=v"(z));
     for (int l = 0; l < N_NFAIL; l++) {
       if (!(mask & (1u << l))) continue;
       const int v = fr.nf[l];
       if (v) {
         if (P.track_nfail) X.nfail[l*NT + c] += v;
-        atomicAdd(&s_cnt[l], (unsigned)v);
+        atomicAdd(&s_cnt[l + z], (unsigned)v);
       }
     }
     if (fr.pflag) {
       unsigned f = 1u | ((fr.pflag == PFLAG_INTERP_PRIM) ? 2u : 4u) | ((fr.boundary & 1) ? 8u : 0u) |
                    ((fr.boundary & 2) ? 16u : 0u);
-      atomicOr(&s_flags, f);
+      atomicOr(&s_flags + z, f);
     }
   }
   __syncthreads();
