@@ -59,8 +59,7 @@ HD void flux_recon(const Params& P, const Ptrs& X, const double* __restrict__ sr
     if (P.degen[1]) jj = NG;
     if (P.degen[2]) kk = NG;
     // every primitive's stencil is loaded before any limiter runs, so their
-    // loads are in flight together (their branches keep the compiler from
-    // moving loads across them)
+    // loads are in flight together
     if (P.recon == RECON_PPM_MC) {
       const long long c0 = cidx(P, ii - 3*di, jj - 3*dj, kk - 3*dk);
       const long long st = cidx(P, di, dj, dk) - cidx(P, 0, 0, 0);
@@ -288,6 +287,8 @@ HD void flux_face(const Params& P, const Ptrs& X, const double* __restrict__ src
 // --------------------------------------------------------------------------
 // Corner EMFs, flux_ct_para_fast2() (src/flux_ct.c:759-846) or flux_ct()
 // (src/flux_ct.c:26-41) for the edge (i,j,k).
+// BR: the limiters by branches.
+template <bool BR = false>
 HD void emf_edge(const Params& P, const Ptrs& X, int i, int j, int k) {
   const long long NT = P.nt;
   const long long c = cidx(P, i, j, k);
@@ -313,8 +314,9 @@ HD void emf_edge(const Params& P, const Ptrs& X, int i, int j, int k) {
     for (int l = 0; l < 6; l++)
 #pragma unroll
       for (int m = 0; m < 6; m++) y[l][m] = line[l][c + (m - 3)*str[l]];
+    loads_issued();
 #pragma unroll
-    for (int l = 0; l < 6; l++) ppm_interface(y[l], &yl[l], &yr[l]);
+    for (int l = 0; l < 6; l++) ppm_interface<BR>(y[l], &yl[l], &yr[l]);
     e0 = (((0.0 + yl[0]) + yr[0]) - yl[1]) - yr[1];
     e1 = (((0.0 + yl[2]) + yr[2]) - yl[3]) - yr[3];
     e2 = (((0.0 + yl[4]) + yr[4]) - yl[5]) - yr[5];

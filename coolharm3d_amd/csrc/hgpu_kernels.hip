@@ -14,6 +14,7 @@ struct ProfEvent { std::string name; hipEvent_t a, b; };
 
 struct GpuPriv {
   hipStream_t stream = nullptr;
+  unsigned simds = 1024;               // SIMDs of the device
   unsigned flag_grid = 1024;           // workgroups of the kernels that mostly find nothing to do
   bool prof = false;
   bool graph = false;                  // replay captured steps
@@ -42,11 +43,12 @@ __global__ __launch_bounds__(64) void k_orbit(Ptrs X, PnBinary B, PnOrbit* out) 
   if (l < 3) pn_orbit_at(B, level_time(X, l), &out[l]);
 }
 
+template <bool BR>
 __global__ __launch_bounds__(BLOCK) void k_emf(Params P, Ptrs X, Box b, Tiling T) {
   if (blockIdx.x == T.nblocks) { fold_flux_words(X); return; }   // a workgroup of its own, beside the edges'
   int i, j, k;
   if (!tile_index<true>(b, T, i, j, k)) return;
-  emf_edge(P, X, i, j, k);
+  emf_edge<BR>(P, X, i, j, k);
 }
 
 __global__ __launch_bounds__(BLOCK) void k_emf_mixed(Params P, Ptrs X, Box b, Tiling T) {
@@ -627,7 +629,7 @@ struct GpuBE {
       int dev = 0, cus = 0;
       if (hipGetDevice(&dev) == hipSuccess &&
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
-        g->flag_grid = 4u * (unsigned)cus;
+        g->flag_grid = g->simds = 4u * (unsigned)cus;
     }
     return hip_check(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking), "hipStreamCreate");
   }
@@ -1097,7 +1099,12 @@ struct GpuBE {
     Scope s(c, "emf");
     const Tiling T = make_tiling(b, spread_shape(priv(c)->shape[FAM_EMF], b, b.count()));
     if (c->P.mixed) hipLaunchKernelGGL(k_emf_mixed, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
-    else hipLaunchKernelGGL(k_emf, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
+    // The limiters' form: as long as the edges are one round of wavefronts (5 per
+    // SIMD) the launch is one wavefront's chain, shorter by selects (24x24x16: 7.0
+    // us against 8.6); from there on the issue of the sides that branches skip
+    // counts (192x192x128: 137 us by branches, 143 by selects).
+    else if (b.count() <= 64ll * 5 * priv(c)->simds) hipLaunchKernelGGL(k_emf<false>, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
+    else hipLaunchKernelGGL(k_emf<true>, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
     return hip_check(hipGetLastError(), "k_emf");
   }
   // reset_slow: empty the slow-zone queue first (the stage's update finds it

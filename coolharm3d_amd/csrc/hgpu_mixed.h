@@ -215,28 +215,26 @@ HD void vchar_f(const StateF* q, GP g, float gam, float* vmax, float* vmin) {
 // Reconstruction on differences.  D[m] = y[m+1] - y[m].
 
 // MC slope of the middle point from its two one-sided differences
-// (linear_recon_vect(), src/recon.c:237-264)
+// (linear_recon_vect(), src/recon.c:237-264), by selects as mc_slope_sel()
 HD float mc_slope_diff(float a, float b) {
-  if (a*b <= 0.f) return 0.f;
   const float aa = fabsf(a), ab = fabsf(b);
-  if (aa + aa + aa <= ab) return a + a;
-  if (ab + ab + ab <= aa) return b + b;
-  return 0.5f*(a + b);
+  float r = 0.5f*(a + b);
+  r = (ab + ab + ab <= aa) ? b + b : r;
+  r = (aa + aa + aa <= ab) ? a + a : r;
+  return (a*b <= 0.f) ? 0.f : r;
 }
 
 // para_vect() limiter (src/recon.c:611-641) on edge values l, r taken
 // relative to the zone value
 HD void ppm_limit_rel(float l, float r, float* lnew, float* rnew) {
-  if (-r*l <= 0.f) { *lnew = *rnew = 0.f; return; }
   const float r2 = r + r, l2 = l + l;
-  *lnew = l; *rnew = r;
-  if (r > l) {
-    if (0.f > (l + r2)) *lnew = -r2;
-    if (0.f < (l2 + r)) *rnew = -l2;
-  } else {
-    if (0.f < (l + r2)) *lnew = -r2;
-    if (0.f > (l2 + r)) *rnew = -l2;
-  }
+  const float sl = l + r2, sr = l2 + r;
+  const bool up = r > l;
+  const bool cl = (up & (0.f > sl)) | (!up & (0.f < sl)), cr = (up & (0.f < sr)) | (!up & (0.f > sr));
+  const bool flat = -r*l <= 0.f;
+  const float ln = cl ? -r2 : l, rn = cr ? -l2 : r;
+  *lnew = flat ? 0.f : ln;
+  *rnew = flat ? 0.f : rn;
 }
 
 // PPM+MC states at the interface between points 2 and 3 of a 6-point window,
@@ -255,11 +253,11 @@ HD void ppm_offsets(const float* D, float* o2, float* o3) {
 // linear_recon() MC limiter (src/recon.c:88-132) on the differences a = y2-y1, b = y3-y2
 HD float mc_linear_diff(float a, float b) {
   const float Dqm = 2.f*a, Dqp = 2.f*b, Dqc = 0.5f*(a + b);
-  if (Dqm*Dqp <= 0.f) return 0.f;
   const float am = fabsf(Dqm), ap = fabsf(Dqp), ac = fabsf(Dqc);
-  if ((am <= ap) && (am <= ac)) return Dqm;
-  if (ap <= ac) return Dqp;
-  return Dqc;
+  const bool m = (am <= ap) & (am <= ac);
+  float r = (ap <= ac) ? Dqp : Dqc;
+  r = m ? Dqm : r;
+  return (Dqm*Dqp <= 0.f) ? 0.f : r;
 }
 
 // ---------------------------------------------------------------------------
@@ -354,6 +352,11 @@ HD void ppm_faces_mixed(const Params& P, const Ptrs& X, const double* __restrict
   for (int m = 0; m < M; m++) raw[0][m] = src[c0 + zm[m]*st];
 #pragma unroll
   for (int v = 0; v < NP; v++) {
+    // this primitive's stencil has come before the next one's loads are issued
+#pragma unroll
+    for (int m = 0; m < M; m++) pin(raw[v & 1][m]);
+    long long next = (v + 1)*NT;
+    pin_uniform(next);
     double fz[M], fo[F];
     if (rs) {
 #pragma unroll
@@ -363,7 +366,7 @@ HD void ppm_faces_mixed(const Params& P, const Ptrs& X, const double* __restrict
     }
     if (v + 1 < NP) {
 #pragma unroll
-      for (int m = 0; m < M; m++) raw[(v + 1) & 1][m] = src[(v + 1)*NT + c0 + zm[m]*st];
+      for (int m = 0; m < M; m++) raw[(v + 1) & 1][m] = src[next + c0 + zm[m]*st];
     }
     double y[M];
 #pragma unroll
@@ -386,6 +389,10 @@ HD void ppm_faces_mixed(const Params& P, const Ptrs& X, const double* __restrict
       pl[f][v] = (float)l;
       pr[f][v] = (float)r;
     }
+    // the next primitive's limiters start after this one's are done (the compiler
+    // gathered all eight primitives' loads, with 28 to 300 registers spilled)
+#pragma unroll
+    for (int f = 0; f < F; f++) { pin(pl[f][v]); pin(pr[f][v]); }
   }
 }
 
@@ -512,6 +519,7 @@ HD void emf_edge_mixed(const Params& P, const Ptrs& X, int i, int j, int k) {
     for (int l = 0; l < 6; l++)
 #pragma unroll
       for (int m = 0; m < 6; m++) y[l][m] = line[l][c + (m - 3)*str[l]];
+    loads_issued();
     e0 = ppm_pair_f(y[0]) - ppm_pair_f(y[1]);
     e1 = ppm_pair_f(y[2]) - ppm_pair_f(y[3]);
     e2 = ppm_pair_f(y[4]) - ppm_pair_f(y[5]);

@@ -244,17 +244,70 @@ HD void vchar_fast(const State* q, GP g, double gam, double* vmax, double* vmin)
 // ---------------------------------------------------------------------------
 // Reconstruction (src/recon.c)
 
+// Order for the compiler (device): a value pinned is formed before what is pinned
+// after it; loads whose index is pinned stay behind what was pinned before, and
+// loads before loads_issued() are not moved behind it.
+template <class T>
+HD void pin(T& x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+v"(x));
+#endif
+}
+template <class T>
+HD void pin_uniform(T& x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+s"(x));
+#endif
+}
+HD void loads_issued() {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" ::: "memory");
+#endif
+}
+
+// The limiters come in two forms with the same results.  By selects between values
+// that all lanes form: neighbouring zones take different sides, and the branches
+// (about 85 per face) cost more than the sides they skip and keep independent chains
+// apart.  By branches, for the FP64 face groups (ppm_faces) and the FP64 EMFs of
+// large grids: FP64 issue is their bound, and whole wavefronts skip sides there.  Face
+// fluxes of a step, branches and selects: FP64 192x192x128 1.61 and 1.74 ms, mixed
+// 1.105 and 1.049, mixed 96x96x64 0.153 and 0.141.
+
 // linear_recon(), MC limiter, src/recon.c:88-132
 HD double mc_slope(double y1, double y2, double y3) {
-  double Dqm = 2.*(y2 - y1);
-  double Dqp = 2.*(y3 - y2);
-  double Dqc = 0.5*(y3 - y1);
-  double s = Dqm*Dqp;
-  if (s <= 0.) return 0.;
-  double aDqm = fabs(Dqm), aDqp = fabs(Dqp), aDqc = fabs(Dqc);
-  if ((aDqm <= aDqp) && (aDqm <= aDqc)) return Dqm;
-  else if (aDqp <= aDqc) return Dqp;
-  else return Dqc;
+  const double Dqm = 2.*(y2 - y1);
+  const double Dqp = 2.*(y3 - y2);
+  const double Dqc = 0.5*(y3 - y1);
+  const double s = Dqm*Dqp;
+  const double aDqm = fabs(Dqm), aDqp = fabs(Dqp), aDqc = fabs(Dqc);
+  const bool m = (aDqm <= aDqp) & (aDqm <= aDqc);
+  double r = (aDqp <= aDqc) ? Dqp : Dqc;
+  r = m ? Dqm : r;
+  return (s <= 0.) ? 0. : r;
+}
+
+// mc_slope_vect() by selects
+HD double mc_slope_sel(double ym, double y0, double yp) {
+  const double a = y0 - ym, b = yp - y0, s = a*b;
+  const double a_abs = fabs(a), b_abs = fabs(b);
+  const double a3 = a_abs + a_abs + a_abs, b3 = b_abs + b_abs + b_abs;
+  double r = 0.5*(a + b);
+  r = (b3 <= a_abs) ? b + b : r;
+  r = (a3 <= b_abs) ? a + a : r;
+  return (s <= 0.) ? 0. : r;
+}
+
+// ppm_limit() by selects
+HD void ppm_limit_sel(double l, double r, double yi, double* lnew, double* rnew) {
+  const double qa = (r - yi)*(yi - l);
+  const double r2 = r + r, l2 = l + l, y3 = yi + yi + yi;
+  const double sl = l + r2, sr = l2 + r;
+  const bool up = r > l;
+  const bool cl = (up & (y3 > sl)) | (!up & (y3 < sl)), cr = (up & (y3 < sr)) | (!up & (y3 > sr));
+  const bool flat = qa <= 0.;
+  const double ln = cl ? y3 - r2 : l, rn = cr ? y3 - l2 : r;
+  *lnew = flat ? yi : ln;
+  *rnew = flat ? yi : rn;
 }
 
 // linear_recon_vect() MC form, src/recon.c:237-264 (slope of the middle point)
@@ -286,17 +339,23 @@ HD void ppm_limit(double l, double r, double yi, double* lnew, double* rnew) {
 // PPM states at the interface between window points 2 and 3 of y[0..5]:
 // *yl = right edge of zone 2 (the reference's pR_vect[2]) and
 // *yr = left edge of zone 3 (pL_vect[3]), src/recon.c:237-264, :611-641.
+// BR: by branches.
+template <bool BR = false>
 HD void ppm_interface(const double* y, double* yl, double* yr) {
-  double dq1 = mc_slope_vect(y[0], y[1], y[2]);
-  double dq2 = mc_slope_vect(y[1], y[2], y[3]);
-  double dq3 = mc_slope_vect(y[2], y[3], y[4]);
-  double dq4 = mc_slope_vect(y[3], y[4], y[5]);
-  double f12 = 0.5*(y[2] + y[1]) - PPM_FACTOR*(dq2 - dq1);
-  double f23 = 0.5*(y[3] + y[2]) - PPM_FACTOR*(dq3 - dq2);
-  double f34 = 0.5*(y[4] + y[3]) - PPM_FACTOR*(dq4 - dq3);
+  double dq[4];
+#pragma unroll
+  for (int m = 0; m < 4; m++) dq[m] = BR ? mc_slope_vect(y[m], y[m + 1], y[m + 2]) : mc_slope_sel(y[m], y[m + 1], y[m + 2]);
+  double f12 = 0.5*(y[2] + y[1]) - PPM_FACTOR*(dq[1] - dq[0]);
+  double f23 = 0.5*(y[3] + y[2]) - PPM_FACTOR*(dq[2] - dq[1]);
+  double f34 = 0.5*(y[4] + y[3]) - PPM_FACTOR*(dq[3] - dq[2]);
   double l2, r2, l3, r3;
-  ppm_limit(f12, f23, y[2], &l2, &r2);
-  ppm_limit(f23, f34, y[3], &l3, &r3);
+  if (BR) {
+    ppm_limit(f12, f23, y[2], &l2, &r2);
+    ppm_limit(f23, f34, y[3], &l3, &r3);
+  } else {
+    ppm_limit_sel(f12, f23, y[2], &l2, &r2);
+    ppm_limit_sel(f23, f34, y[3], &l3, &r3);
+  }
   *yl = r2;
   *yr = l3;
 }
