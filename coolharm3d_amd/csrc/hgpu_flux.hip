@@ -341,7 +341,7 @@ __global__ __launch_bounds__(BLOCK, W) void k_flux_all(Params P, Ptrs X, const d
   }
 }
 
-// The same with one face per thread (MC slopes, degenerate directions)
+// The same with one face per thread (MC slopes, degenerate directions, small grids)
 template <int D, bool MIXED, int K>
 __device__ __forceinline__ void flux_one_block(const Params& P, const Ptrs& X, const double* __restrict__ src,
                                                bool active, int i, int j, int k) {
@@ -461,6 +461,21 @@ static bool flux_all_multi(const Params& P) {
 bool flux_all_possible(const Params& P) {
   return flux_all_multi(P) || P.recon != RECON_PPM_MC;
 }
+// Faces per thread.  A group's zones are reconstructed once for the whole group, so
+// more faces per thread are less work, in fewer and longer wavefronts.  Up to one
+// wavefront per SIMD a launch is one wavefront's chain: one face (24x24x16, a step's
+// fluxes: FP64 0.045 -> 0.027 ms, mixed 0.037 -> 0.026; at 48x48x32, 3900 wavefronts
+// of single faces, mixed 0.046 and 0.044 but a slower step).  Once groups of 4 fill
+// the FP32 solve's 4 wavefronts per SIMD, 4 faces: mixed 192x192x128 1.05 -> 0.885 ms,
+// 96x96x64 0.140 -> 0.136, binary disk 120x64x160 0.343 -> 0.303; 67x45x33, which
+// does not, 0.051 -> 0.057.  FP64 groups of 4 take 254 registers, two wavefronts
+// per SIMD, and gain nothing (1.61 ms at 192x192x128; disk 0.67 -> 0.94).
+constexpr long long ONE_FACE_WAVES = 1024, FOUR_FACE_WAVES = 4096;
+static unsigned flux_all_faces(const Params& P, long long faces) {
+  if (!flux_all_multi(P)) return 1;
+  if (faces <= 64 * ONE_FACE_WAVES && !P.otf) return 1;
+  return (P.mixed && faces >= 4 * 64 * FOUR_FACE_WAVES) ? 4 : 2;
+}
 void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStream_t st, const PnGrid& G, int lvl) {
   // Flat tiles of 256 in dispatch order: round-robin over the XCDs, so that
   // all of them work on one slab (1.62 ms a step on the 192x192x128 torus
@@ -468,19 +483,23 @@ void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStrea
   // the dispatch rate, 2.98 ms; 2D tiles of 64 x 4 take 2.34).
   LaunchShape L;
   L.remap = 0;
-  const bool multi = flux_all_multi(P);
-  L.spread = !multi;
-  const FluxAll A = make_flux_all(P, multi ? 2u : 1u, L);
+  long long faces = 0;
+  for (int d = 0; d < 3; d++) faces += flux_box(P, d).count();
+  const unsigned F = flux_all_faces(P, faces);
+  L.spread = F == 1;
+  const FluxAll A = make_flux_all(P, F, L);
   const dim3 grid(A.nblocks), blk(L.bs);
-  if (multi) {
+  if (F > 1) {
     if (P.otf) {
-      if (P.mixed) hipLaunchKernelGGL((k_flux_all<2, 3, true, GK_GEN, true>), grid, blk, 0, st, P, X, src, A, G, lvl);
+      if (P.mixed && F == 4) hipLaunchKernelGGL((k_flux_all<4, 3, true, GK_GEN, true>), grid, blk, 0, st, P, X, src, A, G, lvl);
+      else if (P.mixed) hipLaunchKernelGGL((k_flux_all<2, 3, true, GK_GEN, true>), grid, blk, 0, st, P, X, src, A, G, lvl);
       else hipLaunchKernelGGL((k_flux_all<2, 1, false, GK_GEN, true>), grid, blk, 0, st, P, X, src, A, G, lvl);
       return;
     }
     const auto go = [&](auto K) {
       constexpr int k = decltype(K)::value;
-      if (P.mixed) hipLaunchKernelGGL((k_flux_all<2, 4, true, k, false>), grid, blk, 0, st, P, X, src, A, G, lvl);
+      if (P.mixed && F == 4) hipLaunchKernelGGL((k_flux_all<4, 4, true, k, false>), grid, blk, 0, st, P, X, src, A, G, lvl);
+      else if (P.mixed) hipLaunchKernelGGL((k_flux_all<2, 4, true, k, false>), grid, blk, 0, st, P, X, src, A, G, lvl);
       else hipLaunchKernelGGL((k_flux_all<2, 3, false, k, false>), grid, blk, 0, st, P, X, src, A, G, lvl);
     };
     if (P.gkind == GK_KS) go(std::integral_constant<int, GK_KS>());

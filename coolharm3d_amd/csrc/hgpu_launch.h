@@ -265,8 +265,8 @@ __device__ __forceinline__ PnOrbit orbit_load(const PnOrbit* p) {
 // hgpu_flux.hip: face fluxes of direction d with launch shape L
 void launch_flux_dir(int d, const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, hipStream_t st,
                      const PnGrid& G, int lvl);
-// The three directions in one launch (flux_all_possible(); 2 faces per thread,
-// or one where flux_all_multi() says no)
+// The three directions in one launch (flux_all_possible()), 1, 2 or 4 faces per
+// thread by the grid's size
 bool flux_all_possible(const Params& P);
 void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStream_t st, const PnGrid& G, int lvl);
 
