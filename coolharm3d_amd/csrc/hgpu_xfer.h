@@ -88,12 +88,17 @@ struct XferRing {
   // at least the chunks that `bytes` can use; nothing may be in flight
   hipError_t reserve(size_t bytes) {
     const size_t want = (bytes + SLOT - 1) / SLOT;
-    const int n = (int)std::min<size_t>(SLOTS, std::max<size_t>(1, want));
+    int n = (int)std::min<size_t>(SLOTS, std::max<size_t>(1, want));
     if (n <= slots) return hipSuccess;
     release();
     void *p = nullptr, *d = nullptr;
     hipError_t e = hipGetDevice(&device);
     if (e == hipSuccess) e = hipHostMalloc(&p, n * SLOT, hipHostMallocDefault);
+    while (e == hipErrorOutOfMemory && n > 1) {   // pinned memory is short: a smaller ring, down to one chunk
+      (void)hipGetLastError();
+      n /= 2;
+      e = hipHostMalloc(&p, n * SLOT, hipHostMallocDefault);
+    }
     if (e != hipSuccess) return e;
     host = static_cast<char*>(p);
     e = hipHostGetDevicePointer(&d, p, 0);
