@@ -152,7 +152,7 @@ __device__ void ppm_faces_x3_staged(const Params& P, const Ptrs& X, const double
 // thread's tile index along D counts groups of F faces from bg.lo[D]; faces
 // past hi_d (the flux box end) are skipped.  Each zone's parabola is computed
 // once per group.  The per-face fail() tally goes to the face's zone here,
-// the block totals through commit_fail().
+// the totals through commit_flux().
 // Along x3 (the fastest index of the arrays) a lane's F faces are adjacent in
 // memory, so the fluxes go through LDS: slot s of lane l stores element
 // s*64 + l of the wavefront's F*64 faces, and each store instruction writes
