@@ -499,11 +499,15 @@ def main():
     units = units_per_launch(n1, n2, n3)
     # faces of a step's two stages and three directions over its flux launches (one a stage, or
     # one per direction)
-    units["flux"] *= 6.0 * args.prof_steps / max(kern["flux"][1], 1)
+    directions = 6.0 * args.prof_steps / max(kern["flux"][1], 1)
+    units["flux"] *= directions
     model = ALGO_BYTES if tag == "fp64" else ALGO_BYTES_MIXED
     per_launch_s = {k: kern[k][0] / max(kern[k][1], 1) / 1e3 for k in ("flux", "emf", "update")}
     workload = f"torus{n1}x{n2}x{n3}_{tag}"
     traffic_tab = measured_traffic(workload)
+    # the flux summary is of the launch over all directions
+    if traffic_tab and directions < 2.5:
+        traffic_tab["flux"] = None
     # the dominant kernel: the conserved update + inversion (k_update), the longest
     # single kernel of the step; its algorithmic bytes are the state's 160 B per zone
     avg_s = per_launch_s["update"]
