@@ -4,6 +4,13 @@
 
 namespace hgpu {
 
+// n GAMMA_CALC failures of a face into the map's zone c.  The faces (i,j,k) of the
+// three directions share the zone and may run at the same time, in workgroups of
+// one launch, so the (rare) addition is atomic.
+__device__ __forceinline__ void tally_face(const Params& P, const Ptrs& X, long long c, int n) {
+  if (P.track_nfail && n) atomicAdd(&X.nfail[NFAIL_GAMMA_CALC*P.nt + c], n);
+}
+
 // W: minimum waves per SIMD the register allocation must allow (1 = the
 // compiler's choice; larger values cap the VGPRs, trading spills for occupancy).
 // K: structure of the geometry records (GK_*).
@@ -17,7 +24,7 @@ __global__ __launch_bounds__(BLOCK, W) void k_flux(Params P, Ptrs X, const doubl
     flux_face<D, K>(P, X, src, i, j, k, fr);
     c = cidx(P, i, j, k);
   }
-  if (P.track_nfail && active && fr.nf[NFAIL_GAMMA_CALC]) X.nfail[NFAIL_GAMMA_CALC*P.nt + c] += fr.nf[NFAIL_GAMMA_CALC];
+  if (active) tally_face(P, X, c, fr.nf[NFAIL_GAMMA_CALC]);
   commit_flux(X, fr, active, D + 1);
 }
 
@@ -32,7 +39,7 @@ __global__ __launch_bounds__(BLOCK, W) void k_flux_mixed(Params P, Ptrs X, const
     flux_face_mixed<D, K>(P, X, src, i, j, k, fr);
     c = cidx(P, i, j, k);
   }
-  if (P.track_nfail && active && fr.nf[NFAIL_GAMMA_CALC]) X.nfail[NFAIL_GAMMA_CALC*P.nt + c] += fr.nf[NFAIL_GAMMA_CALC];
+  if (active) tally_face(P, X, c, fr.nf[NFAIL_GAMMA_CALC]);
   commit_flux(X, fr, active, D + 1);
 }
 
@@ -216,7 +223,7 @@ __device__ __forceinline__ void flux_multi_block(const Params& P, const Ptrs& X,
         else flux_riemann<D, K>(P, X, pl[f], pr[f], fi, fj, fk, fr, TRANSPOSE ? fo[f] : nullptr);
       }
       const int dv = fr.nf[NFAIL_GAMMA_CALC] - g0;
-      if (P.track_nfail && dv) X.nfail[NFAIL_GAMMA_CALC*P.nt + cidx(P, fi, fj, fk)] += dv;
+      tally_face(P, X, cidx(P, fi, fj, fk), dv);
     }
     cb = cidx(P, i, j, k);
     nv = nvalid;
@@ -352,7 +359,7 @@ __device__ __forceinline__ void flux_one_block(const Params& P, const Ptrs& X, c
     else flux_face<D, K>(P, X, src, i, j, k, fr);
     c = cidx(P, i, j, k);
   }
-  if (P.track_nfail && active && fr.nf[NFAIL_GAMMA_CALC]) X.nfail[NFAIL_GAMMA_CALC*P.nt + c] += fr.nf[NFAIL_GAMMA_CALC];
+  if (active) tally_face(P, X, c, fr.nf[NFAIL_GAMMA_CALC]);
   commit_flux(X, fr, active, D + 1);
 }
 template <int W, bool MIXED, int K>
