@@ -464,7 +464,7 @@ HD int source(const Params& P, const Ptrs& X, const double* ph, GP g, int i, int
       return s.gfail;
     }
   }
-  if constexpr (geom_kind<GP>::value == GK_FLAT) return 0;   // no connection, no cooling
+  if constexpr (geom_kind<GP>::value == GK_FLAT) return 0;   // the flat metric: no connection, no cooling
   int gfail = 0;
   State q;
   bool have_q = false;

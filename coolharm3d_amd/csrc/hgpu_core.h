@@ -332,7 +332,7 @@ struct Api {
     if (rc) { destroy(c); return set_error(-3, "device allocation failed: " + g_last_error); }
     if (!c->P.otf) rc |= alloc_levels(c);
     if (rc) { destroy(c); return rc; }
-    if (!T.geom.empty()) c->P.gkind = metric_structure(reinterpret_cast<const Geom*>(T.geom.data()), c->n_geom);
+    if (!T.geom.empty()) c->P.gkind = metric_structure(reinterpret_cast<const Geom*>(T.geom.data()), c->n_geom, P.flat != 0);
     if (!T.geom.empty()) rc |= BE::h2d(c, (void*)X.geom, T.geom.data(), sizeof(double) * T.geom.size());
     if (P.dyn) {
       // coordinate functions along each direction, evaluated once here and

@@ -65,7 +65,8 @@ struct GeomF {
 // zero and reads one of two equal components: the sums keep their order and a
 // dropped term is +-0, so the results keep their bits (a zero may change its
 // sign).  metric_structure() finds the structure from the records themselves.
-//   GK_FLAT: the Minkowski record, every component a known constant
+//   GK_FLAT: the Minkowski record, every component a known constant, of the flat
+//            metric (Params::flat), which has no source terms either
 //   GK_KS:   Kerr-Schild on a diagonal coordinate map -- gcov tt tr tp rr rp hh
 //            pp, gcon tt tr rr rp hh pp, a radial shift
 //   GK_DIAG: a diagonal spatial block with any shift (the binary's metric)
@@ -84,9 +85,11 @@ struct GeomView {
 template <class GP> struct geom_kind { static constexpr int value = GK_GEN; };
 template <int K, class P> struct geom_kind<GeomView<K, P>> { static constexpr int value = K; };
 
-// Structure of n static records: GK_FLAT, GK_KS or GK_GEN
-inline int metric_structure(const Geom* r, long long n) {
-  bool flat = true, ks = true;
+// Structure of n static records: GK_FLAT, GK_KS or GK_GEN.  flat_metric:
+// Params::flat; Minkowski records uploaded to a context of another metric keep
+// that context's connection and cooling, so they are not GK_FLAT.
+inline int metric_structure(const Geom* r, long long n, bool flat_metric) {
+  bool flat = flat_metric, ks = true;
   for (long long m = 0; m < n && (flat || ks); m++) {
     const Geom& g = r[m];
     for (int a = 0; a < 4; a++)

@@ -7,7 +7,7 @@ import pytest
 
 from coolharm3d_amd import Harm3D, balsara1, balsara1_grid, torus, torus_grid
 
-GCON = 0       # offset of gcon[4][4] in a 42-double record
+GCON, GCOV = 0, 16       # offsets of gcon[4][4] and gcov[4][4] in a 42-double record
 
 
 def _run(grid, p, general, hostcheck, steps, **kw):
@@ -61,3 +61,47 @@ def test_structure_equals_general_hostbuild(case):
 @pytest.mark.parametrize("case", CASES, ids=str)
 def test_structure_equals_general_gpu(case):
     _compare(case, hostcheck=False)
+
+
+def _minkowski_on_kerr_context(hostcheck, general, conn_scale, **kw):
+    """A context of the Kerr metric given Minkowski records and a connection of its
+    own (cooling on): its source terms stay."""
+    grid = torus_grid(12, 11, 8)
+    H = Harm3D(grid, hostcheck=hostcheck, **kw)
+    g, c = H.geometry()
+    r = np.zeros(42)
+    r[GCON:GCON + 16] = r[GCOV:GCOV + 16] = np.diag([-1.0, 1.0, 1.0, 1.0]).ravel()
+    r[32:35] = 1.0                                        # g, g_inv, alpha
+    r[38] = 1.0                                           # ncon[0]
+    g[:] = r
+    if general:
+        g[0, GCON + 2] = g[0, GCON + 8] = 5e-324
+    rng = np.random.default_rng(11)
+    H.set_geometry(geom=g, conn=conn_scale * rng.standard_normal(c.shape))
+    p = np.empty(H.shape + (8,))
+    p[..., :2] = rng.uniform(1.0, 2.0, H.shape + (2,))
+    p[..., 2:] = rng.uniform(-0.1, 0.1, H.shape + (6,))
+    H.set_prims(p)
+    H.fixup_bounds()
+    H.set_time(0.0, 1e-4)
+    H.step_ch(2)
+    return H
+
+
+def _compare_minkowski(hostcheck, precision):
+    A, B, N = (_minkowski_on_kerr_context(hostcheck, general, scale, precision=precision)
+               for general, scale in ((False, 1.0), (True, 1.0), (True, 0.0)))
+    assert np.abs(A.prims() - B.prims()).max() <= 1e-300
+    assert np.array_equal(A.nfail(), B.nfail())
+    assert np.abs(B.prims() - N.prims()).max() > 1e-5     # the connection's terms are there
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_minkowski_records_keep_sources_hostbuild(precision):
+    _compare_minkowski(True, precision)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_minkowski_records_keep_sources_gpu(precision):
+    _compare_minkowski(False, precision)
