@@ -7,6 +7,7 @@
 // Failure counters are summed across the wavefront before one atomic per wave.
 #include "hgpu_launch.h"
 #include "hgpu_xfer.h"
+#include <cstdlib>
 
 namespace hgpu {
 
@@ -631,6 +632,8 @@ struct GpuBE {
           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
         g->flag_grid = g->simds = 4u * (unsigned)cus;
     }
+    if (const char* n = std::getenv("HGPU_PINNED_CHUNKS"))
+      g->ring.cap = std::max(0, std::min(std::atoi(n), XferRing::SLOTS));
     return hip_check(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking), "hipStreamCreate");
   }
   static void fini(hgpu_ctx* c) {
@@ -666,10 +669,9 @@ struct GpuBE {
         const unsigned nb = (unsigned)std::min<long long>((n32 / 4 + XFER_B - 1) / XFER_B + 1, 512);
         hipLaunchKernelGGL(k_copy_words, dim3(nb), dim3(XFER_B), 0, g->stream,
                            reinterpret_cast<const unsigned*>(src + off), n32, reinterpret_cast<unsigned*>(chunk));
-      }), "copy to host");
+      }, [&]() { return plain_to_host(g->stream, h, d, bytes); }), "copy to host");
     }
-    return hip_check(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, g->stream), "hipMemcpy D2H") |
-           hip_check(hipStreamSynchronize(g->stream), "hipStreamSynchronize");
+    return hip_check(plain_to_host(g->stream, h, d, bytes), "copy to host");
   }
   // a state array S ([8][nt]) to or from the host's [nt][8]
   static int download_state(hgpu_ctx* c, double* h, const double* S, long long nt) {
@@ -678,7 +680,7 @@ struct GpuBE {
       const long long z0 = (long long)(off / (sizeof(double) * NP)), nz = (long long)(len / (sizeof(double) * NP));
       hipLaunchKernelGGL(k_soa_to_aos, dim3((unsigned)((nz + XFER_B - 1) / XFER_B)), dim3(XFER_B), 0, g->stream, S, nt,
                          z0, nz, reinterpret_cast<double*>(chunk));
-    }), "state to host");
+    }, [&]() { return plain_state_to_host(g->stream, h, S, nt, NP); }), "state to host");
   }
   static int upload_state(hgpu_ctx* c, double* S, const double* h, long long nt) {
     GpuPriv* g = priv(c);
@@ -686,7 +688,7 @@ struct GpuBE {
       const long long z0 = (long long)(off / (sizeof(double) * NP)), nz = (long long)(len / (sizeof(double) * NP));
       hipLaunchKernelGGL(k_aos_to_soa, dim3((unsigned)((nz + XFER_B - 1) / XFER_B)), dim3(XFER_B), 0, g->stream,
                          reinterpret_cast<const double*>(chunk), nt, z0, nz, S);
-    }), "state to device");
+    }, [&]() { return plain_state_to_device(g->stream, S, h, nt, NP); }), "state to device");
   }
   // zero fill with a kernel (no memset nodes on the stream)
   static int zero(hgpu_ctx* c, void* p, size_t bytes) {

@@ -96,7 +96,11 @@ int hgpu_destroy(hgpu_ctx *ctx);
 /* Grid sizes: out[0..6] = N1, N2, N3, N1TOT, N2TOT, N3TOT, NG */
 int hgpu_dims(const hgpu_ctx *ctx, int *out);
 
-/* Primitive state transfer, which = 0: p, 1: ph.  Host layout [i][j][k][8]. */
+/* Primitive state transfer, which = 0: p, 1: ph.  Host layout [i][j][k][8].
+ * Copies to and from the host go through up to 8 pinned chunks of 2 MB a
+ * context; fewer where pinned memory is short, none with HGPU_PINNED_CHUNKS=0 in
+ * the environment when the context is created (any number below 8 is a limit):
+ * the runtime's copies of pageable memory then, which are slower. */
 int hgpu_upload_prims(hgpu_ctx *ctx, int which, const double *host);
 int hgpu_download_prims(hgpu_ctx *ctx, int which, double *host);
 

@@ -38,3 +38,18 @@ def test_maps_after_a_step(n):
     assert np.array_equal(H.download_box(0, (0, 0, 0), hi)[1], H.pflag())
     gam = H.gamma()[3:-3, 3:-3, 3:-3]
     assert (gam >= 1.0).all() and np.isfinite(gam).all()
+
+
+@pytest.mark.parametrize("chunks", [0, 1, 2, 5])
+@pytest.mark.parametrize("n", [(5, 3, 5), (60, 50, 40), (130, 100, 40)], ids=str)
+def test_fewer_pinned_chunks(monkeypatch, chunks, n):
+    """Rings of fewer chunks than a copy wants, and none: the plain copies."""
+    monkeypatch.setenv("HGPU_PINNED_CHUNKS", str(chunks))
+    H = Harm3D(torus_grid(*n), track_nfail=0)
+    p = np.random.default_rng(chunks).random(H.shape + (8,))
+    for which in (0, 1):
+        H.set_prims(p, which)
+        assert np.array_equal(H.prims(which), p)
+    hi = [s - 1 for s in H.shape]
+    box, flags = H.download_box(1, (0, 0, 0), hi)
+    assert np.array_equal(box, p) and np.array_equal(flags, H.pflag())
