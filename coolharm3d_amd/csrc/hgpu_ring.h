@@ -9,6 +9,7 @@
 #include <cstddef>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <new>
 #include <thread>
 #include <vector>
@@ -16,7 +17,8 @@
 namespace hgpu {
 
 // Ring of pinned chunks of one context, on its device; sized by the largest
-// copy so far (at most cap chunks), released with the context.
+// copy so far (at most cap chunks), released with the context.  One copy at a time
+// (busy): threads that read from one context wait for each other.
 struct XferRing {
   static constexpr size_t SLOT = 2u << 20;     // a multiple of 64 B (a zone) and 16 B
   static constexpr int SLOTS = 8;
@@ -24,6 +26,7 @@ struct XferRing {
   char* dev = nullptr;                         // the device's address of host
   hipEvent_t ev[SLOTS] = {};
   int slots = 0, device = 0;
+  std::mutex busy;
   int cap = SLOTS;                             // most chunks to ask for; lowered where pinned memory ran short
 
   void release() {
@@ -84,6 +87,7 @@ inline int xfer_threads(size_t bytes) {
 // holds all of it.
 template <class Fill, class Plain>
 hipError_t xfer_to_host(XferRing& R, hipStream_t st, void* host, size_t bytes, Fill&& fill, Plain&& plain) {
+  std::lock_guard<std::mutex> one(R.busy);
   if (!R.reserve(bytes)) return plain();
   hipError_t e = hipSuccess;
   const long long n = (long long)((bytes + XferRing::SLOT - 1) / XferRing::SLOT);
@@ -152,6 +156,7 @@ hipError_t xfer_to_host(XferRing& R, hipStream_t st, void* host, size_t bytes, F
 // above.  Returns when the device holds all of it.
 template <class Empty, class Plain>
 hipError_t xfer_to_device(XferRing& R, hipStream_t st, const void* host, size_t bytes, Empty&& empty, Plain&& plain) {
+  std::lock_guard<std::mutex> one(R.busy);
   if (!R.reserve(bytes)) return plain();
   hipError_t e = hipSuccess;
   const long long n = (long long)((bytes + XferRing::SLOT - 1) / XferRing::SLOT);

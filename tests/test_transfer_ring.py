@@ -164,6 +164,16 @@ CASES = {
     CHECK(round_trip(R, 2*ZC, 9) && rt.mallocs == asked);
   }
 """,
+    # several threads with a ring between them
+    "threads": r"""
+  XferRing R;
+  std::atomic<int> bad{0};
+  std::vector<std::thread> t;
+  for (int k = 0; k < 4; k++)
+    t.emplace_back([&, k]() { for (int q = 0; q < 12; q++) if (!round_trip(R, (q % 3) * ZC + 900*k + 7, 100*k + q)) bad++; });
+  for (auto& x : t) x.join();
+  CHECK(bad == 0);
+""",
 }
 
 

@@ -53,3 +53,20 @@ def test_fewer_pinned_chunks(monkeypatch, chunks, n):
     hi = [s - 1 for s in H.shape]
     box, flags = H.download_box(1, (0, 0, 0), hi)
     assert np.array_equal(box, p) and np.array_equal(flags, H.pflag())
+
+
+def test_threads_read_one_context():
+    """Several host threads read one context at the same time."""
+    from concurrent.futures import ThreadPoolExecutor
+    H = Harm3D(torus_grid(60, 50, 40))
+    p = np.random.default_rng(2).random(H.shape + (8,))
+    H.set_prims(p)
+    H.set_prims(2.0 * p, 1)
+    H.set_time(1.5, 0.25)
+
+    def read(k):
+        if k % 3 == 2:
+            return H.time() == (1.5, 0.25, 0.25)
+        return np.array_equal(H.prims(k % 3), p * (1 + k % 3))
+    with ThreadPoolExecutor(4) as pool:
+        assert all(pool.map(read, range(24)))
