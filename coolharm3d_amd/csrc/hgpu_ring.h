@@ -4,8 +4,10 @@
 // place where no memory can be pinned.  Host API of the runtime only.
 #pragma once
 #include <hip/hip_runtime_api.h>
+#include <sched.h>
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstddef>
 #include <cstring>
 #include <memory>
@@ -74,10 +76,13 @@ struct XferRing {
 
 // Host threads beside the caller for a copy of `bytes`: none below 4 MB (a few
 // chunks: starting threads would cost what they save), else enough to keep up
-// with the link (a core copies about 29 GB/s, less into fresh pages).
+// with the link (a core copies about 29 GB/s, less into fresh pages), and at most
+// half the CPUs that the process may run on (the ranks of a node share its CPUs).
 inline int xfer_threads(size_t bytes) {
   if (bytes < (4u << 20)) return 0;
-  const unsigned hw = std::thread::hardware_concurrency();
+  cpu_set_t cpus;
+  const unsigned hw = sched_getaffinity(0, sizeof(cpus), &cpus) == 0 ? (unsigned)CPU_COUNT(&cpus)
+                                                                     : std::thread::hardware_concurrency();
   return (int)std::min<unsigned>(hw > 2 ? hw / 2 : 0, bytes < (32u << 20) ? 3 : 6);
 }
 
@@ -109,7 +114,16 @@ hipError_t xfer_to_host(XferRing& R, hipStream_t st, void* host, size_t bytes, F
   std::atomic<long long> copied[XferRing::SLOTS];   // chunks taken out of each slot
   for (auto& x : copied) x.store(0);
   std::atomic<int> err{(int)hipSuccess};
+  // The workers sleep until the first chunk is there: work queued on the stream
+  // before the copy may take long, and the caller alone waits for that.
+  std::mutex gate;
+  std::condition_variable opened;
+  bool open = false;
   const auto worker = [&]() {
+    {
+      std::unique_lock<std::mutex> l(gate);
+      opened.wait(l, [&]() { return open; });
+    }
     if (hipSetDevice(R.device) != hipSuccess) err = (int)hipErrorInvalidDevice;
     for (;;) {
       const long long c = next.fetch_add(1);
@@ -138,11 +152,22 @@ hipError_t xfer_to_host(XferRing& R, hipStream_t st, void* host, size_t bytes, F
       if (e == hipSuccess) e = take(c);
     }
   } else {
-    for (long long c = 0; c < n && err.load() == (int)hipSuccess; c++) {
-      while (copied[c % S].load(std::memory_order_acquire) < c / S && err.load() == (int)hipSuccess) std::this_thread::yield();
+    const auto put = [&](long long c) {
       const hipError_t r = enqueue(c);
-      if (r != hipSuccess) { err = (int)r; break; }
-      enqueued.store(c + 1, std::memory_order_release);
+      if (r != hipSuccess) err = (int)r;
+      else enqueued.store(c + 1, std::memory_order_release);
+    };
+    long long c = 0;
+    for (; c < n && c < S && err.load() == (int)hipSuccess; c++) put(c);
+    if (err.load() == (int)hipSuccess && (e = hipEventSynchronize(R.ev[0])) != hipSuccess) err = (int)e;
+    {
+      std::lock_guard<std::mutex> l(gate);
+      open = true;
+    }
+    opened.notify_all();
+    for (; c < n && err.load() == (int)hipSuccess; c++) {
+      while (copied[c % S].load(std::memory_order_acquire) < c / S && err.load() == (int)hipSuccess) std::this_thread::yield();
+      put(c);
     }
     for (auto& t : pool) t.join();
     e = (hipError_t)err.load();

@@ -10,10 +10,13 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 
 STUB = r"""
 #pragma once
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <sched.h>
 #include <mutex>
+#include <thread>
 enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorInvalidDevice = 101, hipErrorInvalidHandle = 400 };
 enum hipMemcpyKind { hipMemcpyHostToDevice, hipMemcpyDeviceToHost };
 enum { hipHostMallocDefault = 0, hipEventDisableTiming = 2 };
@@ -25,6 +28,8 @@ struct Rt {
   std::map<void*, size_t> pinned;
   size_t budget = ~(size_t)0, used = 0, most = 0;
   int mallocs = 0, events = 0, event_limit = 1 << 20, copies = 0;
+  int busy_ms = 0, waiters_then = 0;
+  std::thread::id first_waiter;
   hipError_t malloc_error = hipErrorOutOfMemory;
 } rt;
 static thread_local int t_device = 0;
@@ -60,7 +65,19 @@ inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
 }
 inline hipError_t hipEventDestroy(hipEvent_t e) { std::lock_guard<std::mutex> l(rt.m); rt.events--; delete e; return hipSuccess; }
 inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t st) { return e->device == *st ? hipSuccess : fails(hipErrorInvalidHandle); }
-inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventSynchronize(hipEvent_t) {
+  std::unique_lock<std::mutex> l(rt.m);
+  if (rt.first_waiter == std::thread::id()) {
+    rt.first_waiter = std::this_thread::get_id();
+    l.unlock();
+    std::this_thread::sleep_for(std::chrono::milliseconds(rt.busy_ms));
+    l.lock();
+    rt.busy_ms = 0;
+  } else if (rt.busy_ms) {
+    rt.waiters_then++;
+  }
+  return hipSuccess;
+}
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
   std::lock_guard<std::mutex> l(rt.m);
@@ -173,6 +190,27 @@ CASES = {
     t.emplace_back([&, k]() { for (int q = 0; q < 12; q++) if (!round_trip(R, (q % 3) * ZC + 900*k + 7, 100*k + q)) bad++; });
   for (auto& x : t) x.join();
   CHECK(bad == 0);
+""",
+    # work queued before the copy is waited for by the caller alone; no more host threads
+    # than the process's CPUs allow
+    "crew": r"""
+  XferRing R;
+  const long long nt = 23*ZC + 7;
+  const std::vector<double> S = values(nt, 1);
+  std::vector<double> h(S.size());
+  rt.busy_ms = 50;                                       // the first wait takes this long
+  CHECK(down(R, h.data(), S.data(), nt) == hipSuccess);
+  for (long long z = 0; z < nt; z++) for (int v = 0; v < NV; v++) CHECK(h[z*NV + v] == S[v*nt + z]);
+  CHECK(rt.first_waiter == std::this_thread::get_id() && rt.waiters_then == 0);
+  cpu_set_t all, some;
+  CHECK(sched_getaffinity(0, sizeof(all), &all) == 0);
+  for (int want : {1, 2, 4}) {
+    CPU_ZERO(&some);
+    for (int c = 0, k = 0; c < CPU_SETSIZE && k < want; c++) if (CPU_ISSET(c, &all)) { CPU_SET(c, &some); k++; }
+    if (CPU_COUNT(&some) < want) break;
+    CHECK(sched_setaffinity(0, sizeof(some), &some) == 0);
+    CHECK(xfer_threads(64u << 20) == (want > 2 ? want / 2 : 0));
+  }
 """,
 }
 
