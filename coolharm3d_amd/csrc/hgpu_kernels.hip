@@ -626,10 +626,10 @@ struct GpuBE {
     // bounds(prim,1)) stride over their zones with 4 workgroups per CU: a
     // full grid of workgroups that find the flag clear costs several
     // microseconds just to dispatch.
-    {
-      int dev = 0, cus = 0;
-      if (hipGetDevice(&dev) == hipSuccess &&
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess) {
+      g->ring.device = dev;
+      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
         g->flag_grid = g->simds = 4u * (unsigned)cus;
     }
     if (const char* n = std::getenv("HGPU_PINNED_CHUNKS"))

@@ -18,6 +18,16 @@
 
 namespace hgpu {
 
+// The calling thread's current device while in scope
+struct DeviceScope {
+  int before = 0;
+  bool moved = false;
+  explicit DeviceScope(int device) {
+    if (hipGetDevice(&before) == hipSuccess && before != device) moved = hipSetDevice(device) == hipSuccess;
+  }
+  ~DeviceScope() { if (moved) (void)hipSetDevice(before); }
+};
+
 // Ring of pinned chunks of one context, on its device; sized by the largest
 // copy so far (at most cap chunks), released with the context.  One copy at a time
 // (busy): threads that read from one context wait for each other.
@@ -27,7 +37,8 @@ struct XferRing {
   char* host = nullptr;
   char* dev = nullptr;                         // the device's address of host
   hipEvent_t ev[SLOTS] = {};
-  int slots = 0, device = 0;
+  int slots = 0;
+  int device = 0;                              // the context's, whatever the calling thread's is
   std::mutex busy;
   int cap = SLOTS;                             // most chunks to ask for; lowered where pinned memory ran short
 
@@ -42,8 +53,7 @@ struct XferRing {
   bool grow(int n) {
     void *p = nullptr, *d = nullptr;
     int have = slots;
-    hipError_t e = hipGetDevice(&device);
-    if (e == hipSuccess) e = hipHostMalloc(&p, n * SLOT, hipHostMallocDefault);
+    hipError_t e = hipHostMalloc(&p, n * SLOT, hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostGetDevicePointer(&d, p, 0);
     for (; e == hipSuccess && have < n; have++) {
       e = hipEventCreateWithFlags(&ev[have], hipEventDisableTiming);
@@ -93,6 +103,7 @@ inline int xfer_threads(size_t bytes) {
 template <class Fill, class Plain>
 hipError_t xfer_to_host(XferRing& R, hipStream_t st, void* host, size_t bytes, Fill&& fill, Plain&& plain) {
   std::lock_guard<std::mutex> one(R.busy);
+  const DeviceScope on(R.device);
   if (!R.reserve(bytes)) return plain();
   hipError_t e = hipSuccess;
   const long long n = (long long)((bytes + XferRing::SLOT - 1) / XferRing::SLOT);
@@ -182,6 +193,7 @@ hipError_t xfer_to_host(XferRing& R, hipStream_t st, void* host, size_t bytes, F
 template <class Empty, class Plain>
 hipError_t xfer_to_device(XferRing& R, hipStream_t st, const void* host, size_t bytes, Empty&& empty, Plain&& plain) {
   std::lock_guard<std::mutex> one(R.busy);
+  const DeviceScope on(R.device);
   if (!R.reserve(bytes)) return plain();
   hipError_t e = hipSuccess;
   const long long n = (long long)((bytes + XferRing::SLOT - 1) / XferRing::SLOT);

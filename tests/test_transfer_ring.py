@@ -191,6 +191,15 @@ CASES = {
   for (auto& x : t) x.join();
   CHECK(bad == 0);
 """,
+    # a thread whose current device is another than the context's
+    "device": r"""
+  stream_device = 1;
+  XferRing R;
+  R.device = 1;
+  CHECK(round_trip(R, 3*ZC + 5, 1) && rt.copies == 0 && R.slots == 4);
+  int now = -1;
+  CHECK(hipGetDevice(&now) == hipSuccess && now == 0);
+""",
     # work queued before the copy is waited for by the caller alone; no more host threads
     # than the process's CPUs allow
     "crew": r"""
