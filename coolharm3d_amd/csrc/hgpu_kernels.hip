@@ -21,7 +21,6 @@ struct GpuPriv {
   bool graph = false;                  // replay captured steps
   hipGraphExec_t step_exec = nullptr;  // one step_ch(), captured on first use
   LaunchShape shape[N_FAM];            // per kernel family
-  bool flux_all = true;                // the three face-flux directions in one launch
   std::vector<ProfEvent> pending;
   std::vector<hipEvent_t> pool;
   std::map<std::string, std::pair<double, long long>> acc;
@@ -612,6 +611,7 @@ struct GpuBE {
       g->shape[f].fpt = 2;
       g->shape[f].occ = mixed ? 0u : 1u;
       g->shape[f].remap = 0;
+      g->shape[f].all = 1;
     }
     // x2 stencils share rows with the neighbouring tiles: XCD-contiguous
     // tiles keep those in one L2 (half the HBM reads of round-robin tiles)
@@ -813,7 +813,18 @@ struct GpuBE {
   // inversion keeps its own shape (it rewrites the state) unless set.
   static unsigned fpt_code(unsigned fpt) { return fpt == 4 ? 2u : (fpt == 2 ? 1u : 0u); }
   static unsigned shape_flags(const LaunchShape& L) {
-    return L.remap | (L.order << 1) | (L.occ << 2) | (L.fused << 3) | (fpt_code(L.fpt) << 4) | (L.stage << 6);
+    return L.remap | (L.order << 1) | (L.occ << 2) | (L.fused << 3) | (fpt_code(L.fpt) << 4) | (L.stage << 6) |
+           (L.all << 7);
+  }
+  // the flags as a caller sees them: bit 7 only where the directions can share a launch
+  static unsigned shown_flags(hgpu_ctx* c, int fam) {
+    LaunchShape L = priv(c)->shape[fam];
+    if (!flux_all_possible(c->P)) L.all = 0;
+    return shape_flags(L);
+  }
+  static bool flux_in_one(hgpu_ctx* c) {
+    const LaunchShape* s = priv(c)->shape;
+    return s[FAM_FLUX1].all && s[FAM_FLUX2].all && s[FAM_FLUX3].all && flux_all_possible(c->P);
   }
   static int check_shape(const LaunchShape& L) {
     if (L.bs != 64 && L.bs != 128 && L.bs != 256) return set_error(-2, "workgroup size must be 64, 128 or 256");
@@ -833,14 +844,15 @@ struct GpuBE {
     const unsigned fcode = ((unsigned)flags >> 4) & 3u;
     L.fpt = 1u << fcode;
     L.stage = ((unsigned)flags >> 6) & 1u;
-    if (bs < 0 || kc < 0 || flags < 0 || flags > 127 || fcode > 2) return set_error(-2, "bad launch-shape field");
+    L.all = ((unsigned)flags >> 7) & 1u;
+    if (bs < 0 || kc < 0 || flags < 0 || flags > 255 || fcode > 2) return set_error(-2, "bad launch-shape field");
     if (L.stage && fam != FAM_FLUX3) return set_error(-2, "flag bit 6 (staged pencils) applies to the x3 face fluxes only");
     if (L.fused && fam != FAM_CONS) return set_error(-2, "flag bit 3 (fused update) applies to the conserved update only");
     if (L.fpt > 1 && fam > FAM_FLUX3) return set_error(-2, "flag bits 4-5 (faces per thread) apply to the face fluxes only");
+    if (L.all && fam > FAM_FLUX3) return set_error(-2, "flag bit 7 (one launch over the directions) applies to the face fluxes only");
     if (int rc = check_shape(L)) return rc;
     int rc = invalidate_graph(c);
     priv(c)->shape[fam] = L;
-    if (fam <= FAM_FLUX3) priv(c)->flux_all = false;
     return rc;
   }
   static int get_shape(hgpu_ctx* c, int fam, int* bs, int* kc, int* remap) {
@@ -848,7 +860,7 @@ struct GpuBE {
     const LaunchShape& L = priv(c)->shape[fam];
     if (bs) *bs = (int)L.bs;
     if (kc) *kc = (int)L.kc;
-    if (remap) *remap = (int)shape_flags(L);
+    if (remap) *remap = (int)shown_flags(c, fam);
     return 0;
   }
   static void launch_conserved(hgpu_ctx* c, const LaunchShape& L, const Tiling& T, const Box& b, const Ptrs& X,
@@ -936,11 +948,15 @@ struct GpuBE {
     const bool prof = g->prof;
     g->prof = false;
     hipEvent_t e0 = ev(g), e1 = ev(g);
+    const auto set_all = [&](const unsigned* all) { for (int d = 0; d < 3; d++) g->shape[FAM_FLUX1 + d].all = all[d]; };
+    unsigned all_was[3];
+    for (int d = 0; d < 3; d++) all_was[d] = g->shape[FAM_FLUX1 + d].all;
     // fluxes first, so the EMF and update candidates read current face values
     for (int d = 0; d < 3 && !rc; d++) rc |= flux(c, c->X.p, d);
     const unsigned bss[3] = {64, 128, 256}, kcs[4] = {0, 16, 32, 64};
     for (int fam = FAM_FLUX1; fam <= FAM_CONS && !rc; fam++) {
-      const LaunchShape incumbent = g->shape[fam];
+      LaunchShape incumbent = g->shape[fam];
+      incumbent.all = 0;   // a launch per direction is timed here, against the one launch below
       LaunchShape best = incumbent;
       float best_ms = 1e30f;
       auto time_shape_n = [&](const LaunchShape& L, int n) -> float {
@@ -1036,7 +1052,8 @@ struct GpuBE {
       float ms[2] = {1e30f, 1e30f};
       for (int round = 0; round < 2 && !rc; round++)
         for (int all = 0; all < 2; all++) {
-          g->flux_all = all != 0;
+          const unsigned on[3] = {(unsigned)all, (unsigned)all, (unsigned)all};
+          set_all(on);
           rc |= flux_stage(c, c->X.p);
           rc |= hip_check(hipEventRecord(e0, st), "hipEventRecord");
           for (int r = 0; r < 3 * reps; r++) rc |= flux_stage(c, c->X.p);
@@ -1046,8 +1063,11 @@ struct GpuBE {
           rc |= hip_check(hipEventElapsedTime(&t, e0, e1), "hipEventElapsedTime");
           ms[all] = std::min(ms[all], t);
         }
-      g->flux_all = ms[1] < ms[0];
+      for (unsigned& a : all_was) a = ms[1] < ms[0];
     }
+    set_all(all_was);
+    if (report)
+      for (int fam = FAM_FLUX1; fam <= FAM_FLUX3; fam++) report[fam*4 + 2] = shown_flags(c, fam);
     g->pool.push_back(e0);
     g->pool.push_back(e1);
     g->prof = prof;
@@ -1082,7 +1102,7 @@ struct GpuBE {
   // chose shapes per direction
   static int flux_stage(hgpu_ctx* c, const double* src) {
     GpuPriv* g = priv(c);
-    if (g->flux_all && flux_all_possible(c->P)) {
+    if (flux_in_one(c)) {
       Scope s(c, "flux");
       launch_flux_all(c->P, c->X, src, g->stream, c->pn, c->otf_stage);
       return hip_check(hipGetLastError(), "k_flux_all");

@@ -21,6 +21,7 @@ struct LaunchShape {
   unsigned fused = 0;    // conserved update only: 1 = update and inversion in one kernel
   unsigned fpt = 1;      // face fluxes only: faces per thread along the direction (1, 2, 4)
   unsigned stage = 0;    // x3 face fluxes (FP64, PPM, fpt > 1): reconstruction from LDS-staged pencils
+  unsigned all = 0;      // face fluxes: 1: in one launch with the other directions, while they have it too
   unsigned spread = 0;   // 1: small grids are spread over more wavefronts (spread_shape)
   unsigned sp = 0;       // only the first 64 >> sp lanes of a wavefront take a point
 };

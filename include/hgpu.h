@@ -145,12 +145,17 @@ int hgpu_set_graph(hgpu_ctx *ctx, int on);
  * sharing each zone's parabola, bit 6 (family 2, FP64, 2 or 4 faces per
  * thread): the reconstruction reads LDS-staged x3 pencils (each wavefront's
  * zones loaded once, coalesced, into LDS) instead of per-lane stencil loads.
- * The three face-flux directions run in one launch until a shape of families
- * 0-2 is set by hand or hgpu_autotune() finds a launch per direction faster.
+ * Bit 7 (families 0-2): the direction runs in one launch with the other two,
+ * while all three have the bit; the kernel then goes by the size of the grid,
+ * and the rest of the shape is that of the launch per direction in its place.
+ * It is set from the start, cleared by a shape set without it and by
+ * hgpu_autotune() where a launch per direction is faster, and neither shown nor
+ * heeded where the directions cannot share a launch (PPM with a degenerate
+ * direction).
  * hgpu_autotune() times every candidate of families 0-4 on the current state
  * (reps launches each; family 4 as the whole predictor update, split or fused)
  * and keeps the fastest; report (NULL or [5][4]) gets
- * bs, kc, flags, ms per launch.  The state (p, ph), p_gamma, the flags and
+ * bs, kc, flags, ms per launch (families 0-2: of the launch per direction).  The state (p, ph), p_gamma, the flags and
  * the counters are unchanged; the face fluxes hgpu_download_fluxes() returns
  * are then those of the tuning pass.  Results do not depend on the shapes.
  * No counterpart in the reference. */

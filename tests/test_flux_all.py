@@ -37,7 +37,9 @@ def test_one_launch_equals_three(case):
     for per_direction in (False, True):
         H = Harm3D(grid, **kw)
         if per_direction:
-            H.set_launch_shape("flux1", *H.launch_shape("flux1"))
+            bs, kc, flags = H.launch_shape("flux1")
+            assert flags & 128
+            H.set_launch_shape("flux1", bs, kc, flags & ~128)
         H.set_prims(p)
         H.fixup_bounds()
         H.set_time(0.0, grid.dx[0])

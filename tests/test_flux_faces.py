@@ -29,7 +29,8 @@ def test_faces_per_thread(case):
         H = Harm3D(grid, **kw)
         if per_direction:
             for f in ("flux1", "flux2", "flux3"):
-                H.set_launch_shape(f, *H.launch_shape(f))
+                bs, kc, flags = H.launch_shape(f)
+                H.set_launch_shape(f, bs, kc, flags & ~128)
                 assert (H.launch_shape(f)[2] >> 4) & 3 == 1
         H.set_prims(p)
         H.fixup_bounds()

@@ -31,7 +31,7 @@ def test_every_failing_face_counts(case):
         if per_direction:
             for f in ("flux1", "flux2", "flux3"):
                 bs, kc, flags = H.launch_shape(f)
-                H.set_launch_shape(f, bs, kc, flags & 127)
+                H.set_launch_shape(f, bs, kc, flags & ~128)
         H.set_prims(p)
         H.fixup_bounds()
         g, _ = H.geometry()
