@@ -814,7 +814,7 @@ struct GpuBE {
   static unsigned fpt_code(unsigned fpt) { return fpt == 4 ? 2u : (fpt == 2 ? 1u : 0u); }
   static unsigned shape_flags(const LaunchShape& L) {
     return L.remap | (L.order << 1) | (L.occ << 2) | (L.fused << 3) | (fpt_code(L.fpt) << 4) | (L.stage << 6) |
-           (L.all << 7);
+           (L.all << 7) | (L.spread << 8);
   }
   // the flags as a caller sees them: bit 7 only where the directions can share a launch
   static unsigned shown_flags(hgpu_ctx* c, int fam) {
@@ -845,11 +845,13 @@ struct GpuBE {
     L.fpt = 1u << fcode;
     L.stage = ((unsigned)flags >> 6) & 1u;
     L.all = ((unsigned)flags >> 7) & 1u;
-    if (bs < 0 || kc < 0 || flags < 0 || flags > 255 || fcode > 2) return set_error(-2, "bad launch-shape field");
+    L.spread = ((unsigned)flags >> 8) & 1u;
+    if (bs < 0 || kc < 0 || flags < 0 || flags > 511 || fcode > 2) return set_error(-2, "bad launch-shape field");
     if (L.stage && fam != FAM_FLUX3) return set_error(-2, "flag bit 6 (staged pencils) applies to the x3 face fluxes only");
     if (L.fused && fam != FAM_CONS) return set_error(-2, "flag bit 3 (fused update) applies to the conserved update only");
     if (L.fpt > 1 && fam > FAM_FLUX3) return set_error(-2, "flag bits 4-5 (faces per thread) apply to the face fluxes only");
     if (L.all && fam > FAM_FLUX3) return set_error(-2, "flag bit 7 (one launch over the directions) applies to the face fluxes only");
+    if (L.spread && fam != FAM_EMF && fam != FAM_CONS) return set_error(-2, "flag bit 8 (small grids spread) applies to the EMFs and the conserved update only");
     if (int rc = check_shape(L)) return rc;
     int rc = invalidate_graph(c);
     priv(c)->shape[fam] = L;
@@ -982,6 +984,7 @@ struct GpuBE {
         LaunchShape L;
         L.bs = bs; L.kc = kc; L.remap = flags & 1u; L.order = flags >> 1; L.fpt = 1u << fc;
         L.occ = (fc > 0) ? oc : 0u;
+        L.spread = incumbent.spread;
         if (fc == 0 && oc == 1) continue;
         if (check_shape(L)) { g_last_error.clear(); continue; }
         const float ms = time_shape(L);
@@ -1011,6 +1014,7 @@ struct GpuBE {
         for (unsigned bs : bss) for (unsigned kc : kcs) for (unsigned flags = 0; flags < 4; flags++) {
           LaunchShape L;
           L.bs = bs; L.kc = kc; L.remap = flags & 1u; L.order = flags >> 1; L.fused = 1;
+          L.spread = incumbent.spread;
           if (check_shape(L)) { g_last_error.clear(); continue; }
           const float ms = time_shape(L);
           if (rc) break;

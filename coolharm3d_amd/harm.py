@@ -193,7 +193,8 @@ class Harm3D:
         update and inversion fused in one kernel; bits 4-5 (face fluxes, PPM):
         0/1/2 for 1/2/4 faces per thread; bit 6 (x3 face fluxes, FP64): staged
         pencils; bit 7 (face fluxes): one launch over the three directions,
-        while all three have it."""
+        while all three have it; bit 8 (EMFs, conserved update): small grids with
+        short x3 rows spread over more wavefronts."""
         fam = self.FAMILIES.index(family) if isinstance(family, str) else int(family)
         self._chk(self.lib.hgpu_set_launch_shape(self.h, fam, bs, kc, flags), "hgpu_set_launch_shape")
 

@@ -152,6 +152,9 @@ int hgpu_set_graph(hgpu_ctx *ctx, int on);
  * hgpu_autotune() where a launch per direction is faster, and neither shown nor
  * heeded where the directions cannot share a launch (PPM with a degenerate
  * direction).
+ * Bit 8 (families 3 and 4; set from the start): flat tiles of a small grid whose
+ * rows along x3 are shorter than 8 zones take fewer points per wavefront, on
+ * more of the compute units; no other grid is touched by it.
  * hgpu_autotune() times every candidate of families 0-4 on the current state
  * (reps launches each; family 4 as the whole predictor update, split or fused)
  * and keeps the fastest; report (NULL or [5][4]) gets

@@ -6,7 +6,7 @@ from coolharm3d_amd import Harm3D, balsara1, balsara1_grid, torus, torus_grid
 
 pytestmark = pytest.mark.gpu
 
-ONE_LAUNCH = 128
+ONE_LAUNCH, SPREAD = 128, 256
 
 
 def _context(n, **kw):
@@ -63,3 +63,16 @@ def test_autotuner_reports_the_launch_that_runs(n):
     assert all(ones) or not any(ones)
     assert [H.launch_shape(f) for f in FLUXES] == [rep[f][:3] for f in FLUXES]
     assert _flux_launches(H) == (2 if ones[0] else 6)
+
+
+def test_autotuner_keeps_the_spread():
+    H = _context(1024)
+    before = {f: H.launch_shape(f) for f in ("emf", "conserved")}
+    assert all(s[2] & SPREAD for s in before.values())
+    rep = H.autotune(reps=1)
+    for f in before:
+        assert rep[f][2] & SPREAD and H.launch_shape(f)[2] & SPREAD
+        H.set_launch_shape(f, *before[f])
+        assert H.launch_shape(f) == before[f]
+    with pytest.raises(RuntimeError):
+        H.set_launch_shape("flux1", 256, 0, SPREAD)

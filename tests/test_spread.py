@@ -27,7 +27,8 @@ def test_spread_equals_full_wavefronts(case):
         if full:
             for f in ("flux1", "emf", "conserved"):
                 bs, kc, flags = H.launch_shape(f)
-                H.set_launch_shape(f, bs, kc, flags & ~128)   # one launch over the directions off
+                assert f == "flux1" or flags & 256
+                H.set_launch_shape(f, bs, kc, flags & ~(128 | 256))   # neither one launch nor spread
         H.set_prims(p)
         H.fixup_bounds()
         H.set_time(0.0, min(grid.dx[0], 1e-7) if isinstance(n, int) else grid.dx[0])
