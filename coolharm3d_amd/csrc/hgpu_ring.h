@@ -126,16 +126,17 @@ hipError_t xfer_to_host(XferRing& R, hipStream_t st, void* host, size_t bytes, F
   for (auto& x : copied) x.store(0);
   std::atomic<int> err{(int)hipSuccess};
   // The workers sleep until the first chunk is there: work queued on the stream
-  // before the copy may take long, and the caller alone waits for that.
+  // before the copy may take long, and the caller alone waits for that.  (The caller
+  // only keeps the chunks filled: taking some itself made 93 MB 0.9 ms slower.)
   std::mutex gate;
   std::condition_variable opened;
   bool open = false;
   const auto worker = [&]() {
+    if (hipSetDevice(R.device) != hipSuccess) err = (int)hipErrorInvalidDevice;
     {
       std::unique_lock<std::mutex> l(gate);
       opened.wait(l, [&]() { return open; });
     }
-    if (hipSetDevice(R.device) != hipSuccess) err = (int)hipErrorInvalidDevice;
     for (;;) {
       const long long c = next.fetch_add(1);
       if (c >= n) return;
