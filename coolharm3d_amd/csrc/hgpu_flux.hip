@@ -278,7 +278,7 @@ struct FluxAll {
   unsigned per, nblocks;     // workgroups per slab, in all
   unsigned remap;            // XCD-contiguous slabs
 };
-static FluxAll make_flux_all(const Params& P, unsigned F, LaunchShape& L) {
+static FluxAll make_flux_all(const Params& P, unsigned F, LaunchShape& L, unsigned simds) {
   FluxAll A;
   long long points = 0;
   bool small = false;
@@ -289,7 +289,7 @@ static FluxAll make_flux_all(const Params& P, unsigned F, LaunchShape& L) {
     A.bg[d].hi[d] = b.lo[d] + (b.hi[d] - b.lo[d] + (int)F) / (int)F - 1;
     points += A.bg[d].count();
   }
-  L = spread_shape(L, A.bg[0], points);
+  L = spread_shape(L, A.bg[0], points, simds);
   for (int d = 0; d < 3; d++) {
     A.T[d] = make_tiling(A.bg[d], L);
     small = small || A.T[d].pp > 1;
@@ -470,20 +470,20 @@ bool flux_all_possible(const Params& P) {
 }
 // Faces per thread.  A group's zones are reconstructed once for the whole group, so
 // more faces per thread are less work, in fewer and longer wavefronts.  Up to one
-// wavefront per SIMD a launch is one wavefront's chain: one face (24x24x16, a step's
-// fluxes: FP64 0.045 -> 0.027 ms, mixed 0.037 -> 0.026; at 48x48x32, 3900 wavefronts
+// wavefront per SIMD (simds: the device's, 1024 where the figures were taken) a
+// launch is one wavefront's chain: one face (24x24x16, a step's fluxes: FP64 0.045 -> 0.027 ms, mixed 0.037 -> 0.026; at 48x48x32, 3900 wavefronts
 // of single faces, mixed 0.046 and 0.044 but a slower step).  Once groups of 4 fill
 // the FP32 solve's 4 wavefronts per SIMD, 4 faces: mixed 192x192x128 1.05 -> 0.885 ms,
 // 96x96x64 0.140 -> 0.136, binary disk 120x64x160 0.343 -> 0.303; 67x45x33, which
 // does not, 0.051 -> 0.057.  FP64 groups of 4 take 254 registers, two wavefronts
 // per SIMD, and gain nothing (1.61 ms at 192x192x128; disk 0.67 -> 0.94).
-constexpr long long ONE_FACE_WAVES = 1024, FOUR_FACE_WAVES = 4096;
-static unsigned flux_all_faces(const Params& P, long long faces) {
+static unsigned flux_all_faces(const Params& P, long long faces, unsigned simds) {
   if (!flux_all_multi(P)) return 1;
-  if (faces <= 64 * ONE_FACE_WAVES && !P.otf) return 1;
-  return (P.mixed && faces >= 4 * 64 * FOUR_FACE_WAVES) ? 4 : 2;
+  if (faces <= 64ll * simds && !P.otf) return 1;
+  return (P.mixed && faces >= 4 * 64ll * (4 * simds)) ? 4 : 2;
 }
-void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStream_t st, const PnGrid& G, int lvl) {
+void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStream_t st, const PnGrid& G, int lvl,
+                     unsigned simds) {
   // Flat tiles of 256 in dispatch order: round-robin over the XCDs, so that
   // all of them work on one slab (1.62 ms a step on the 192x192x128 torus
   // against 1.70 with a contiguous range of slabs per XCD; tiles of 64 run into
@@ -492,9 +492,9 @@ void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStrea
   L.remap = 0;
   long long faces = 0;
   for (int d = 0; d < 3; d++) faces += flux_box(P, d).count();
-  const unsigned F = flux_all_faces(P, faces);
+  const unsigned F = flux_all_faces(P, faces, simds);
   L.spread = F == 1;
-  const FluxAll A = make_flux_all(P, F, L);
+  const FluxAll A = make_flux_all(P, F, L, simds);
   const dim3 grid(A.nblocks), blk(L.bs);
   if (F > 1) {
     if (P.otf) {

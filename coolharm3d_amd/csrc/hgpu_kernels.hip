@@ -1108,7 +1108,7 @@ struct GpuBE {
     GpuPriv* g = priv(c);
     if (flux_in_one(c)) {
       Scope s(c, "flux");
-      launch_flux_all(c->P, c->X, src, g->stream, c->pn, c->otf_stage);
+      launch_flux_all(c->P, c->X, src, g->stream, c->pn, c->otf_stage, g->simds);
       return hip_check(hipGetLastError(), "k_flux_all");
     }
     int rc = 0;
@@ -1123,7 +1123,7 @@ struct GpuBE {
   static int emf(hgpu_ctx* c) {
     Box b = edge_box(c->P);
     Scope s(c, "emf");
-    const Tiling T = make_tiling(b, spread_shape(priv(c)->shape[FAM_EMF], b, b.count()));
+    const Tiling T = make_tiling(b, spread_shape(priv(c)->shape[FAM_EMF], b, b.count(), priv(c)->simds));
     if (c->P.mixed) hipLaunchKernelGGL(k_emf_mixed, dim3(T.nblocks + 1), dim3(T.bs), 0, priv(c)->stream, c->P, c->X, b, T);
     // The limiters' form: as long as the edges are one round of wavefronts (5 per
     // SIMD) the launch is one wavefront's chain, shorter by selects (24x24x16: 7.0
@@ -1147,7 +1147,7 @@ struct GpuBE {
     Box b = interior_box(c->P);
     Scope s(c, "update");
     LaunchShape L = priv(c)->shape[FAM_CONS];
-    if (L.fused || c->P.otf) L = spread_shape(L, b, b.count());
+    if (L.fused || c->P.otf) L = spread_shape(L, b, b.count(), priv(c)->simds);
     const Tiling T = make_tiling(b, L);
     const Tiling T2 = make_tiling(b, priv(c)->shape[FAM_INV]);
     if ((long long)T.nblocks * (T.bs / 64) > c->mpart_cap) return set_error(-3, "update grid exceeds the M_tot parts buffer");

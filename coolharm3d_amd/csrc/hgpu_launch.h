@@ -148,16 +148,15 @@ struct Tiling {
 // ones in x1 and x2): the 64 lanes of a wavefront touch a line each with every
 // load, about 60 loads one after the other on one compute unit, and most compute
 // units have no wavefront at all.  Workgroups of one wavefront with 64 >> sp
-// points each spread them, as long as that makes no more than SPREAD_WAVES
-// wavefronts.  1024-zone shock tube: update 21 -> 10 us a launch, step 0.097 ->
+// points each spread them, as long as that makes no more than one wavefront for
+// two SIMDs (512 on the 256-CU part).  1024-zone shock tube: update 21 -> 10 us a launch, step 0.097 ->
 // 0.074 ms (0.075 up to 1024 wavefronts, 0.081 up to 2048, where the dispatch of
 // the workgroups takes over).  Longer rows share their lines between lanes and lose:
 // 24x24x16, spread twofold 0.170 -> 0.172 ms, fourfold 0.187.
-constexpr long long SPREAD_WAVES = 512;
-static inline LaunchShape spread_shape(LaunchShape L, const Box& b, long long points) {
+static inline LaunchShape spread_shape(LaunchShape L, const Box& b, long long points, unsigned simds) {
   if (!L.spread || L.kc || b.hi[2] - b.lo[2] + 1 >= 8) return L;
   const long long waves = (points + 63) / 64;
-  while (L.sp < 4 && (waves << (L.sp + 1)) <= SPREAD_WAVES) L.sp++;
+  while (L.sp < 4 && (waves << (L.sp + 1)) <= simds / 2) L.sp++;
   if (L.sp) L.bs = 64;
   return L;
 }
@@ -267,8 +266,9 @@ __device__ __forceinline__ PnOrbit orbit_load(const PnOrbit* p) {
 void launch_flux_dir(int d, const Params& P, const Ptrs& X, const LaunchShape& L, const double* src, hipStream_t st,
                      const PnGrid& G, int lvl);
 // The three directions in one launch (flux_all_possible()), 1, 2 or 4 faces per
-// thread by the grid's size
+// thread by the grid's size and the device's SIMDs
 bool flux_all_possible(const Params& P);
-void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStream_t st, const PnGrid& G, int lvl);
+void launch_flux_all(const Params& P, const Ptrs& X, const double* src, hipStream_t st, const PnGrid& G, int lvl,
+                     unsigned simds);
 
 }  // namespace hgpu
