@@ -2,6 +2,9 @@
 pattern, Minkowski) against the general ones: the same state, flags and counters
 bit for bit.  The general kernels are reached with records whose zero pattern is
 broken by the smallest subnormal, which changes no sum that is not zero."""
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -50,6 +53,52 @@ CASES = [
     dict(problem="shock", n=128),
     dict(problem="shock", n=128, precision="mixed"),
 ]
+
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "coolharm3d_amd", "csrc")
+GK_GEN, GK_FLAT, GK_KS = 0, 1, 2
+KIND = r"""
+#include <cstdio>
+#include <vector>
+#include "hgpu_types.h"
+int main(int, char** a) {
+  FILE* f = fopen(a[1], "rb");
+  fseek(f, 0, SEEK_END);
+  const long long n = ftell(f) / (long long)sizeof(hgpu::Geom);
+  rewind(f);
+  std::vector<hgpu::Geom> r(n);
+  if (fread(r.data(), sizeof(hgpu::Geom), n, f) != (size_t)n) return 1;
+  printf("%d\n", hgpu::metric_structure(r.data(), n, a[2][0] == '1'));
+}
+"""
+
+
+def test_structure_found(tmp_path):
+    """The contexts compared here do run the kernels of the structure that they are
+    named for: what metric_structure() finds on their records, and on broken ones."""
+    src, exe, rec = tmp_path / "kind.cpp", tmp_path / "kind", tmp_path / "records"
+    src.write_text(KIND)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + CSRC, "-o",
+                    str(exe), str(src)], check=True)
+
+    def kind(g, flat_metric):
+        np.ascontiguousarray(g).tofile(rec)
+        return int(subprocess.run([str(exe), str(rec), "1" if flat_metric else "0"], capture_output=True, text=True,
+                                  check=True).stdout)
+    for coords in ("mks", "diag3"):
+        g, _ = Harm3D(torus_grid(13, 12, 8, coords=coords), hostcheck=True).geometry()
+        assert kind(g, False) == GK_KS
+        for at in (GCON + 2, GCOV + 6, 35 + 1, 38 + 2):       # g^{t2}, g_{12}, beta^2, n^2 of one record
+            b = g.copy()
+            b[len(b) // 2, at] = 5e-324
+            assert kind(b, False) == GK_GEN
+        b = g.copy()
+        b[3, GCOV + 5] = np.nan
+        assert kind(b, False) == GK_GEN
+    m, _ = Harm3D(balsara1_grid(64), hostcheck=True).geometry()
+    assert kind(m, True) == GK_FLAT and kind(m, False) != GK_FLAT
+    m[0, 32] = 1.0 + 2.0 ** -52
+    assert kind(m, True) != GK_FLAT
 
 
 @pytest.mark.parametrize("case", CASES, ids=str)
