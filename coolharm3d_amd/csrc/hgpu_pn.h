@@ -28,7 +28,8 @@
 // * The metric's first derivatives, time derivatives of the moving metric
 //   included, are closed-form (pn_metric_dg_coords()); the connection Gamma^a_bc
 //   is formed from them.  The orbit's time derivatives come from forward-mode
-//   numbers (ad::Dual), once per time level.
+//   numbers (Dual4), once per time level.  The functions of the metric itself are
+//   called with T = double.
 #pragma once
 #include "hgpu_types.h"
 #include <math.h>
@@ -36,34 +37,53 @@
 namespace hgpu {
 
 // ---------------------------------------------------------------------------
-// forward-mode numbers (value and derivative in t) for the orbit; their functions
-// are found by argument-dependent lookup, so double arguments keep the libm functions
+// forward-mode numbers for the orbit's derivatives in t (the others stay zero and
+// cost nothing once compiled); their functions are found by argument-dependent
+// lookup, so double arguments keep the libm functions
 namespace ad {
-struct Dual {
-  double v, d;
+struct Dual4 {
+  double v, d[4];
 };
-HD Dual dc(double v) { return {v, 0.}; }
-HD Dual dvar(double v) { return {v, 1.}; }
-HD Dual operator+(const Dual& a, const Dual& b) { return {a.v + b.v, a.d + b.d}; }
-HD Dual operator-(const Dual& a, const Dual& b) { return {a.v - b.v, a.d - b.d}; }
-HD Dual operator-(const Dual& a) { return {-a.v, -a.d}; }
-HD Dual operator*(const Dual& a, const Dual& b) { return {a.v * b.v, a.d * b.v + a.v * b.d}; }
-HD Dual operator/(const Dual& a, const Dual& b) {
-  const double ib = 1. / b.v, q = a.v * ib;
-  return {q, (a.d - q * b.d) * ib};
+HD Dual4 dc(double v) { Dual4 r; r.v = v; r.d[0] = r.d[1] = r.d[2] = r.d[3] = 0.; return r; }
+HD Dual4 dvar(double v, int k) { Dual4 r = dc(v); r.d[k] = 1.; return r; }
+HD Dual4 operator+(const Dual4& a, const Dual4& b) {
+  Dual4 r; r.v = a.v + b.v; for (int k = 0; k < 4; k++) r.d[k] = a.d[k] + b.d[k]; return r;
 }
-HD Dual operator+(const Dual& a, double s) { return {a.v + s, a.d}; }
-HD Dual operator+(double s, const Dual& a) { return a + s; }
-HD Dual operator-(const Dual& a, double s) { return {a.v - s, a.d}; }
-HD Dual operator-(double s, const Dual& a) { return (-a) + s; }
-HD Dual operator*(const Dual& a, double s) { return {a.v * s, a.d * s}; }
-HD Dual operator*(double s, const Dual& a) { return a * s; }
-HD Dual operator/(double s, const Dual& a) { return dc(s) / a; }
-HD Dual chain(const Dual& a, double f, double df) { return {f, df * a.d}; }
-HD Dual sin(const Dual& a) { return chain(a, ::sin(a.v), ::cos(a.v)); }
-HD Dual cos(const Dual& a) { return chain(a, ::cos(a.v), -::sin(a.v)); }
-HD Dual pow(const Dual& a, double p) { const double f = ::pow(a.v, p); return chain(a, f, p * f / a.v); }
+HD Dual4 operator-(const Dual4& a, const Dual4& b) {
+  Dual4 r; r.v = a.v - b.v; for (int k = 0; k < 4; k++) r.d[k] = a.d[k] - b.d[k]; return r;
+}
+HD Dual4 operator-(const Dual4& a) {
+  Dual4 r; r.v = -a.v; for (int k = 0; k < 4; k++) r.d[k] = -a.d[k]; return r;
+}
+HD Dual4 operator*(const Dual4& a, const Dual4& b) {
+  Dual4 r; r.v = a.v * b.v; for (int k = 0; k < 4; k++) r.d[k] = a.d[k] * b.v + a.v * b.d[k]; return r;
+}
+HD Dual4 operator/(const Dual4& a, const Dual4& b) {
+  const double ib = 1. / b.v;
+  Dual4 r; r.v = a.v * ib;
+  for (int k = 0; k < 4; k++) r.d[k] = (a.d[k] - r.v * b.d[k]) * ib;
+  return r;
+}
+HD Dual4 operator+(const Dual4& a, double s) { Dual4 r = a; r.v += s; return r; }
+HD Dual4 operator+(double s, const Dual4& a) { return a + s; }
+HD Dual4 operator-(const Dual4& a, double s) { Dual4 r = a; r.v -= s; return r; }
+HD Dual4 operator-(double s, const Dual4& a) { return (-a) + s; }
+HD Dual4 operator*(const Dual4& a, double s) {
+  Dual4 r; r.v = a.v * s; for (int k = 0; k < 4; k++) r.d[k] = a.d[k] * s; return r;
+}
+HD Dual4 operator*(double s, const Dual4& a) { return a * s; }
+HD Dual4 operator/(const Dual4& a, double s) { return a * (1. / s); }
+HD Dual4 operator/(double s, const Dual4& a) { return dc(s) / a; }
+HD Dual4 chain(const Dual4& a, double f, double df) {
+  Dual4 r; r.v = f; for (int k = 0; k < 4; k++) r.d[k] = df * a.d[k]; return r;
+}
+HD Dual4 sin(const Dual4& a) { return chain(a, ::sin(a.v), ::cos(a.v)); }
+HD Dual4 cos(const Dual4& a) { return chain(a, ::cos(a.v), -::sin(a.v)); }
+HD Dual4 pow(const Dual4& a, double p) { const double f = ::pow(a.v, p); return chain(a, f, p * f / a.v); }
 }  // namespace ad
+using ad::Dual4;
+using ad::dc;
+using ad::dvar;
 
 // seesaw(x, 0, 1) of the theta coordinate, src/coord.c:4316-4324: ghost zones
 // beyond a pole reflect back into [0, 1]
@@ -116,41 +136,49 @@ struct PnOrbit {
 
 HD void pn_orbit_at(const PnBinary& B, double t, PnOrbit* o) {
   pn_orbit(B, t, o->y[0], o->y[1], o->v[0], o->v[1]);
-  ad::Dual yd[2][3], vd[2][3];
-  pn_orbit(B, ad::dvar(t), yd[0], yd[1], vd[0], vd[1]);
+  Dual4 yd[2][3], vd[2][3];
+  pn_orbit(B, dvar(t, 0), yd[0], yd[1], vd[0], vd[1]);
   for (int a = 0; a < 2; a++)
-    for (int i = 0; i < 3; i++) { o->ydot[a][i] = yd[a][i].d; o->vdot[a][i] = vd[a][i].d; }
+    for (int i = 0; i < 3; i++) { o->ydot[a][i] = yd[a][i].d[0]; o->vdot[a][i] = vd[a][i].d[0]; }
 }
 
 // Potentials of the 1PN near-zone metric at Cartesian point x for holes at y
 // moving with v: the Newtonian U, the 1PN V and the vector potential V_i, so
 // that g00 = -1 + 2V - 2U^2, g0i = -4 V_i, gij = (1 + 2U) delta_ij.
-HD void pn_potentials_yv(const PnBinary& B, const double y[2][3], const double v[2][3], const double x[3],
-                         double& U, double& V, double Vi[3]) {
+template <class T>
+HD void pn_potentials_yv(const PnBinary& B, const T y[2][3], const T v[2][3], const T x[3], T& U, T& V, T Vi[3]) {
   const double m[2] = {B.m1, B.m2};
-  double r[2], nv[2], vsq[2];
+  T r[2], nv[2], vsq[2];
   for (int a = 0; a < 2; a++) {
-    const double dx = x[0] - y[a][0], dy = x[1] - y[a][1], dz = x[2] - y[a][2];
+    const T dx = x[0] - y[a][0], dy = x[1] - y[a][1], dz = x[2] - y[a][2];
     r[a] = sqrt(dx * dx + dy * dy + dz * dz);
     nv[a] = (dx * v[a][0] + dy * v[a][1] + dz * v[a][2]) / r[a];
     vsq[a] = v[a][0] * v[a][0] + v[a][1] * v[a][1] + v[a][2] * v[a][2];
   }
-  const double ex = y[0][0] - y[1][0], ey = y[0][1] - y[1][1], ez = y[0][2] - y[1][2];
-  const double r12 = sqrt(ex * ex + ey * ey + ez * ez);
-  const double r12_3 = r12 * r12 * r12;
-  U = 0.;
-  V = 0.;
+  const T ex = y[0][0] - y[1][0], ey = y[0][1] - y[1][1], ez = y[0][2] - y[1][2];
+  const T r12 = sqrt(ex * ex + ey * ey + ez * ez);
+  const T r12_3 = r12 * r12 * r12;
+  U = r12 * 0.;
+  V = r12 * 0.;
   for (int a = 0; a < 2; a++) {
     const int b = 1 - a;
-    const double mr = m[a] / r[a];
+    const T mr = m[a] / r[a];
     U = U + mr;
     V = V + mr * (1. + 2. * vsq[a] - 0.5 * nv[a] * nv[a]) - m[a] * m[b] / (r[a] * r12)
           + (m[a] * m[b] / 4.) * (r[b] * r[b] - r[a] * r[a] - r12 * r12) / (r[a] * r12_3);
   }
   for (int i = 0; i < 3; i++) {
-    Vi[i] = 0.;
+    Vi[i] = r12 * 0.;
     for (int a = 0; a < 2; a++) Vi[i] = Vi[i] + m[a] * v[a][i] / r[a];
   }
+}
+
+// The potentials at Cartesian point x, time t.
+template <class T>
+HD void pn_potentials(const PnBinary& B, const T& t, const T x[3], T& U, T& V, T Vi[3]) {
+  T y[2][3], v[2][3];
+  pn_orbit(B, t, y[0], y[1], v[0], v[1]);
+  pn_potentials_yv<T>(B, y, v, x, U, V, Vi);
 }
 
 // Metric in the numerical coordinates (t, X1, X2, X3) of the spherical grid.
@@ -159,25 +187,29 @@ HD void pn_potentials_yv(const PnBinary& B, const double y[2][3], const double v
 //   g_tt = g00,  g_tn = -4 V_i J^i_n,
 //   g_11 = A r'^2,  g_22 = A (r theta')^2,  g_33 = A (r sin theta)^2,  A = 1 + 2U,
 // with no other spatial components (r' = dr/dX1, theta' = dtheta/dX2).
+// pot(x, U, V, Vi) evaluates the potentials at the Cartesian point x.
 // The coordinate functions of the spherical map, one numerical coordinate
 // each: r and dr/dX1 of X1; sin, cos of theta and dtheta/dX2 of X2; sin, cos
 // of phi = X3.
+template <class T>
 struct PnCoords {
-  double r, dr, st, ct, dth, sp, cp;
+  T r, dr, st, ct, dth, sp, cp;
 };
-HD void pn_coord1(const PnBinary& B, double X1, double* r, double* dr) {
-  const double er = exp(X1);
+template <class T>
+HD void pn_coord1(const PnBinary& B, const T& X1, T* r, T* dr) {
+  const T er = exp(X1);
   *r = er + B.R0;
   *dr = er;
 }
-HD void pn_coord2(const PnBinary& B, double X2, double* st, double* ct, double* dth) {
+template <class T>
+HD void pn_coord2(const PnBinary& B, const T& X2, T* st, T* ct, T* dth) {
   // theta from the reflected X2, as x_of_xp() and dx_dxp_calc() form it
   // (src/coord.c:240-382): COORD_DIAGONAL's derivative from X2 itself,
   // COORD_DIAGONAL3's from f = 2 seesaw(X2) - 1 (src/coord.c:270-276, :468-472)
-  const double X2s = X2 + (seesaw_unit(X2) - X2);
-  double th;
+  const T X2s = X2 + (seesaw_unit(X2) - X2);
+  T th;
   if (B.coords == 4) {
-    const double f = 2. * X2s - 1.;
+    const T f = 2. * X2s - 1.;
     th = 0.5 * M_PI * (1. + B.h_slope * f + B.diag3_factor * pow(f, (double)B.diag3_exponent));
     *dth = M_PI * (B.h_slope + (B.diag3_exponent * B.diag3_factor) * pow(f, (double)(B.diag3_exponent - 1)));
   } else {
@@ -197,24 +229,26 @@ HD double pn_ddtheta(const PnBinary& B, double X2) {
   }
   return -4. * M_PI * M_PI * B.h_slope * ::sin(2. * M_PI * X2);
 }
-HD void pn_coord3(double X3, double* sp, double* cp) {
+template <class T>
+HD void pn_coord3(const T& X3, T* sp, T* cp) {
   *sp = sin(X3);
   *cp = cos(X3);
 }
 
-// The metric from the coordinate functions at a time level whose orbit is known
-HD void pn_gcov_from_coords(const PnBinary& B, const PnOrbit& o, const PnCoords& C, double g[4][4]) {
-  const double r = C.r, dr = C.dr, st = C.st, ct = C.ct, dth = C.dth, sp = C.sp, cp = C.cp;
-  const double rs = r * st;
-  const double x[3] = {rs * cp, rs * sp, r * ct};
-  double U, V, Vi[3];
-  pn_potentials_yv(B, o.y, o.v, x, U, V, Vi);
+// The metric from the coordinate functions; zero is a zero of type T.
+template <class T, class Pot>
+HD void pn_gcov_from_coords(const PnCoords<T>& C, const T& zero, T g[4][4], const Pot& pot) {
+  const T r = C.r, dr = C.dr, st = C.st, ct = C.ct, dth = C.dth, sp = C.sp, cp = C.cp;
+  const T rs = r * st;
+  T x[3] = {rs * cp, rs * sp, r * ct};
+  T U, V, Vi[3];
+  pot(x, U, V, Vi);
   // columns n = 1..3 of J = d(x, y, z)/d(X1, X2, X3)
-  const double J1[3] = {st * cp * dr, st * sp * dr, ct * dr};
-  const double rdth = r * dth;
-  const double J2[3] = {ct * cp * rdth, ct * sp * rdth, -st * rdth};
-  const double J3[2] = {-rs * sp, rs * cp};
-  const double A = 1. + 2. * U;
+  const T J1[3] = {st * cp * dr, st * sp * dr, ct * dr};
+  const T rdth = r * dth;
+  const T J2[3] = {ct * cp * rdth, ct * sp * rdth, -st * rdth};
+  const T J3[3] = {-rs * sp, rs * cp, zero};
+  const T A = 1. + 2. * U;
   g[0][0] = -1. + 2. * V - 2. * U * U;
   g[0][1] = g[1][0] = -4. * (Vi[0] * J1[0] + Vi[1] * J1[1] + Vi[2] * J1[2]);
   g[0][2] = g[2][0] = -4. * (Vi[0] * J2[0] + Vi[1] * J2[1] + Vi[2] * J2[2]);
@@ -222,16 +256,28 @@ HD void pn_gcov_from_coords(const PnBinary& B, const PnOrbit& o, const PnCoords&
   g[1][1] = A * dr * dr;
   g[2][2] = A * rdth * rdth;
   g[3][3] = A * rs * rs;
-  g[1][2] = g[2][1] = g[1][3] = g[3][1] = g[2][3] = g[3][2] = 0.;
+  g[1][2] = g[2][1] = g[1][3] = g[3][1] = g[2][3] = g[3][2] = zero;
 }
 
-// The same at numerical coordinates.
-HD void pn_gcov_num(const PnBinary& B, const PnOrbit& o, double X1, double X2, double X3, double g[4][4]) {
-  PnCoords C;
+template <class T, class Pot>
+HD void pn_gcov_num_pot(const PnBinary& B, const T& X1, const T& X2, const T& X3, T g[4][4], const Pot& pot) {
+  PnCoords<T> C;
   pn_coord1(B, X1, &C.r, &C.dr);
   pn_coord2(B, X2, &C.st, &C.ct, &C.dth);
   pn_coord3(X3, &C.sp, &C.cp);
-  pn_gcov_from_coords(B, o, C, g);
+  pn_gcov_from_coords(C, X1 * 0., g, pot);
+}
+
+template <class T>
+HD void pn_gcov_num(const PnBinary& B, const T& t, const T& X1, const T& X2, const T& X3, T g[4][4]) {
+  pn_gcov_num_pot(B, X1, X2, X3, g, [&](const T x[3], T& U, T& V, T Vi[3]) { pn_potentials(B, t, x, U, V, Vi); });
+}
+
+// The same at a time level whose orbit is known.
+HD void pn_gcov_num_orb(const PnBinary& B, const PnOrbit& o, double X1, double X2, double X3, double g[4][4]) {
+  pn_gcov_num_pot(B, X1, X2, X3, g, [&](const double x[3], double& U, double& V, double Vi[3]) {
+    pn_potentials_yv<double>(B, o.y, o.v, x, U, V, Vi);
+  });
 }
 
 // Components of the numerical metric that are not identically zero (the
@@ -254,7 +300,7 @@ constexpr int PN_NDG = 4 * PN_NG;   // dg[nu * PN_NG + m] = d g_{ab(m)} / dx^nu,
 // operation, most of them zeros) took ~2500 FP64 operations and 200 registers
 // for the 28 values; this takes ~350.  Source kernel of the binary disk,
 // 120x64x160: 125 -> 76 us a stage (capped at 3 wavefronts per SIMD: the same).
-HD void pn_metric_dg_coords(const PnBinary& B, const PnOrbit& o, const PnCoords& C, double ddth, double* dg) {
+HD void pn_metric_dg_coords(const PnBinary& B, const PnOrbit& o, const PnCoords<double>& C, double ddth, double* dg) {
   const double er[3] = {C.st*C.cp, C.st*C.sp, C.ct}, et[3] = {C.ct*C.cp, C.ct*C.sp, -C.st}, ep[2] = {-C.sp, C.cp};
   const double R = C.r*C.dth, rs = C.r*C.st;
   const double sc[3] = {C.dr, R, rs};          // |J_n|
@@ -353,7 +399,7 @@ HD void pn_metric_dg_coords(const PnBinary& B, const PnOrbit& o, const PnCoords&
 
 // The same at numerical coordinates.
 HD void pn_metric_dg(const PnBinary& B, const PnOrbit& o, double X1, double X2, double X3, double* dg) {
-  PnCoords C;
+  PnCoords<double> C;
   pn_coord1(B, X1, &C.r, &C.dr);
   pn_coord2(B, X2, &C.st, &C.ct, &C.dth);
   pn_coord3(X3, &C.sp, &C.cp);
@@ -419,16 +465,17 @@ HD void pn_geom_from_gcov(const double g[4][4], Geom* G) {
   G->beta[1] = -G->gcon[0][2] / G->gcon[0][0];
   G->beta[2] = -G->gcon[0][3] / G->gcon[0][0];
 }
-// The record at a time level whose orbit is known
-HD void pn_geom_orb(const PnBinary& B, const PnOrbit& o, double X1, double X2, double X3, Geom* G) {
+HD void pn_geom(const PnBinary& B, double t, double X1, double X2, double X3, Geom* G) {
   double g[4][4];
-  pn_gcov_num(B, o, X1, X2, X3, g);
+  pn_gcov_num(B, t, X1, X2, X3, g);
   pn_geom_from_gcov(g, G);
 }
-HD void pn_geom(const PnBinary& B, double t, double X1, double X2, double X3, Geom* G) {
-  PnOrbit o;   // positions and velocities, all that the metric reads
-  pn_orbit(B, t, o.y[0], o.y[1], o.v[0], o.v[1]);
-  pn_geom_orb(B, o, X1, X2, X3, G);
+// The record at a time level whose orbit is known: the same values as
+// pn_geom() at that level's time.
+HD void pn_geom_orb(const PnBinary& B, const PnOrbit& o, double X1, double X2, double X3, Geom* G) {
+  double g[4][4];
+  pn_gcov_num_orb(B, o, X1, X2, X3, g);
+  pn_geom_from_gcov(g, G);
 }
 
 // Binary and grid of a context whose metric is the binary's: the numerical
@@ -444,7 +491,7 @@ HD void zone_X(const Params& P, const PnGrid& G, int i, int j, int k, int pos, d
 }
 // Coordinate functions of zone (i,j,k) at position pos from the tables (the
 // values pn_gcov_num() forms from the coordinates).
-HD void pn_zone_coords(const Params& P, const PnGrid& G, int i, int j, int k, int pos, PnCoords& C) {
+HD void pn_zone_coords(const Params& P, const PnGrid& G, int i, int j, int k, int pos, PnCoords<double>& C) {
   const int h1 = (pos == FACE1 || pos == CORN) ? 0 : 1;
   const int h2 = (pos == FACE2 || pos == CORN) ? 0 : 1;
   const int h3 = (pos == FACE3 || pos == CORN) ? 0 : 1;
@@ -482,7 +529,7 @@ HD long long pn_tab_entries(const Params& P) { return 2LL * (P.n1t + P.n2t + P.n
 // Metric derivatives at the centre of zone (i,j,k) and the level of orbit o, from
 // the tables
 HD void pn_zone_dg(const Params& P, const PnGrid& G, const PnOrbit& o, int i, int j, int k, double* dg) {
-  PnCoords C;
+  PnCoords<double> C;
   pn_zone_coords(P, G, i, j, k, CENT, C);
   pn_metric_dg_coords(G.B, o, C, G.tab[4 * P.n1t + 4 * (P.n2t + j) + 3], dg);
 }
@@ -493,7 +540,7 @@ HD void pn_zone_dg(const Params& P, const PnGrid& G, const PnOrbit& o, int i, in
 // S = g_tt - sum b_i q_i = -alpha^2 and 1 + S = 2V - 2U^2 - sum b_i q_i.
 HD void pn_zone_geomf(const Params& P, const PnGrid& G, const PnOrbit& o, int i, int j, int k, int pos,
                       GeomF* out) {
-  PnCoords C;
+  PnCoords<double> C;
   pn_zone_coords(P, G, i, j, k, pos, C);
   const float r = (float)C.r, dr = (float)C.dr, st = (float)C.st, ct = (float)C.ct, dth = (float)C.dth;
   const float sp = (float)C.sp, cp = (float)C.cp;
@@ -568,10 +615,12 @@ HD void pn_zone_geom(const Params& P, const PnGrid& G, const PnOrbit& o, int i, 
     pn_geom_orb(G.B, o, X[1], X[2], X[3], out);
     return;
   }
-  PnCoords C;
+  PnCoords<double> C;
   pn_zone_coords(P, G, i, j, k, pos, C);
   double g[4][4];
-  pn_gcov_from_coords(G.B, o, C, g);
+  pn_gcov_from_coords(C, 0., g, [&](const double x[3], double& U, double& V, double Vi[3]) {
+    pn_potentials_yv<double>(G.B, o.y, o.v, x, U, V, Vi);
+  });
   pn_geom_from_gcov(g, out);
 }
 
@@ -583,7 +632,7 @@ HD void pn_conn(const PnBinary& B, double t, double X1, double X2, double X3, do
   PnOrbit o;
   pn_orbit_at(B, t, &o);
   double gv[4][4], gi[4][4], dg[PN_NDG];
-  pn_gcov_num(B, o, X1, X2, X3, gv);
+  pn_gcov_num_orb(B, o, X1, X2, X3, gv);
   pn_metric_dg(B, o, X1, X2, X3, dg);
   invert4(gv, gi);
   double d[4][4][4];   // d[c][a][b] = d g_ab / dx^c
