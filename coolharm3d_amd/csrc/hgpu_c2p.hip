@@ -247,8 +247,9 @@ __global__ __launch_bounds__(CB) void k_c2p_guess(C2pArgs A, const float* __rest
 }
 
 // First pass; with MLP the network's outputs come from k_c2p_guess.  Bound by
-// FP64 issue (2^24 zones move 2.6 GB in 1.30 ms; ~150 VALU instructions an
-// iteration, as many iterations as the wavefront's slowest zone): the
+// the issue of FP64 instructions for wavefronts that run as long as their slowest
+// zone (2^24 zones move 2.6 GB in 1.30 ms; ~150 VALU instructions an iteration; by
+// the counters 66 % of VALU issue, 56 % of the lanes in the mean instruction): the
 // convergence test compares without dividing, one counter holds the stopping
 // rule, sin and cos share their reduction and the Kerr-Schild zeros are left out
 // (1.42 ms before).  At 4 wavefronts per SIMD (128 VGPRs) spills cost more than
@@ -344,7 +345,9 @@ __global__ __launch_bounds__(CB) void k_mlp_forward(long long n, const float* __
 // tiles, with a sample's units and a unit's samples both read from LDS rows.
 // One thread per sample on the vector units took 98 us for 4096 samples;
 // this form takes 13 us.  The rows are padded to 68 words: an A operand's 16 rows x 4
-// columns then fall on distinct banks.
+// columns then fall on distinct banks.  The operands read as 4 rows x 16 columns
+// (weights, and both sides of the weight gradients) still meet on some: conflicts
+// are 36 % of the LDS cycles, the matrix cores busy for 25 % of the time.
 constexpr int LP = MLP_H + 4;          // padded LDS row
 constexpr int GRAD_T = 512;            // threads of a gradient workgroup
 __device__ __forceinline__ mfma_f4 mfma4(float a, float b, mfma_f4 c) {

@@ -129,9 +129,9 @@ int hgpu_fixup_bounds(hgpu_ctx *ctx);
 int hgpu_step(hgpu_ctx *ctx, int nsteps);
 
 /* on != 0: hgpu_step() captures one step_ch() into a HIP graph on first use and
- * replays it (one launch per step instead of 16 kernel launches); per-kernel
- * profile scopes are then not recorded, "step" still is.  No counterpart in
- * the reference (launch mechanics only; results are identical). */
+ * replays it (one launch per step instead of 16 kernel launches, 19 on the binary
+ * metric); per-kernel profile scopes are then not recorded, "step" still is.  No
+ * counterpart in the reference (launch mechanics only; results are identical). */
 int hgpu_set_graph(hgpu_ctx *ctx, int on);
 
 /* Launch shapes of the stencil kernel families (0-2: face fluxes in x1, x2,
